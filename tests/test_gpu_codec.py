@@ -259,3 +259,14 @@ def test_host_pointer_codec_entry_points(O, tfq, gpu):
     assert np.array_equal(out.view(np.uint32), O.decode_tensor("Q_G_4", pay, w.size).view(np.uint32))
     # a format this build does not handle must say so, not encode on the CPU
     assert L.tfq_encode_blocks_host(119, w.ctypes.data, w.size, dst.ctypes.data, dst.size, None) in (2, 3)
+
+
+@pytest.mark.parametrize("n", [256, 1024 + 32, 4096, 4096 + 256 + 96, 4 * 4096 - 256])
+@pytest.mark.parametrize("fmt", ["B32S4", "B32S8", "Q_G_4", "Q_G_3", "Q_G_2", "SB256A3", "SB256A2", "Q_1_5", "Q_G_8", "Q_8", "Q_4", "Q_G_6"])
+def test_decode_block_counts_around_a_workgroups_share(O, tfq, gpu, fmt, n):
+    """A wavefront decodes four consecutive blocks and a short last block takes one more workgroup: one block, a share
+    of a workgroup (16 blocks) and its neighbours, with and without a short block behind; bit for bit."""
+    import torch
+    pay = O.encode_tensor(fmt, O.rng_normal(5, n, 0.02))
+    got = tfq.decode(fmt, torch.from_numpy(pay).to(gpu), n).cpu().numpy()
+    assert np.array_equal(got.view(np.uint32), O.decode_tensor(fmt, pay, n).view(np.uint32))

@@ -189,9 +189,7 @@ int tfq_decode_blocks(uint8_t fmt, const uint8_t* src, size_t bytes, int64_t n, 
     if (int r = check_tensor("tfq_decode_blocks", fmt, n, &need, &tail)) return r;
     if (bytes < need) return fail(TFQ_ERR_SHAPE, "tfq_decode_blocks: payload shorter than the blocks of n weights");
     if (int r = ensure_device()) return r;
-    if (int r = launch_decode(fmt, src, n / 256, out, (hipStream_t)stream)) return r;
-    if (!tail.n) return TFQ_OK;
-    return launch_decode_short(tail, src + need - (size_t)tail.bytes, out + (n / 256) * 256, (hipStream_t)stream);
+    return launch_decode(fmt, src, n / 256, out, (hipStream_t)stream, &tail);
 }
 
 int tfq_encode_blocks_host(uint8_t fmt, const float* w, int64_t n, uint8_t* dst, size_t cap, uint32_t* per_block_bytes) {
@@ -233,8 +231,7 @@ int tfq_decode_blocks_host(uint8_t fmt, const uint8_t* src, size_t bytes, int64_
     hipError_t e = hipMalloc(&dout, (size_t)n * 4);
     if (e != hipSuccess) { (void)hipFree(ds); return hip_fail(e, "hipMalloc"); }
     int rc = hip_fail(hipMemcpy(ds, src, need, hipMemcpyHostToDevice), "hipMemcpy H2D");
-    if (!rc) rc = launch_decode(fmt, ds, n / 256, dout, nullptr);
-    if (!rc && tail.n) rc = launch_decode_short(tail, ds + need - (size_t)tail.bytes, dout + (n / 256) * 256, nullptr);
+    if (!rc) rc = launch_decode(fmt, ds, n / 256, dout, nullptr, &tail);
     if (!rc) rc = hip_fail(hipMemcpy(out, dout, (size_t)n * 4, hipMemcpyDeviceToHost), "hipMemcpy D2H");
     (void)hipFree(ds);
     (void)hipFree(dout);

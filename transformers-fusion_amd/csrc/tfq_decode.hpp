@@ -177,7 +177,9 @@ __device__ __forceinline__ uint32_t half_at(const uint8_t* p) { return *reinterp
 template <int FMT>
 constexpr bool kHasQuad = spec_of(FMT).codec == Codec::Raw32 || spec_of(FMT).codec == Codec::Lattice ||
                           spec_of(FMT).codec == Codec::Grp16 || spec_of(FMT).codec == Codec::Q6K ||
-                          spec_of(FMT).codec == Codec::Fixed || spec_of(FMT).codec == Codec::Grp12;
+                          spec_of(FMT).codec == Codec::Fixed || spec_of(FMT).codec == Codec::Grp12 ||
+                          spec_of(FMT).codec == Codec::Affine || spec_of(FMT).codec == Codec::Grp8 ||
+                          spec_of(FMT).codec == Codec::Sym32;
 
 // v[t] = decode_weight<FMT>(p, 4 * lane + t), the same arithmetic on the same operands
 template <int FMT>
@@ -219,6 +221,38 @@ __device__ __forceinline__ void decode_quad(const uint8_t* __restrict__ p, uint3
         const float d = half_bits_to_float(half_at(p + lev_bits / 8 + 12));
 #pragma unroll
         for (uint32_t t = 0; t < 4; ++t) v[t] = grid_value(bits, (w >> (bits * t)) & ((1u << bits) - 1u)) * d * sc;
+    } else if constexpr (sp.codec == Codec::Affine) {
+        // four codes are 4 bits .. 16 bits; the header parts start at whole dwords of the block and the block is whole
+        // dwords long, so the second dword of a window stays inside it wherever the field needs it
+        constexpr uint32_t ng = 256 / sp.gsz, lev_bits = 256u * bits;
+        constexpr uint32_t sc_bits = ((ng * sp.scb + 7) / 8) * 8, mn_bits = ((ng * sp.mb + 7) / 8) * 8;
+        static_assert((lev_bits + sc_bits + mn_bits) % 32 == 0 && sp.block_bytes % 4 == 0, "d and dm are one aligned dword");
+        const uint32_t g = lane * 4u / (uint32_t)sp.gsz;
+        const uint32_t w = window32(p, 4u * bits * lane, limit);
+        const uint32_t dd = *reinterpret_cast<const uint32_t*>(p + (lev_bits + sc_bits + mn_bits) / 8);
+        const float sc = (float)(window32(p, lev_bits + g * sp.scb, limit) & ((1u << sp.scb) - 1u));
+        const float mc = (float)(window32(p, lev_bits + sc_bits + g * sp.mb, limit) & ((1u << sp.mb) - 1u)) - (float)((1 << sp.mb) / 2);
+        const float es = half_bits_to_float(dd & 0xFFFFu) * sc;
+        const float neg = -(half_bits_to_float(dd >> 16) * mc);
+#pragma unroll
+        for (uint32_t t = 0; t < 4; ++t) v[t] = __builtin_fmaf(es, unit_level(bits, (w >> (bits * t)) & ((1u << bits) - 1u)), neg);
+    } else if constexpr (sp.codec == Codec::Grp8) {
+        const uint32_t w = *reinterpret_cast<const uint32_t*>(p + 4 * lane);
+        const float d = half_bits_to_float(half_at(p + 256 + 2 * (lane >> 3)));
+#pragma unroll
+        for (uint32_t t = 0; t < 4; ++t) v[t] = d * __uint_as_float(kComp8Bits[(w >> (8u * t)) & 255u]);
+    } else if constexpr (sp.codec == Codec::Sym32) {
+        const float d = half_bits_to_float(half_at(p + 32 * bits + 2 * (lane >> 3)));
+        uint32_t w;
+        if constexpr (bits == 4) w = half_at(p + 2 * lane);
+        else w = *reinterpret_cast<const uint32_t*>(p + 4 * lane);
+#pragma unroll
+        for (uint32_t t = 0; t < 4; ++t) {
+            int q;
+            if constexpr (bits == 4) q = (int)((w >> (4u * t)) & 15u) - 8;
+            else q = (int)(int8_t)(w >> (8u * t));
+            v[t] = (float)q * d;
+        }
     } else {  // Q6K
         const uint32_t w = window32(p, 24u * lane, limit);
         const float sc = (float)(int)(int8_t)p[192 + (lane >> 2)];

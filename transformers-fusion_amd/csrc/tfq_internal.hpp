@@ -361,7 +361,8 @@ struct BlockLayout {
 bool block_layout(int fmt, int n, BlockLayout* out);
 
 // ------------------------------------------------------------- kernel launchers
-int launch_decode(int fmt, const uint8_t* src, int64_t nblocks, float* out, hipStream_t s);
+// nblocks full blocks, then (short_block given and not empty) the short last block of the tensor behind them
+int launch_decode(int fmt, const uint8_t* src, int64_t nblocks, float* out, hipStream_t s, const BlockLayout* short_block = nullptr);
 // one block of L.n <= 256 weights in the layout L
 int launch_decode_short(const BlockLayout& L, const uint8_t* src, float* out, hipStream_t s);
 int launch_tile16(int fmt, const uint8_t* wire, uint8_t* tiled, int64_t N, int64_t K, hipStream_t s);
@@ -524,23 +525,11 @@ int launch_lut_gemv_batch(int bits, const uint8_t* packed, const void* cb, float
 // subnormals, independent of the device's denormal mode
 // (f16_to_f32, src/codec/block_codec.cpp:76-99).
 __device__ __forceinline__ float half_bits_to_float(uint32_t h) {
-    const uint32_t sign = (h & 0x8000u) << 16;
-    const uint32_t ex = (h >> 10) & 0x1Fu;
-    const uint32_t man = h & 0x3FFu;
-    uint32_t u;
-    if (ex == 0) {
-        if (man == 0) {
-            u = sign;
-        } else {
-            const int lz = __clz(man) - 21;  // shifts needed to bring bit 10 up
-            const uint32_t m = (man << lz) & 0x3FFu;
-            u = sign | ((uint32_t)(113 - lz) << 23) | (m << 13);
-        }
-    } else if (ex == 31) {
-        u = sign | 0x7F800000u | (man << 13);
-    } else {
-        u = sign | ((ex + 112u) << 23) | (man << 13);
-    }
+    const uint32_t sign = (h & 0x8000u) << 16, mag = h & 0x7FFFu;
+    uint32_t u = (mag << 13) + (112u << 23);
+    if (mag >= 0x7C00u) u += 112u << 23;                                         // infinity and NaN
+    if (mag < 0x0400u) u = __float_as_uint((float)mag * 5.9604644775390625e-8f);  // subnormal: mag 2^-24, a normal binary32
+    u |= sign;
     return __uint_as_float(u);
 }
 
