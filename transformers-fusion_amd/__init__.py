@@ -1,7 +1,8 @@
-"""ctypes binding of libtfq.so, the gfx950 backend for the block-quantized
+"""Python binding of libtfq.so, the gfx950 backend for the block-quantized
 weight matmul.  PyTorch is used only to own device memory and streams; every
 computation is a hand-written HIP kernel reached through the C ABI declared in
-include/tfq.h.  There is no fallback: importing works without a GPU (so the
+include/tfq.h: ctypes for set-up and the rarer entry points, _tfq_torch.so
+(csrc/tfq_torch.cpp) for the calls a serving loop makes per token.  There is no fallback: importing works without a GPU (so the
 symbol table can be inspected), but every compute call raises TfqError when
 the library or the device is missing.
 
@@ -148,6 +149,24 @@ def lib():
     return _lib
 
 
+_native = None
+
+
+def native():
+    """_tfq_torch.so: the per-call part of this binding (tensors in, C ABI calls on torch's current stream) in C++."""
+    global _native
+    if _native is None:
+        lib()  # libtfq.so first: the extension links against it
+        import torch  # noqa: F401  (loads the libraries the extension links against)
+        try:
+            from . import _tfq_torch
+        except ImportError as e:
+            raise TfqError(f"_tfq_torch.so cannot be loaded ({e}): run __graft_entry__.build() first") from e
+        _tfq_torch.set_error(TfqError)
+        _native = _tfq_torch
+    return _native
+
+
 SHIMS_PATH = os.path.join(_HERE, "libtfq_shims.so")
 _shims = None
 
@@ -218,26 +237,17 @@ def init(device: int = 0):
 
 def encode(fmt, w):
     """fp32 device tensor -> uint8 device tensor of payloads (256-weight blocks, the last one possibly short)."""
-    import torch
-    w = w.contiguous()
-    assert w.is_cuda and w.dtype == torch.float32
-    n = w.numel()
-    nbytes = (n // 256) * block_bytes(fmt) + (block_bytes(fmt, n % 256) if n % 256 else 0)
-    out = torch.empty(nbytes, dtype=torch.uint8, device=w.device)
-    _check(lib().tfq_encode_blocks(fmt_id(fmt), w.data_ptr(), n, out.data_ptr(), out.numel(), _stream()))
-    return out
+    return (_native or native()).encode(FMT[fmt] if isinstance(fmt, str) else int(fmt), w)
 
 
 def decode(fmt, payload, n: int):
-    import torch
-    assert payload.is_cuda and payload.dtype == torch.uint8
-    out = torch.empty(n, dtype=torch.float32, device=payload.device)
-    _check(lib().tfq_decode_blocks(fmt_id(fmt), payload.data_ptr(), payload.numel(), n, out.data_ptr(), _stream()))
-    return out
+    return (_native or native()).decode(FMT[fmt] if isinstance(fmt, str) else int(fmt), payload, n)
 
 
 class Weight:
     """Device-resident packed matrix W[N][K] (N rows of K/256 wire blocks)."""
+
+    _h = 0  # the handle's address as a plain int, what the native calls take
 
     def __init__(self, fmt, N: int, K: int, packed, handle=None):
         import numpy as np
@@ -245,6 +255,7 @@ class Weight:
         self.fmt, self.N, self.K = fmt_id(fmt), int(N), int(K)
         if handle is not None:  # adopted from tfq_container_weight
             self.handle = C.c_void_p(handle)
+            self._h = self.handle.value
             return
         if isinstance(packed, torch.Tensor) and packed.is_cuda:
             # device payload: copied into the handle's own layout, the caller may drop its tensor
@@ -256,6 +267,7 @@ class Weight:
         if not h:
             raise TfqError(lib().tfq_last_error().decode())
         self.handle = C.c_void_p(h)
+        self._h = self.handle.value
 
     @classmethod
     def mixed(cls, N: int, K: int, block_formats, packed):
@@ -273,6 +285,7 @@ class Weight:
         if getattr(self, "handle", None):
             lib().tfq_weight_free(self.handle)
             self.handle = None
+            self._h = 0
 
     def __del__(self):
         try:
@@ -286,35 +299,11 @@ class Weight:
         _check(lib().tfq_weight_decode(self.handle, out.data_ptr(), _stream()))
         return out
 
-    def _mm(self, fn, x, out_dtype):
-        import torch
-        x = x.contiguous()
-        assert x.is_cuda and x.shape[-1] == self.K
-        B = x.numel() // self.K
-        y = torch.empty((B, self.N), dtype=out_dtype or torch.float32, device=x.device)
-        _check(fn(self.handle, x.data_ptr(), _dtype_code(x), B, y.data_ptr(), _dtype_code(y), _stream()))
-        return y
-
     def gemv(self, x, out_dtype=None, out=None, workspace=None):
         """y[B][N] = x[B][K] . W^T for 1 <= B <= 16 (decode).  Calls that cut K into parts (five or more rows, K above
         4096) go through tfq_gemv_ws; `workspace` is a uint8 tensor of tfq_gemv_workspace_bytes or more (one is made
         per call when none is given; pass one when the call is captured into a graph and replayed)."""
-        import torch
-        x = x.contiguous()
-        assert x.is_cuda and x.shape[-1] == self.K
-        B = x.numel() // self.K
-        if out is None:
-            out = torch.empty((B, self.N), dtype=out_dtype or torch.float32, device=x.device)
-        need = int(lib().tfq_gemv_workspace_bytes(self.handle, _dtype_code(x), B))
-        if need == 0:
-            _check(lib().tfq_gemv(self.handle, x.data_ptr(), _dtype_code(x), B, out.data_ptr(), _dtype_code(out), _stream()))
-            return out
-        if workspace is None:
-            workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
-        assert workspace.numel() >= need and workspace.data_ptr() % 256 == 0
-        _check(lib().tfq_gemv_ws(self.handle, x.data_ptr(), _dtype_code(x), B, out.data_ptr(), _dtype_code(out),
-                                 workspace.data_ptr(), workspace.numel(), _stream()))
-        return out
+        return (_native or native()).gemv(self._h, self.N, self.K, x, out_dtype, out, workspace)
 
     def gemv_workspace_bytes(self, x_dtype_code: int, B: int) -> int:
         return int(lib().tfq_gemv_workspace_bytes(self.handle, x_dtype_code, B))
@@ -322,18 +311,7 @@ class Weight:
     def gemm(self, x, out_dtype=None, workspace=True):
         """y[M][N] = x[M][K] . W^T for any M (prefill).  With `workspace` the call goes through tfq_gemm_ws with
         as much scratch memory as tfq_gemm_workspace_bytes asks for (the K split of the prefill kernel)."""
-        import torch
-        if not workspace:
-            return self._mm(lib().tfq_gemm, x, out_dtype)
-        x = x.contiguous()
-        assert x.is_cuda and x.shape[-1] == self.K
-        M = x.numel() // self.K
-        y = torch.empty((M, self.N), dtype=out_dtype or torch.float32, device=x.device)
-        need = int(lib().tfq_gemm_workspace_bytes(self.handle, _dtype_code(x), M))
-        ws = torch.empty(max(need, 16), dtype=torch.uint8, device=x.device)
-        _check(lib().tfq_gemm_ws(self.handle, x.data_ptr(), _dtype_code(x), M, y.data_ptr(), _dtype_code(y),
-                                 ws.data_ptr(), need, _stream()))
-        return y
+        return (_native or native()).gemm(self._h, self.N, self.K, x, out_dtype, workspace)
 
 
 class _ChainPhase(C.Structure):
@@ -501,18 +479,7 @@ class Container:
 
 def gemv_multi(weights, x, outs):
     """One launch for up to four matrices that share K, format and x (q/k/v, gate/up)."""
-    n = len(weights)
-    hs = (C.c_void_p * n)(*[w.handle for w in weights])
-    ys = (C.c_void_p * n)(*[o.data_ptr() for o in outs])
-    B = x.numel() // weights[0].K
-    _check(lib().tfq_gemv_multi(hs, n, x.data_ptr(), _dtype_code(x), B, ys, _dtype_code(outs[0]), _stream()))
-    return outs
-
-
-class _Prologue(C.Structure):
-    """tfq_prologue_t (include/tfq.h)."""
-    _fields_ = [("op", C.c_int), ("gamma", C.c_void_p), ("eps", C.c_float), ("gamma_plus_one", C.c_int),
-                ("up", C.c_void_p), ("mid_dtype", C.c_int), ("pair_swiglu", C.c_int), ("accumulate", C.c_int)]
+    return (_native or native()).gemv_multi(weights, x, outs)
 
 
 PRO_NONE, PRO_RMSNORM, PRO_SWIGLU = 0, 1, 2
@@ -522,46 +489,12 @@ def gemv_multi_fused(ws, x, outs, *, rmsnorm=None, swiglu_up=None, eps=1e-6, gam
                      pair_swiglu=False):
     """tfq_gemv_multi_fused: up to four matrices on fp32 x [B][K] with RMSNorm (rmsnorm = the fp32 gain vector)
     or SwiGLU (x = the gate product, swiglu_up = the up product) applied while the activations are staged."""
-    import torch
-    n = len(ws)
-    assert x.is_contiguous()
-    B = x.shape[0]
-    hs = (C.c_void_p * n)(*[w.handle for w in ws])
-    ys = (C.c_void_p * n)(*[o.data_ptr() for o in outs])
-    pro = _Prologue()
-    pro.accumulate = 1 if accumulate else 0
-    pro.pair_swiglu = 1 if pair_swiglu else 0
-    if pair_swiglu and len(outs) == 1:  # ys[1] is not written; the C call still wants two pointers
-        ys = (C.c_void_p * n)(outs[0].data_ptr(), outs[0].data_ptr())
-    if rmsnorm is not None:
-        assert rmsnorm.dtype == torch.float32
-        pro.op, pro.gamma, pro.eps, pro.gamma_plus_one = PRO_RMSNORM, rmsnorm.data_ptr(), eps, 1 if gamma_plus_one else 0
-    elif swiglu_up is not None:
-        assert swiglu_up.dtype == torch.float32 and swiglu_up.shape == x.shape and swiglu_up.is_contiguous()
-        pro.op, pro.up = PRO_SWIGLU, swiglu_up.data_ptr()
-        pro.mid_dtype = BF16 if mid_dtype == torch.bfloat16 else F32
-    _check(lib().tfq_gemv_multi_fused(hs, n, x.data_ptr(), _dtype_code(x), B, ys, _dtype_code(outs[0]), C.byref(pro), _stream()))
-    return outs
+    return (_native or native()).gemv_multi_fused(ws, x, outs, rmsnorm, swiglu_up, eps, gamma_plus_one, mid_dtype, accumulate, pair_swiglu)
 
 
 def moe_router(x, router_w, k: int, bias=None):
     """Router Linear + softmax + top-k on the device: returns (logits, probs, idx int32, weights)."""
-    import torch
-    T, D = x.shape
-    E = router_w.shape[0]
-    assert router_w.dtype == torch.float32 and router_w.is_contiguous() and x.is_contiguous()
-    logits = torch.empty(T, E, device=x.device)
-    probs = torch.empty(T, E, device=x.device)
-    kk = max(1, min(k, E))
-    idx = torch.empty(T, kk, device=x.device, dtype=torch.int32)
-    w = torch.empty(T, kk, device=x.device)
-    L = lib()
-    L.tfq_moe_router.restype = C.c_int
-    L.tfq_moe_router.argtypes = [C.c_void_p, C.c_int, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int,
-                                 C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]
-    _check(L.tfq_moe_router(x.data_ptr(), _dtype_code(x), router_w.data_ptr(), bias.data_ptr() if bias is not None else None,
-                            T, D, E, k, logits.data_ptr(), probs.data_ptr(), idx.data_ptr(), w.data_ptr(), _stream()))
-    return logits, probs, idx, w
+    return (_native or native()).moe_router(x, router_w, k, bias)
 
 
 def moe_route(logits, k: int):
@@ -579,37 +512,16 @@ def moe_route(logits, k: int):
 
 def mlp_step(gate, up, down, x, out_dtype=None, mid_dtype=None):
     """Dense SwiGLU feed-forward y = down(silu(gate x) * (up x)) for x [B][D] on the device."""
-    import torch
-    x = x.contiguous()
-    B = x.numel() // gate.K
-    y = torch.empty((B, down.N), dtype=out_dtype or torch.float32, device=x.device)
-    mid = BF16 if (mid_dtype or x.dtype) == torch.bfloat16 else F32
-    nbytes = lib().tfq_mlp_workspace_bytes(B, gate.N)
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
-    _check(lib().tfq_mlp_step(gate.handle, up.handle, down.handle, x.data_ptr(), _dtype_code(x), B, y.data_ptr(),
-                              _dtype_code(y), mid, ws.data_ptr(), nbytes, _stream()))
-    return y
+    return (_native or native()).mlp_step(gate, up, down, x, out_dtype, mid_dtype)
 
 
 def moe_ffn(gate, up, down, topk_idx, topk_w, x, out_dtype=None, mid_dtype=None):
     """MoE expert FFN.  gate/up/down: lists of Weight; topk_idx/topk_w: host arrays [T][k]; x: device [T][D]."""
     import numpy as np
-    import torch
-    E = len(gate)
     idx = np.ascontiguousarray(topk_idx, np.int64)
     wts = np.ascontiguousarray(topk_w, np.float32)
     T, k = idx.shape
-    D, F = gate[0].K, gate[0].N
-    x = x.contiguous()
-    y = torch.empty((T, D), dtype=out_dtype or torch.float32, device=x.device)
-    mid = BF16 if (mid_dtype or x.dtype) == torch.bfloat16 else F32
-    nbytes = lib().tfq_moe_workspace_bytes(T, k, D, F)
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
-    arr = lambda ws_: (C.c_void_p * E)(*[w.handle for w in ws_])
-    _check(lib().tfq_moe_ffn(arr(gate), arr(up), arr(down), E, idx.ctypes.data, wts.ctypes.data, T, k,
-                             x.data_ptr(), _dtype_code(x), y.data_ptr(), _dtype_code(y), mid,
-                             ws.data_ptr(), nbytes, _stream()))
-    return y
+    return (_native or native()).moe_ffn(gate, up, down, idx, wts, T, k, x, out_dtype, mid_dtype)
 
 
 class RoutedMoe:
@@ -630,13 +542,10 @@ class RoutedMoe:
         if self.nbytes == 0:
             raise TfqError("tfq_moe_ffn_routed does not take this configuration")
         self.ws = torch.empty(self.nbytes, dtype=torch.uint8, device=device)
+        self._arrays = tuple(C.addressof(a) for a in (self._g, self._u, self._d))
 
     def __call__(self, idx, wts, x, y):
-        assert idx.is_cuda and wts.is_cuda and idx.dtype.itemsize == 4 and x.is_contiguous() and y.is_contiguous()
-        _check(lib().tfq_moe_ffn_routed(self._g, self._u, self._d, self.E, self.table.data_ptr(), idx.data_ptr(), wts.data_ptr(),
-                                        self.T, self.k, x.data_ptr(), _dtype_code(x), y.data_ptr(), _dtype_code(y), BF16,
-                                        self.ws.data_ptr(), self.nbytes, _stream()))
-        return y
+        return (_native or native()).moe_ffn_routed(*self._arrays, self.E, self.table, idx, wts, self.T, self.k, x, y, self.ws)
 
 
 def moe_plan_dispatch(topk_idx, topk_w, E: int, slots_per_expert: int):

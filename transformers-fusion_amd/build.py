@@ -72,6 +72,29 @@ def build_shims(verbose: bool = False) -> str:
     return SHIMS
 
 
+TORCH_EXT = os.path.join(HERE, "_tfq_torch.so")
+
+
+def build_torch_binding(verbose: bool = False) -> str:
+    """Host C++ (g++): the per-call part of the Python binding against torch's C++ tensors and streams."""
+    import sysconfig
+
+    import torch
+    tdir = os.path.dirname(torch.__file__)
+    inc = [os.path.join(tdir, "include"), os.path.join(tdir, "include", "torch", "csrc", "api", "include"),
+           sysconfig.get_paths()["include"], os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include")]
+    cmd = ["g++", "-std=c++17", "-O2", "-fPIC", "-shared", "-Wall", "-Wno-attributes", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *[f"-isystem{i}" for i in inc], os.path.join(CSRC, "tfq_torch.cpp"), "-o", TORCH_EXT,
+           "-L" + HERE, "-ltfq", "-L" + os.path.join(tdir, "lib"), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip",
+           "-Wl,-rpath,$ORIGIN"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    subprocess.check_call(cmd)
+    return TORCH_EXT
+
+
 if __name__ == "__main__":
     print(build_library(verbose=True))
     print(build_shims(verbose=True))
+    print(build_torch_binding(verbose=True))
