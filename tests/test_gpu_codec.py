@@ -270,3 +270,24 @@ def test_decode_block_counts_around_a_workgroups_share(O, tfq, gpu, fmt, n):
     pay = O.encode_tensor(fmt, O.rng_normal(5, n, 0.02))
     got = tfq.decode(fmt, torch.from_numpy(pay).to(gpu), n).cpu().numpy()
     assert np.array_equal(got.view(np.uint32), O.decode_tensor(fmt, pay, n).view(np.uint32))
+
+
+# 64 / lanes-per-block blocks share a wavefront; runs get more lanes below 8192 blocks (Q_8, the lattices) or groups * 8
+# of them (Q_G_8); the level of a weight is taken from a product unless it lies near a rounding boundary, where the
+# quotient decides: the tied inputs (halves of a step, powers of two, one huge or tiny value) take that branch.
+@pytest.mark.parametrize("nblk,tail", [(1, 0), (3, 96), (4, 0), (5, 223), (8, 32), (9, 0), (17, 255), (8193, 64)])
+@pytest.mark.parametrize("fmt", ["B32S4", "B32S8", "Q_G_4", "Q_G_3", "Q_G_2", "SB256A3", "Q_1_5", "Q_G_8", "Q_8", "Q_4", "Q_2", "Q_3", "Q_6", "Q_G_6"])
+def test_encode_block_counts_and_ties(O, tfq, gpu, fmt, nblk, tail):
+    import torch
+    if fmt.startswith("B32"):
+        tail = tail // 32 * 32
+    n = nblk * 256 + tail
+    w = O.rng_normal(1000 + nblk, n, 0.02)
+    w[: n // 2] = np.round(w[: n // 2] * 150.0) * 0.25  # quarters: many levels at exactly half a step
+    b = w[: nblk * 256].reshape(nblk, 256)
+    b[0, :16] = np.ldexp(1.0, np.arange(-8, 8)).astype(np.float32)
+    b[nblk // 2, 40] = 3.0e31
+    b[nblk - 1, 64:96] = 1.0e-31
+    print(f"encode {fmt} {nblk} {tail}", flush=True)
+    got = tfq.encode(fmt, torch.from_numpy(w).to(gpu)).cpu().numpy()
+    assert np.array_equal(got, O.encode_tensor(fmt, w))

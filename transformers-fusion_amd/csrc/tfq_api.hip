@@ -177,9 +177,7 @@ int tfq_encode_blocks(uint8_t fmt, const float* w, int64_t n, uint8_t* dst, size
     if (int r = check_tensor("tfq_encode_blocks", fmt, n, &need, &tail)) return r;
     if (cap < need) return fail(TFQ_ERR_SHAPE, "tfq_encode_blocks: destination too small");
     if (int r = ensure_device()) return r;
-    if (int r = launch_encode(fmt, w, n / 256, dst, (hipStream_t)stream)) return r;
-    if (!tail.n) return TFQ_OK;
-    return launch_encode_short(fmt, tail, w + (n / 256) * 256, dst + need - (size_t)tail.bytes, (hipStream_t)stream);
+    return launch_encode(fmt, w, n / 256, dst, (hipStream_t)stream, &tail);
 }
 
 int tfq_decode_blocks(uint8_t fmt, const uint8_t* src, size_t bytes, int64_t n, float* out, tfq_stream_t stream) {
@@ -205,8 +203,7 @@ int tfq_encode_blocks_host(uint8_t fmt, const float* w, int64_t n, uint8_t* dst,
     hipError_t e = hipMalloc(&dd, need);
     if (e != hipSuccess) { (void)hipFree(dw); return hip_fail(e, "hipMalloc"); }
     int rc = hip_fail(hipMemcpy(dw, w, (size_t)n * 4, hipMemcpyHostToDevice), "hipMemcpy H2D");
-    if (!rc) rc = launch_encode(fmt, dw, n / 256, dd, nullptr);
-    if (!rc && tail.n) rc = launch_encode_short(fmt, tail, dw + (n / 256) * 256, dd + need - (size_t)tail.bytes, nullptr);
+    if (!rc) rc = launch_encode(fmt, dw, n / 256, dd, nullptr, &tail);
     if (!rc) rc = hip_fail(hipMemcpy(dst, dd, need, hipMemcpyDeviceToHost), "hipMemcpy D2H");
     (void)hipFree(dw);
     (void)hipFree(dd);

@@ -5,6 +5,7 @@
 // at most 1 KB, so these kernels are bound by the fp32 side (4 B per weight).
 
 #include "tfq_decode.hpp"
+#include "tfq_encode_short.hpp"
 
 #include <cmath>
 
@@ -59,38 +60,56 @@ __global__ __launch_bounds__(256) void decode_short_kernel(BlockLayout L, const 
 //   qmax = 7, lo = -8 (4-bit) or qmax = 127, lo = -127 (8-bit); d == 0 or not
 //   finite gives q = 0.  (The reference holds this quantizer only as comparator
 //   code: src/adapters/tools/bench_ollama_comparison.cpp:61-75, 121-134.)
+// Four weights per lane, a wavefront per block, kEncodeBlocks blocks in a row; a group of 32 is eight lanes.  Bound by
+// the reads (4 bytes per weight).  The tensor's short last block (tail_n weights, whole groups) is one more block with
+// fewer lanes.  58.7 M weights of B32S4: 168 us with a lane per weight and byte stores, 67 us.
+constexpr int kEncodeBlocks = 2;
 template <int FMT>
-__global__ __launch_bounds__(256) void encode_sym32_kernel(const float* __restrict__ w,
-                                                           uint8_t* __restrict__ dst) {
+__global__ __launch_bounds__(256) void encode_sym32_kernel(const float* __restrict__ w, uint8_t* __restrict__ dst, int64_t nblocks, int tail_n) {
     constexpr Spec sp = spec_of(FMT);
-    constexpr uint32_t code_bytes = 256u * sp.bits / 8;
     constexpr float qmax = sp.bits == 4 ? 7.0f : 127.0f;
     constexpr int lo = sp.bits == 4 ? -8 : -127, hi = sp.bits == 4 ? 7 : 127;
-    const int64_t blk = blockIdx.x;
-    const uint32_t i = threadIdx.x;
-    uint8_t* p = dst + blk * (int64_t)sp.block_bytes;
-    const float x = w[blk * 256 + i];
-    float amax = fabsf(x);
+    const uint32_t lane = threadIdx.x & 63;
+    const int64_t first = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * kEncodeBlocks;
+    float4 v[kEncodeBlocks];
 #pragma unroll
-    for (int m = 16; m >= 1; m >>= 1) amax = fmaxf(amax, __shfl_xor(amax, m, 32));
-    const uint32_t h = float_to_half_bits(amax / qmax);
-    const float d = half_bits_to_float(h);
-    int q = 0;
-    if (d > 0.0f && (h & 0x7C00u) != 0x7C00u) {
-        const float r = roundf(x / d);
-        q = r <= (float)lo ? lo : r >= (float)hi ? hi : (int)r;
+    for (int k = 0; k < kEncodeBlocks; ++k) {
+        const int64_t blk = first + k;
+        v[k] = float4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (blk < nblocks || (blk == nblocks && 4 * (int)lane < tail_n)) __builtin_memcpy(&v[k], w + blk * 256 + 4 * lane, 16);  // (aligned to a float only)
     }
-    if constexpr (sp.bits == 4) {
-        const uint32_t mine = (uint32_t)(q + 8);
-        const uint32_t next = __shfl_down(mine, 1, 64);
-        if ((i & 1u) == 0) p[i >> 1] = (uint8_t)(mine | (next << 4));
-    } else {
-        p[i] = (uint8_t)(int8_t)q;
+#pragma unroll
+    for (int k = 0; k < kEncodeBlocks; ++k) {
+        const int64_t blk = first + k;
+        const float x[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
+        float amax = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3])));
+#pragma unroll
+        for (int m = 4; m >= 1; m >>= 1) amax = fmaxf(amax, __shfl_xor(amax, m, 64));
+        const uint32_t h = float_to_half_bits(amax / qmax);
+        const float d = half_bits_to_float(h);
+        uint32_t packed = sp.bits == 4 ? 0x8888u : 0u;
+        if (d > 0.0f && (h & 0x7C00u) != 0x7C00u) {
+            packed = 0;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const float r = roundf(x[t] / d);
+                const int q = r <= (float)lo ? lo : r >= (float)hi ? hi : (int)r;
+                packed |= sp.bits == 4 ? (uint32_t)(q + 8) << (4 * t) : (uint32_t)(uint8_t)(int8_t)q << (8 * t);
+            }
+        }
+        const int n = blk < nblocks ? 256 : blk == nblocks ? tail_n : 0;
+        if (4 * (int)lane < n) {
+            uint8_t* p = dst + blk * (int64_t)sp.block_bytes;
+            __builtin_memcpy(p + lane * (sp.bits / 2), &packed, sp.bits / 2);
+            if ((lane & 7u) == 0) __builtin_memcpy(p + n * sp.bits / 8 + 2 * (lane >> 3), &h, 2);
+        }
     }
-    if ((i & 31u) == 0) {
-        p[code_bytes + 2 * (i >> 5)] = (uint8_t)(h & 0xFF);
-        p[code_bytes + 2 * (i >> 5) + 1] = (uint8_t)(h >> 8);
-    }
+}
+
+template <int FMT>
+static void launch_encode_sym32(const float* w, int64_t nblocks, uint8_t* dst, int tail_n, hipStream_t s) {
+    const int64_t grid = (nblocks + (tail_n > 0) + 4 * kEncodeBlocks - 1) / (4 * kEncodeBlocks);
+    hipLaunchKernelGGL(encode_sym32_kernel<FMT>, dim3((unsigned)grid), dim3(256), 0, s, w, dst, nblocks, tail_n);
 }
 
 __global__ __launch_bounds__(256) void encode_raw32_kernel(const float* __restrict__ w,
@@ -253,12 +272,19 @@ __global__ __launch_bounds__(256) void encode_q1_kernel(const float* __restrict_
 }
 
 // Affine family encoder: quant_affine with grp16_fit_affine (src/codec/block_codec.cpp:1337-1521) for
-// Q_G_4 / Q_G_3 / Q_G_2, the superblock formats and Q_1_5.  One wavefront per block; lane g owns group g
-// (8 or 16 lanes work): the per-group Lloyd fit (4 x assign + least-squares refit, +-15 % scale polish,
-// closing refit) and the per-group part of the 5 joint refinements run sequentially in that lane, in the
-// reference's order, with double sums; lane 0 does the sums over groups.  Multiply-adds are fused exactly
-// where the reference's Release build (GCC, -ffp-contract=fast) fuses them and nowhere else.  The payload
-// is then assembled a byte per lane from the codes in LDS.
+// Q_G_4 / Q_G_3 / Q_G_2, the superblock formats and Q_1_5.  A lane owns a group and keeps its 32 or 16 weights in
+// registers, so a wavefront encodes eight or four blocks: the per-group Lloyd fit (4 x assign + least-squares refit,
+// +-15 % scale polish, closing refit) and the per-group part of the 5 joint refinements run in the lane, in the
+// reference's order, with double sums; the sums over the groups of a block are read from LDS by all of its lanes.
+// Multiply-adds are fused exactly where the reference's Release build (GCC, -ffp-contract=fast) fuses them and
+// nowhere else.
+// Bound by vector instructions: 17 passes over the weights, about 12 instructions per weight and pass.  What a pass
+// needs of a weight is its level, lround(clamp((x - m) / s) * top) in fp32; the correctly rounded division alone is
+// ten instructions.  level_pass therefore takes the level from one multiply-add by top / s, which differs from the
+// reference's value before the rounding by less than `2^-24 (128 + 4 |m top / s|)`, and remembers how close any weight
+// of the group came to a rounding boundary; where that is closer than the bound (4 % of the wavefronts and passes)
+// the lane repeats the pass with the reference's own arithmetic.  The payload is therefore the reference's in every
+// case.  58.7 M weights of Q_G_4: 7.46 ms with one block per wavefront and the division, 450 us.
 __device__ __forceinline__ uint32_t unit_nearest_dev(float value, int bits) {
     const float v = fmaxf(0.0f, fminf(1.0f, value));
     const float top = bits == 1 ? 1.0f : bits == 4 ? 15.0f : bits == 3 ? 7.0f : bits == 6 ? 63.0f : bits == 8 ? 255.0f : 3.0f;
@@ -268,87 +294,137 @@ __device__ __forceinline__ double fms2(double a, double b, double c, double d) {
     return __builtin_fma(a, b, -(c * d));
 }
 
+// use(i, n) for every weight of the group, n (float) = its level index for offset m and scale s; `reset` forgets what
+// `use` gathered.  odd: the group holds a NaN, an infinity or a magnitude the bound does not cover.
+template <int BITS, int GSZ, class Reset, class Use>
+__device__ __forceinline__ void level_pass(const float (&x)[GSZ], float m, float s, bool odd, Reset&& reset, Use&& use) {
+    constexpr float top = (float)((1 << BITS) - 1);
+    const float r = top / s;
+    const float mr = m * r;
+    float far = 0.0f;
+    reset();
+#pragma unroll
+    for (int i = 0; i < GSZ; ++i) {
+        const float t = __builtin_amdgcn_fmed3f(__builtin_fmaf(x[i], r, -mr), 0.0f, top);
+        const float n = __builtin_rintf(t);
+        far = fmaxf(far, fabsf(t - n));
+        use(i, n);
+    }
+    // (written so that a NaN bound, as from s = 0, takes the branch)
+    if (odd || !(far <= 0.5f - 5.9604644775390625e-8f * (128.0f + 4.0f * fabsf(mr)))) {
+        reset();
+#pragma unroll
+        for (int i = 0; i < GSZ; ++i) {
+            use(i, (float)unit_nearest_dev((x[i] - m) / s, BITS));
+            __builtin_amdgcn_sched_barrier(0);  // one division at a time: interleaved, they would take the registers of the fast path
+        }
+    }
+}
+
 template <int FMT>
-__global__ __launch_bounds__(64) void encode_affine_kernel(const float* __restrict__ wg, uint8_t* __restrict__ dst) {
+__global__ __launch_bounds__(64, 4) void encode_affine_kernel(const float* __restrict__ wg, uint8_t* __restrict__ dst, int64_t nblocks, ShortJob job) {
     constexpr Spec sp = spec_of(FMT);
     constexpr int bits = sp.bits, gsz = sp.gsz, ng = 256 / gsz;
     constexpr int scq = (1 << sp.scb) - 1, mq = (1 << sp.mb) - 1, bias = (mq + 1) / 2;
     constexpr float eps = 1e-15f;
-    __shared__ float w[256];
-    __shared__ float s_[16], m_[16];
-    __shared__ int sc_[16], mc_[16];
-    __shared__ float dd[2];
-    __shared__ uint8_t code[256];
-    const int64_t blk = blockIdx.x;
-    const int t = threadIdx.x;
-    for (int i = t; i < 256; i += 64) w[i] = wg[blk * 256 + i];
-    __syncthreads();
-    const float* x = w + t * gsz;
+    constexpr float unit = bits == 1 ? 1.0f : 1.0f / (float)((1 << bits) - 1);  // unit_level(bits, n) = n * unit
+    __shared__ double2 sums[64];  // (value, its integer code) of every group
+    __shared__ uint8_t hcode[128];
+    __shared__ Team short_team;
+    const int with_short = job.L.n > 0;
+    if (with_short && blockIdx.x == 0) { encode_short_block<FMT>(job, short_team); return; }
+    const int t = threadIdx.x, g = t & (ng - 1), first = t & ~(ng - 1);
+    const int64_t mine = (int64_t)(blockIdx.x - with_short) * (64 / ng) + t / ng;
+    const int64_t blk = mine < nblocks ? mine : nblocks - 1;  // past the end: the last block again, stored by nobody
+    float x[gsz];
+#pragma unroll
+    for (int i = 0; i < gsz; i += 4) {
+        float4 v;  // (the caller's pointer is aligned to a float only)
+        __builtin_memcpy(&v, wg + blk * 256 + g * gsz + i, 16);
+        x[i] = v.x; x[i + 1] = v.y; x[i + 2] = v.z; x[i + 3] = v.w;
+    }
+    float maxw = -1e30f, minw = 1e30f;
+    uint32_t top_bits = 0;
+    double sx = 0;  // the same in every refit
+#pragma unroll
+    for (int i = 0; i < gsz; ++i) {
+        maxw = fmaxf(maxw, x[i]);
+        minw = fminf(minw, x[i]);
+        top_bits = max(top_bits, __float_as_uint(x[i]) & 0x7FFFFFFFu);
+        sx += (double)x[i];
+    }
+    const bool odd = top_bits > 0x71000000u;  // above 2^99, infinite or NaN
+    constexpr double sw = (double)gsz;
+
+    double sl, sl2, sxl;
+    auto solve = [&](float& s, float& m) __attribute__((always_inline)) {
+        const double D = fms2(sw, sl2, sl, sl);
+        if (D > 1e-20) {
+            s = (float)(fms2(sw, sxl, sx, sl) / D);
+            m = (float)(fms2(sl2, sx, sl, sxl) / D);
+        }
+    };
+    auto clear = [&]() __attribute__((always_inline)) { sl = 0; sl2 = 0; sxl = 0; };
 
     // ---- per-group fit
-    if (t < ng) {
-        float maxw = -1e30f, minw = 1e30f;
-        for (int i = 0; i < gsz; ++i) { maxw = fmaxf(maxw, x[i]); minw = fminf(minw, x[i]); }
-        float s = maxw - minw, m = minw;
-        if (!(fabsf(s) > 1e-30f)) { s = 0.0f; m = 0.0f; }
-        else {
-            // assign levels with (am, as), then refit (s, m) by least squares over (level, weight)
-            auto assign_refit = [&](float am, float as) __attribute__((always_inline)) {
-                double sw = 0, sl = 0, sl2 = 0, sx = 0, sxl = 0;
-                for (int i = 0; i < gsz; ++i) {
-                    const double l = (double)unit_level(bits, unit_nearest_dev((x[i] - am) / as, bits));
-                    sw += 1.0; sl += l; sl2 = __builtin_fma(l, l, sl2);
-                    sx += (double)x[i]; sxl = __builtin_fma((double)x[i], l, sxl);
+    float s = maxw - minw, m = minw;
+    if (!(fabsf(s) > 1e-30f)) { s = 0.0f; m = 0.0f; }
+    else {
+        // assign levels, then refit (s, m) by least squares over (level, weight): four times, then once more behind the polish
+#pragma unroll 1
+        for (int iter = 0; iter < 5; ++iter) {
+            if (iter == 4) {
+                float best_s = s;
+                double best = 1e300;
+#pragma unroll 1
+                for (int k = -3; k <= 3; ++k) {
+                    if (k == 0) continue;
+                    const float cs = s * __builtin_fmaf(0.05f, (float)k, 1.0f);
+                    double e;
+                    level_pass<bits, gsz>(x, m, cs, odd, [&]() __attribute__((always_inline)) { e = 0.0; },
+                                          [&](int i, float n) __attribute__((always_inline)) {
+                                              const float d = __builtin_fmaf(cs, n * unit, m) - x[i];
+                                              e = __builtin_fma((double)d, (double)d, e);
+                                          });
+                    if (e < best) { best = e; best_s = cs; }
                 }
-                const double D = fms2(sw, sl2, sl, sl);
-                if (D > 1e-20) {
-                    s = (float)(fms2(sw, sxl, sx, sl) / D);
-                    m = (float)(fms2(sl2, sx, sl, sxl) / D);
-                }
-            };
-            for (int iter = 0; iter < 4; ++iter) assign_refit(m, s);
-            float best_s = s;
-            const float best_m = m;
-            double best = 1e300;
-            for (int k = -3; k <= 3; ++k) {
-                if (k == 0) continue;
-                const float cs = s * __builtin_fmaf(0.05f, (float)k, 1.0f);
-                double e = 0.0;
-                for (int i = 0; i < gsz; ++i) {
-                    const float l = unit_level(bits, unit_nearest_dev((x[i] - m) / cs, bits));
-                    const float d = __builtin_fmaf(cs, l, m) - x[i];
-                    e = __builtin_fma((double)d, (double)d, e);
-                }
-                if (e < best) { best = e; best_s = cs; }
+                s = best_s;
             }
-            s = best_s;
-            assign_refit(best_m, s);
+            level_pass<bits, gsz>(x, m, s, odd, clear, [&](int i, float n) __attribute__((always_inline)) {
+                const double l = (double)(n * unit);
+                sl += l;
+                sl2 = __builtin_fma(l, l, sl2);
+                sxl = __builtin_fma((double)x[i], l, sxl);
+            });
+            solve(s, m);
         }
-        s_[t] = s;
-        m_[t] = m;
-        sc_[t] = 0;
-        mc_[t] = 0;
     }
-    __syncthreads();
 
     // ---- global d / dm and the joint refinement
-    if (t == 0) {
-        float max_s = 0.0f, max_m = 0.0f;
-        for (int g = 0; g < ng; ++g) { max_s = fmaxf(max_s, fabsf(s_[g])); max_m = fmaxf(max_m, fabsf(m_[g])); }
-        float d = 1.0f, dm = 1.0f;
-        if (max_s <= eps) d = 0.0f;
-        else {
-            d = half_bits_to_float(float_to_half_bits(max_s / (float)scq));
-            if (max_m > eps) dm = half_bits_to_float(float_to_half_bits(max_m / (float)bias));
+    auto block_max = [&](float v) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = ng / 2; k >= 1; k >>= 1) v = fmaxf(v, __shfl_xor(v, k, 64));
+        return v;
+    };
+    // binary16 of (sum of value x code) / (sum of code^2) over the groups in order, 0 where there is no support
+    auto joint_scale = [&](float value, int code) __attribute__((always_inline)) {
+        __syncthreads();
+        sums[t] = double2{(double)value, (double)code};
+        __syncthreads();
+        double num = 0, den = 0;
+#pragma unroll
+        for (int k = 0; k < ng; ++k) {
+            const double2 v = sums[first + k];
+            num = __builtin_fma(v.x, v.y, num);
+            den = __builtin_fma(v.y, v.y, den);
         }
-        dd[0] = d;
-        dd[1] = (max_s <= eps) ? 1.0f : dm;
-        code[0] = (uint8_t)((max_s <= eps ? 1 : 0) | (max_m > eps ? 2 : 0));
-    }
-    __syncthreads();
-    const bool dead = (code[0] & 1) != 0;          // all scales vanish: d = 0, codes 0, dm stays 1
-    const bool have_min = (code[0] & 2) != 0;
-    __syncthreads();
+        const float q = (den > 1e-20) ? half_bits_to_float(float_to_half_bits((float)(num / den))) : 0.0f;
+        return fabsf(q) <= eps ? 0.0f : q;
+    };
+    const float max_s = block_max(fabsf(s)), max_m = block_max(fabsf(m));
+    const bool dead = max_s <= eps;  // all scales vanish: d = 0, codes 0, dm stays 1
+    float d = 0.0f, dm = 1.0f;
+    int sc = 0, mc = 0;
     auto snap_scale = [&](float s, float d) __attribute__((always_inline)) {
         return (s == 0.0f) ? 0 : max(0, min(scq, (int)lroundf(s / d)));
     };
@@ -356,339 +432,297 @@ __global__ __launch_bounds__(64) void encode_affine_kernel(const float* __restri
         return max(-bias, min(mq - bias, (int)lroundf(-m / dm)));
     };
     if (!dead) {
-        if (t < ng) {
-            sc_[t] = snap_scale(s_[t], dd[0]);
-            if (have_min) mc_[t] = snap_min(m_[t], dd[1]);
-        }
-        __syncthreads();
-        for (int iter = 0; iter < 5; ++iter) {
-            const float d = dd[0], dm = dd[1];
-            if (t < ng) {
-                const float eff_s = d * (float)sc_[t];
-                const float eff_m = -dm * (float)mc_[t];
-                if (eff_s != 0.0f) {
-                    double sw = 0, sl = 0, sl2 = 0, sx = 0, sxl = 0;
-                    for (int i = 0; i < gsz; ++i) {
-                        const float l = unit_level(bits, unit_nearest_dev((x[i] - eff_m) / eff_s, bits));
-                        sw += 1.0; sl += l; sl2 += l * l;  // the square is a float product here, not fused
-                        sx += (double)x[i]; sxl = __builtin_fma((double)x[i], (double)l, sxl);
-                    }
-                    const double D = fms2(sw, sl2, sl, sl);
-                    if (D > 1e-20) {
-                        s_[t] = (float)(fms2(sw, sxl, sx, sl) / D);
-                        m_[t] = (float)(fms2(sl2, sx, sl, sxl) / D);
-                    }
-                }
-                sc_[t] = snap_scale(s_[t], d);
-            }
-            __syncthreads();
-            if (t == 0) {
-                double num = 0, den = 0;
-                for (int g = 0; g < ng; ++g) {
-                    num = __builtin_fma((double)s_[g], (double)sc_[g], num);
-                    den = __builtin_fma((double)sc_[g], (double)sc_[g], den);
-                }
-                float nd = (den > 1e-20) ? half_bits_to_float(float_to_half_bits((float)(num / den))) : 0.0f;
-                if (fabsf(nd) <= eps) nd = 0.0f;
-                dd[0] = nd;
-            }
-            if (t < ng) mc_[t] = (fabsf(dm) > eps) ? snap_min(m_[t], dm) : 0;
-            __syncthreads();
-            if (t == 0) {
-                double num2 = 0, den2 = 0;
-                for (int g = 0; g < ng; ++g) {
-                    num2 = __builtin_fma(-(double)m_[g], (double)mc_[g], num2);
-                    den2 = __builtin_fma((double)mc_[g], (double)mc_[g], den2);
-                }
-                float ndm = (den2 > 1e-20) ? half_bits_to_float(float_to_half_bits((float)(num2 / den2))) : 0.0f;
-                if (fabsf(ndm) <= eps) ndm = 0.0f;
-                dd[1] = ndm;
-            }
-            __syncthreads();
-        }
+        d = half_bits_to_float(float_to_half_bits(max_s / (float)scq));
+        if (max_m > eps) dm = half_bits_to_float(float_to_half_bits(max_m / (float)bias));
+        sc = snap_scale(s, d);
+        if (max_m > eps) mc = snap_min(m, dm);
     }
-    // ---- codes
-    const float d = dd[0], dm = dd[1];
-    if (t < ng) {
-        const float eff_s = d * (float)sc_[t];
-        const float eff_m = -dm * (float)mc_[t];
-        for (int i = 0; i < gsz; ++i)
-            code[t * gsz + i] = (eff_s == 0.0f) ? 0 : (uint8_t)unit_nearest_dev((x[i] - eff_m) / eff_s, bits);
+#pragma unroll 1
+    for (int iter = 0; iter < 5; ++iter) {  // (dead blocks come along for the barriers and keep their values)
+        const float eff_s = d * (float)sc;
+        const float eff_m = -dm * (float)mc;
+        if (eff_s != 0.0f) {
+            level_pass<bits, gsz>(x, eff_m, eff_s, odd, clear, [&](int i, float n) __attribute__((always_inline)) {
+                const float l = n * unit;
+                sl += (double)l;
+                sl2 += (double)(l * l);  // the square is a float product here, not fused
+                sxl = __builtin_fma((double)x[i], (double)l, sxl);
+            });
+            solve(s, m);
+        }
+        if (!dead) sc = snap_scale(s, d);
+        const float nd = joint_scale(s, sc);
+        if (!dead) mc = (fabsf(dm) > eps) ? snap_min(m, dm) : 0;
+        const float ndm = joint_scale(-m, mc);
+        if (!dead) { d = nd; dm = ndm; }
+    }
+    // ---- payload: levels | scale codes | biased min codes | binary16 d | binary16 dm, one LSB-first stream.  A lane's
+    // levels are whole bytes; the header is put together from the lanes' codes in LDS.
+    constexpr int lane_bytes = gsz * bits / 8, lane_dwords = (lane_bytes + 3) / 4;
+    uint32_t packed[lane_dwords];
+    auto clear_packed = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < lane_dwords; ++i) packed[i] = 0;
+    };
+    const float eff_s = d * (float)sc;
+    const float eff_m = -dm * (float)mc;
+    clear_packed();
+    if (eff_s != 0.0f) {
+        level_pass<bits, gsz>(x, eff_m, eff_s, odd, clear_packed, [&](int i, float n) __attribute__((always_inline)) {
+            const uint32_t c = (uint32_t)n;
+            packed[i * bits / 32] |= c << (i * bits % 32);
+            if (i * bits % 32 + bits > 32) packed[i * bits / 32 + 1] |= c >> (32 - i * bits % 32);
+        });
     }
     __syncthreads();
-    // ---- payload: levels | scale codes | biased min codes | binary16 d | binary16 dm, one LSB-first stream
-    constexpr int lev_bits = 256 * bits, sc_end = lev_bits + ng * sp.scb, mn_end = sc_end + ng * sp.mb;
-    const uint32_t dh = float_to_half_bits(d) | (float_to_half_bits(dm) << 16);
+    hcode[t] = (uint8_t)sc;
+    hcode[64 + t] = (uint8_t)(mc + bias);
+    __syncthreads();
+    if (mine >= nblocks) return;
     uint8_t* p = dst + blk * (int64_t)sp.block_bytes;
-    for (int byte = t; byte < sp.block_bytes; byte += 64) {
+#pragma unroll
+    for (int i = 0; i < lane_bytes / 4; ++i) __builtin_memcpy(p + g * lane_bytes + 4 * i, &packed[i], 4);
+    if constexpr (lane_bytes % 4 == 2) __builtin_memcpy(p + g * lane_bytes + lane_bytes - 2, &packed[lane_dwords - 1], 2);
+    constexpr int head = 32 * bits, sc_end = ng * sp.scb, mn_end = sc_end + ng * sp.mb;
+    const uint32_t dh = float_to_half_bits(d) | (float_to_half_bits(dm) << 16);
+    for (int byte = g; byte < sp.block_bytes - head; byte += ng) {
         uint32_t v = 0;
 #pragma unroll
         for (int b = 0; b < 8; ++b) {
             const int pos = 8 * byte + b;
             uint32_t bit;
-            if (pos < lev_bits) bit = ((uint32_t)code[pos / bits] >> (pos % bits)) & 1u;
-            else if (pos < sc_end) bit = ((uint32_t)sc_[(pos - lev_bits) / sp.scb] >> ((pos - lev_bits) % sp.scb)) & 1u;
-            else if (pos < mn_end) bit = ((uint32_t)(mc_[(pos - sc_end) / sp.mb] + bias) >> ((pos - sc_end) % sp.mb)) & 1u;
+            if (pos < sc_end) bit = ((uint32_t)hcode[first + pos / sp.scb] >> (pos % sp.scb)) & 1u;
+            else if (pos < mn_end) bit = ((uint32_t)hcode[64 + first + (pos - sc_end) / sp.mb] >> ((pos - sc_end) % sp.mb)) & 1u;
             else bit = (dh >> (pos - mn_end)) & 1u;
             v |= bit << b;
         }
-        p[byte] = (uint8_t)v;
+        p[head + byte] = (uint8_t)v;
+    }
+}
+
+// (all launchers of this kind: `job` rides along as the first workgroup)
+template <int FMT>
+static void launch_encode_affine(const float* w, int64_t nblocks, uint8_t* dst, const ShortJob& job, hipStream_t s) {
+    constexpr int per_wave = 64 / (256 / spec_of(FMT).gsz);
+    const int64_t grid = (nblocks + per_wave - 1) / per_wave + (job.L.n > 0);
+    hipLaunchKernelGGL(encode_affine_kernel<FMT>, dim3((unsigned)grid), dim3(64), 0, s, w, dst, nblocks, job);
+}
+
+// ---- encoders with one scale per run of weights (a group of 32 or a block of 256)
+// (Comp8Team and ordered_sums, which the short blocks use too, are in tfq_encode_short.hpp)
+// `width` (<= 48) bits of v at bit `pos` of an LDS image that starts out as zeros
+__device__ __forceinline__ void image_bits(uint32_t* img, uint32_t pos, uint64_t v, int width) {
+    const uint32_t sh = pos & 31u;
+    atomicOr(&img[pos >> 5], (uint32_t)(v << sh));
+    if (sh + (uint32_t)width > 32u) atomicOr(&img[(pos >> 5) + 1], (uint32_t)((v << sh) >> 32));
+    if (sh + (uint32_t)width > 64u) atomicOr(&img[(pos >> 5) + 2], (uint32_t)(v >> (64u - sh)));
+}
+// the codes of PER consecutive weights from weight `i0` (a multiple of 4) into a lattice block's image:
+// [binary16 scale][16 codes, the last a bit short] x 16
+template <int BITS, int PER>
+__device__ __forceinline__ void image_lattice(uint32_t* img, int i0, const uint32_t (&code)[PER]) {
+#pragma unroll
+    for (int k = 0; k < PER; k += 4) {
+        const int i = i0 + k;
+        const bool slot = (i & 15) == 12;  // weight i + 3 gives up its low bit
+        uint64_t v = (uint64_t)code[k] | ((uint64_t)code[k + 1] << BITS) | ((uint64_t)code[k + 2] << (2 * BITS));
+        v |= (uint64_t)(slot ? code[k + 3] >> 1 : code[k + 3]) << (3 * BITS);
+        image_bits(img, (uint32_t)(16 + BITS * i - (i >> 4)), v, 4 * BITS - (slot ? 1 : 0));
     }
 }
 
 // Companded 8-bit encoders: Q_G_8 (quant_grp8_compound, src/codec/block_codec.cpp:365-388, a scale per 32
 // weights) and Q_8 (quant_lattice with bits = 8, :458-470, one scale per block, 7-bit slots), both on
 // comp8_fit_scale_fp16 (:306-358): three least-squares seeds, 14 golden-section steps on the true squared
-// error over [0.75 s, 1.25 s], then the +-4 neighbouring binary16 values.  One wavefront per scale group.
-// Every evaluation is split so that the result is the reference's: the lanes do the per-weight part in
-// parallel (nearest level by bisection, residual r = level * s - w as one fused multiply-add in double),
-// lane 0 then adds r * r in index order with the same fused operations the reference's Release build uses.
-// The search state lives in every lane (all decisions come from values lane 0 publishes).
-template <int CNT>
-struct Comp8Team {
-    float* lv;       // 256 levels, LDS
-    double* buf;     // 2 * CNT doubles, LDS
-    double* res;     // 2 doubles, LDS
-    const float* w;  // this group's weights, LDS
-    int lane;
-    static constexpr int PER = CNT / 64 ? CNT / 64 : 1;  // weights per lane
-    __device__ __forceinline__ bool mine(int k, int* i) const { *i = lane * PER + k; return *i < CNT; }
-    __device__ __forceinline__ uint32_t nearest(float v) const {
-        if (v <= lv[0]) return 0;
-        if (v >= lv[255]) return 255;
-        int lo = 0, hi = 255;
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) / 2;
-            if (lv[mid] <= v) lo = mid; else hi = mid;
-        }
-        return (v - lv[lo] <= lv[hi] - v) ? (uint32_t)lo : (uint32_t)hi;
-    }
-    __device__ double sq_err(double s) const {
-        const double inv = 1.0 / s;
-        for (int k = 0; k < PER; ++k) {
-            int i;
-            if (mine(k, &i)) buf[i] = __builtin_fma((double)lv[nearest((float)((double)w[i] * inv))], s, -(double)w[i]);
-        }
-        __syncthreads();
-        if (lane == 0) {
-            double err = 0.0;
-            for (int i = 0; i < CNT; ++i) err = __builtin_fma(buf[i], buf[i], err);
-            res[0] = err;
-        }
-        __syncthreads();
-        const double e = res[0];
-        __syncthreads();
-        return e;
-    }
-    // false when the refit has no support (den <= 1e-20)
-    __device__ bool seed(double s, double* out) const {
-        for (int k = 0; k < PER; ++k) {
-            int i;
-            if (mine(k, &i)) buf[i] = (double)lv[nearest((float)((double)w[i] / s))];
-        }
-        __syncthreads();
-        if (lane == 0) {
-            double num = 0.0, den = 0.0;
-            for (int i = 0; i < CNT; ++i) {
-                num = __builtin_fma((double)w[i], buf[i], num);
-                den = __builtin_fma(buf[i], buf[i], den);
-            }
-            res[0] = num;
-            res[1] = den;
-        }
-        __syncthreads();
-        const double num = res[0], den = res[1];
-        __syncthreads();
-        if (!(den > 1e-20)) return false;
-        *out = num / den;
-        return true;
-    }
-    __device__ float fit(double maxa) const {
-        if (!(maxa > 0.0)) return 0.0f;
-        const double hi = maxa * 1.0000001;
-        double s = maxa;
-        for (int it = 0; it < 3; ++it) {
-            double ls;
-            if (!seed(s, &ls)) break;
-            s = ls < hi ? ls : hi;
-        }
-        double a = s * 0.75, b = s * 1.25;
-        const double phi = 0.6180339887498949;
-        double c = __builtin_fma(-phi, b - a, b), d = __builtin_fma(phi, b - a, a);
-        double fc = sq_err(c), fd = sq_err(d);
-        for (int it = 0; it < 14 && (b - a) > 1e-11 * (a + b); ++it) {
-            if (fc < fd) {
-                b = d; d = c; fd = fc;
-                c = __builtin_fma(-phi, b - a, b); fc = sq_err(c);
-            } else {
-                a = c; c = d; fc = fd;
-                d = __builtin_fma(phi, b - a, a); fd = sq_err(d);
-            }
-        }
-        double raw = 0.5 * (a + b);
-        const double fraw = sq_err(raw);
-        if (fraw > fc && fc <= fd) raw = c;
-        else if (fraw > fd) raw = d;
-        const uint32_t hf = float_to_half_bits((float)raw);
-        float best = half_bits_to_float(hf);
-        double best_e = sq_err((double)best);
-        for (int delta = -4; delta <= 4; ++delta) {
-            if (delta == 0) continue;
-            const int hc = (int)hf + delta;
-            if (hc < 0 || hc > 0xFFFF) continue;
-            const float cand = half_bits_to_float((uint32_t)hc);
-            if (!(cand > 0.0f) || !((double)cand <= hi * 1.02)) continue;
-            const double e = sq_err((double)cand);
-            if (e < best_e) { best_e = e; best = cand; }
-        }
-        return best;
-    }
-};
-
-// FMT = Q_G_8: grid = 8 groups per block, a wavefront each (32 lanes hold a weight).  FMT = Q_8: a wavefront
-// per block, four weights per lane.
-template <int FMT>
-__global__ __launch_bounds__(64) void encode_comp8_kernel(const float* __restrict__ wg, uint8_t* __restrict__ dst, float smult) {
+// error over [0.75 s, 1.25 s], then the +-4 neighbouring binary16 values, about 29 evaluations of every weight.
+// Bound by vector instructions.  The grid is a line to within 0.01 of a step, so the two levels around a value are
+// known from one multiply-add (the level below may be missed by one where the value lies on a level; both pairs then
+// give that level) and the comparison of the two distances is the reference's; a bisection was eight dependent LDS
+// reads.  58.7 M weights of Q_G_8: 11.4 ms with a wavefront per group, bisection and lane 0 adding, 0.94 ms; Q_8:
+// 9.84 and 1.38 ms.  Lanes per run: as few as leave a wavefront per SIMD.
+template <int FMT, int T>
+__global__ __launch_bounds__(64) void encode_comp8_kernel(const float* __restrict__ wg, uint8_t* __restrict__ dst, float smult, int64_t nunits, ShortJob job) {
     constexpr bool GROUPED = spec_of(FMT).codec == Codec::Grp8;
-    constexpr int CNT = GROUPED ? 32 : 256;
+    constexpr int CNT = GROUPED ? 32 : 256, PER = CNT / T, TEAMS = 64 / T;
     __shared__ float lv[256];
-    __shared__ float w[CNT];
-    __shared__ double buf[CNT];
-    __shared__ double res[2];
-    __shared__ uint8_t code[CNT];
-    const int lane = threadIdx.x;
-    const int64_t unit = blockIdx.x;  // group or block
+    __shared__ uint32_t img[GROUPED ? 1 : TEAMS * 64];
+    __shared__ Team short_team;
+    const int with_short = job.L.n > 0;
+    if (with_short && blockIdx.x == 0) { encode_short_block<FMT>(job, short_team); return; }
+    const int lane = threadIdx.x, tl = lane % T;
+    const int64_t mine = (int64_t)(blockIdx.x - with_short) * TEAMS + lane / T;  // group or block
+    const int64_t unit = mine < nunits ? mine : nunits - 1;       // past the end: the last one again, stored by nobody
     for (int i = lane; i < 256; i += 64) lv[i] = __uint_as_float(kComp8Bits[i]);
-    for (int i = lane; i < CNT; i += 64) w[i] = wg[unit * CNT + i];
-    __syncthreads();
+    if constexpr (!GROUPED)
+        for (int i = lane; i < TEAMS * 64; i += 64) img[i] = 0;
+    Comp8Team<CNT, T> team;
+    team.lv = lv;
+    team.first = lane - tl;
     float m = 0.0f;
-    for (int i = lane; i < CNT; i += 64) m = fmaxf(m, fabsf(w[i]));
 #pragma unroll
-    for (int sft = 32; sft >= 1; sft >>= 1) m = fmaxf(m, __shfl_xor(m, sft, 64));
-    Comp8Team<CNT> team{lv, buf, res, w, lane};
-    const float s = team.fit((double)m) * smult;  // the _K tiers try scaled copies of the fitted scale
-    for (int i = lane; i < CNT; i += 64) code[i] = (uint8_t)((s > 0.0f) ? team.nearest(w[i] / s) : 0u);
+    for (int k = 0; k < PER; k += 4) {
+        float4 v;  // (the caller's pointer is aligned to a float only)
+        __builtin_memcpy(&v, wg + unit * CNT + tl * PER + k, 16);
+        team.w[k] = v.x; team.w[k + 1] = v.y; team.w[k + 2] = v.z; team.w[k + 3] = v.w;
+    }
+#pragma unroll
+    for (int k = 0; k < PER; ++k) m = fmaxf(m, fabsf(team.w[k]));
+#pragma unroll
+    for (int sft = T / 2; sft >= 1; sft >>= 1) m = fmaxf(m, __shfl_xor(m, sft, 64));
     __syncthreads();
+    const float s = team.fit((double)m) * smult;  // the _K tiers try scaled copies of the fitted scale
+    uint32_t code[PER];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) code[k] = (s > 0.0f) ? team.nearest(team.w[k] / s) : 0u;
     const uint32_t h = float_to_half_bits(s);
     if constexpr (GROUPED) {
+        if (mine >= nunits) return;
         uint8_t* p = dst + (unit >> 3) * 272;
         const int g = (int)(unit & 7);
-        if (lane < 32) p[32 * g + lane] = code[lane];
-        if (lane == 0) { p[256 + 2 * g] = (uint8_t)(h & 0xFF); p[257 + 2 * g] = (uint8_t)(h >> 8); }
-    } else {
-        // [binary16 scale][256 codes, every 16th with 7 bits (the even index below it)]: 16 + 16 * 127 bits
-        uint8_t* p = dst + unit * 256;
-        for (int byte = lane; byte < 256; byte += 64) {
-            uint32_t v = 0;
 #pragma unroll
-            for (int b = 0; b < 8; ++b) {
-                const int pos = 8 * byte + b;
-                uint32_t bit;
-                if (pos < 16) bit = (h >> pos) & 1u;
-                else {
-                    const int q = pos - 16, c = q / 127, r = q - 127 * c;
-                    const int k = r / 8 < 15 ? r / 8 : 15, off = r - 8 * k;
-                    const uint32_t idx = code[16 * c + k];
-                    bit = ((k == 15 ? idx >> 1 : idx) >> off) & 1u;
-                }
-                v |= bit << b;
-            }
-            p[byte] = (uint8_t)v;
+        for (int k = 0; k < PER; k += 4) {
+            const uint32_t v = code[k] | (code[k + 1] << 8) | (code[k + 2] << 16) | (code[k + 3] << 24);
+            __builtin_memcpy(p + 32 * g + tl * PER + k, &v, 4);
         }
+        if (tl == 0) { p[256 + 2 * g] = (uint8_t)(h & 0xFF); p[257 + 2 * g] = (uint8_t)(h >> 8); }
+    } else {
+        uint32_t* mimg = img + (lane / T) * 64;
+        image_lattice<8, PER>(mimg, tl * PER, code);
+        if (tl == 0) atomicOr(&mimg[0], h);
+        __syncthreads();
+        const int64_t b0 = (int64_t)(blockIdx.x - with_short) * TEAMS;
+        const int words = (int)min((int64_t)TEAMS, nunits - b0) * 64;
+        for (int i = lane; i < words; i += 64) __builtin_memcpy(dst + b0 * 256 + 4 * i, &img[i], 4);
     }
+}
+
+// Lanes per run: 32 weights per lane keep the index-order sums short in total; where that leaves SIMDs of the chip
+// without a wavefront, runs are spread over more lanes.
+template <int FMT>
+static void launch_encode_comp8(const float* w, int64_t nblocks, uint8_t* dst, float smult, const ShortJob& job, hipStream_t s) {
+    constexpr bool GROUPED = spec_of(FMT).codec == Codec::Grp8;
+    constexpr int T = GROUPED ? 1 : 8, SPREAD = GROUPED ? 4 : 16;
+    const int64_t units = GROUPED ? nblocks * 8 : nblocks;
+    const bool wide = (units * T + 63) / 64 < 1024;
+    const unsigned grid = (unsigned)((units * (wide ? SPREAD : T) + 63) / 64 + (job.L.n > 0));
+    if (grid == 0) return;
+    if (wide) hipLaunchKernelGGL((encode_comp8_kernel<FMT, SPREAD>), dim3(grid), dim3(64), 0, s, w, dst, smult, units, job);
+    else hipLaunchKernelGGL((encode_comp8_kernel<FMT, T>), dim3(grid), dim3(64), 0, s, w, dst, smult, units, job);
 }
 
 // Plain lattice encoders Q_4 / Q_2 (quant_lattice, src/codec/block_codec.cpp:443-497) and the fixed-codebook
 // encoders Q_3 / Q_6 / Q_12 (quant_fixed_codebook, :624-663), which differ in the level table only:
 // s = absmax / top level * smult, `iters` least-squares refits over the nearest levels, binary16; codes are the
 // nearest level of w / s, slots (every 16th weight) keep the even index below.  The base ids run 2 (lattice) or
-// 3 (fixed) refits with smult 1; the _K tiers try more.  A wavefront per block; sums in index order on lane 0.
-template <int FMT>
+// 3 (fixed) refits with smult 1; the _K tiers try more.  Teams of eight lanes, of sixteen where that leaves SIMDs without a wavefront.
+// The tables of up to sixteen levels are looked up by bucket: a bucket is narrower than the distance of two
+// midpoints, so it names the only two levels that can be nearest; the comparison of their distances is the
+// reference's, and so is the scan over all levels that far-off values take.  58.7 M weights of Q_4: 1.30 ms with a block
+// per wavefront, the scan for every weight and lane 0 adding, 265 us.
+template <int FMT, int T>
 __global__ __launch_bounds__(64) void encode_lattice_kernel(const float* __restrict__ wg, uint8_t* __restrict__ dst,
-                                                            int iters, float smult) {
+                                                            int iters, float smult, int64_t nblocks, ShortJob job) {
     constexpr Spec sp = spec_of(FMT);
-    constexpr int bits = sp.bits, BB = sp.block_bytes, CHUNK = 16 * bits - 1, NL = 1 << bits;
+    constexpr int bits = sp.bits, BB = sp.block_bytes, NL = 1 << bits, PER = 256 / T, TEAMS = 64 / T;
     constexpr bool FIXED = sp.codec == Codec::Fixed;
     constexpr bool SEARCH = FIXED && bits > 3;  // ascending quantile table: binary search on |v| (:596-622)
     __shared__ float tab[NL];
-    __shared__ float w[256];
-    __shared__ float lev[256];
-    __shared__ float sres;
-    __shared__ uint16_t code[256];
-    const int lane = threadIdx.x;
-    const int64_t blk = blockIdx.x;
+    __shared__ float4 bucket[SEARCH ? 1 : 64];  // (level lo, level lo + 1, lo)
+    __shared__ uint32_t img[TEAMS * BB / 4];
+    __shared__ Team short_team;
+    const int with_short = job.L.n > 0;
+    if (with_short && blockIdx.x == 0) { encode_short_block<FMT>(job, short_team); return; }
+    const int lane = threadIdx.x, tl = lane % T, first = lane - tl;
+    const int64_t mine = (int64_t)(blockIdx.x - with_short) * TEAMS + lane / T;
+    const int64_t blk = mine < nblocks ? mine : nblocks - 1;  // past the end: the last block again, stored by nobody
     for (int i = lane; i < NL; i += 64) tab[i] = FIXED ? fixed_value(bits, (uint32_t)i) : grid_value(bits, (uint32_t)i);
-    for (int i = lane; i < 256; i += 64) w[i] = wg[blk * 256 + i];
+    for (int i = lane; i < TEAMS * BB / 4; i += 64) img[i] = 0;
     __syncthreads();
+    const float reach = tab[NL - 1] + 0.1f, per_unit = 32.0f / reach;  // buckets over [-reach, reach]
+    if constexpr (!SEARCH) {
+        const float edge = (float)lane * (reach / 32.0f) - reach - 0.001f;
+        int lo = 0;
+        for (int i = 1; i < NL - 1; ++i) lo += 0.5f * (tab[i - 1] + tab[i]) < edge;
+        bucket[lane] = float4{tab[lo], tab[lo + 1], __int_as_float(lo), 0.0f};
+        __syncthreads();
+    }
+    float w[PER];
     float m = 0.0f;
-    for (int i = lane; i < 256; i += 64) m = fmaxf(m, fabsf(w[i]));
 #pragma unroll
-    for (int sft = 32; sft >= 1; sft >>= 1) m = fmaxf(m, __shfl_xor(m, sft, 64));
-    auto nearest = [&](float v) __attribute__((always_inline)) {
+    for (int k = 0; k < PER; k += 4) {
+        float4 v;  // (the caller's pointer is aligned to a float only)
+        __builtin_memcpy(&v, wg + blk * 256 + tl * PER + k, 16);
+        w[k] = v.x; w[k + 1] = v.y; w[k + 2] = v.z; w[k + 3] = v.w;
+    }
+#pragma unroll
+    for (int k = 0; k < PER; ++k) m = fmaxf(m, fabsf(w[k]));
+#pragma unroll
+    for (int sft = T / 2; sft >= 1; sft >>= 1) m = fmaxf(m, __shfl_xor(m, sft, 64));
+    auto nearest = [&](float v, float* level) __attribute__((always_inline)) {
         if constexpr (SEARCH) {
             constexpr int half = NL / 2;
             const float a = fabsf(v);
-            int lo = half, hi = NL - 1;
-            while (lo < hi) {
-                const int mid = (lo + hi) / 2;
-                if (tab[mid] < a) lo = mid + 1; else hi = mid;
-            }
+            int lo = half;  // the first level of the upper half that is not below a, the last one at most
+#pragma unroll
+            for (int len = half / 2; len >= 1; len /= 2) lo += tab[lo + len - 1] < a ? len : 0;
             if (lo > half) {
                 const float d0 = a - tab[lo - 1];
                 const float d1 = tab[lo] - a;
                 if (d1 >= d0) --lo;
             }
-            return (v >= 0.0f) ? (uint32_t)lo : (uint32_t)(half - 1 - (lo - half));
+            const uint32_t best = (v >= 0.0f) ? (uint32_t)lo : (uint32_t)(half - 1 - (lo - half));
+            *level = tab[best];
+            return best;
         } else {
-            uint32_t best = 0;
-            float bd = fabsf(v - tab[0]);
-            for (int i = 1; i < NL; ++i) {
-                const float d = fabsf(v - tab[i]);
-                if (d < bd) { bd = d; best = (uint32_t)i; }
+            const float4 e = bucket[(int)fminf(fmaxf((v + reach) * per_unit, 0.0f), 63.0f)];
+            const bool up = fabsf(v - e.y) < fabsf(v - e.x);
+            uint32_t best = (uint32_t)__float_as_int(e.z) + (up ? 1u : 0u);
+            float l = up ? e.y : e.x;
+            if (!(fabsf(v) <= 64.0f)) {  // distances may round to the same number, and a NaN is level 0: the scan decides
+                best = 0;
+                float bd = fabsf(v - tab[0]);
+                for (int i = 1; i < NL; ++i) {
+                    const float d = fabsf(v - tab[i]);
+                    if (d < bd) { bd = d; best = (uint32_t)i; }
+                }
+                l = tab[best];
             }
+            *level = l;
             return best;
         }
     };
     float s = (m > 1e-30f) ? m / tab[NL - 1] * smult : 0.0f;
     if (s > 0.0f) {
+#pragma unroll 1
         for (int it = 0; it < iters; ++it) {
-            for (int i = lane; i < 256; i += 64) lev[i] = tab[nearest(w[i] / s)];
-            __syncthreads();
-            if (lane == 0) {
-                double num = 0.0, den = 0.0;
-                for (int i = 0; i < 256; ++i) {
-                    num = __builtin_fma((double)w[i], (double)lev[i], num);
-                    den = __builtin_fma((double)lev[i], (double)lev[i], den);
+            float l[PER];
+#pragma unroll
+            for (int k = 0; k < PER; ++k) nearest(w[k] / s, &l[k]);
+            double num, den;
+            ordered_sums<T>(first, num, den, [&](double& a, double& b) __attribute__((always_inline)) {
+#pragma unroll
+                for (int k = 0; k < PER; ++k) {
+                    a = __builtin_fma((double)w[k], (double)l[k], a);
+                    b = __builtin_fma((double)l[k], (double)l[k], b);
                 }
-                sres = (den > 1e-20) ? (float)(num / den) : s;
-            }
-            __syncthreads();
-            s = sres;
-            __syncthreads();
+            });
+            if (den > 1e-20) s = (float)(num / den);
         }
     }
     if (!(s > 0.0f)) s = 0.0f;
-    for (int i = lane; i < 256; i += 64) code[i] = (uint16_t)nearest((s == 0.0f) ? 0.0f : w[i] / s);
-    __syncthreads();
-    const uint32_t h = float_to_half_bits(s);
-    uint8_t* p = dst + blk * BB;
-    for (int byte = lane; byte < BB; byte += 64) {
-        uint32_t v = 0;
+    uint32_t code[PER];
 #pragma unroll
-        for (int b = 0; b < 8; ++b) {
-            const int pos = 8 * byte + b;
-            uint32_t bit;
-            if (pos < 16) bit = (h >> pos) & 1u;
-            else {
-                const int q = pos - 16, c = q / CHUNK, r = q - CHUNK * c;
-                const int k = r / bits < 15 ? r / bits : 15, off = r - bits * k;
-                const uint32_t idx = code[16 * c + k];
-                bit = ((k == 15 ? idx >> 1 : idx) >> off) & 1u;
-            }
-            v |= bit << b;
-        }
-        p[byte] = (uint8_t)v;
+    for (int k = 0; k < PER; ++k) {
+        float l;
+        code[k] = nearest((s == 0.0f) ? 0.0f : w[k] / s, &l);
     }
+    uint32_t* mimg = img + (lane / T) * (BB / 4);
+    image_lattice<bits, PER>(mimg, tl * PER, code);
+    if (tl == 0) atomicOr(&mimg[0], float_to_half_bits(s));
+    __syncthreads();
+    const int64_t b0 = (int64_t)(blockIdx.x - with_short) * TEAMS;
+    const int words = (int)min((int64_t)TEAMS, nblocks - b0) * (BB / 4);
+    for (int i = lane; i < words; i += 64) __builtin_memcpy(dst + b0 * BB + 4 * i, &img[i], 4);
 }
 
 // 12-bit compound encoder (quant_grp12_compound, src/codec/block_codec.cpp:969-1004): every group of 32 weights
@@ -908,115 +942,153 @@ __device__ __forceinline__ int q6k_level_dev(float ratio) {
     return max(-32, min(31, q6k_round_dev(ratio)));
 }
 
-// passes / giters / polish / joint: the search effort (2, 4, 3, 3 for Q_G_6 and _K_L)
-__global__ __launch_bounds__(64) void encode_q6k_kernel(const float* __restrict__ wg, uint8_t* __restrict__ dst,
-                                                        int giters, int polish, int joint) {
+// giters / polish / joint: the search effort (4, 3, 3 for Q_G_6 and _K_L).  A lane owns a group of 16, a wavefront four
+// blocks, as in encode_affine_kernel, and levels are taken from a product by 1 / scale in the same way: its distance to
+// the correctly rounded quotient is below 2^-22 |x / scale| and the quotient matters up to 32, so 0.5 - 2^-16 decides.
+// 58.7 M weights: 1.96 ms with one block per wavefront, 280 us.
+__global__ __launch_bounds__(64, 4) void encode_q6k_kernel(const float* __restrict__ wg, uint8_t* __restrict__ dst,
+                                                           int giters, int polish, int joint, int64_t nblocks, ShortJob job) {
     constexpr int ng = 16;
     constexpr float eps = 1e-15f;
-    __shared__ float w[256];
-    __shared__ float s_[16];
-    __shared__ int sc_[16];
-    __shared__ float dsh;
-    __shared__ uint8_t code[256];
-    const int64_t blk = blockIdx.x;
-    const int t = threadIdx.x;
-    for (int i = t; i < 256; i += 64) w[i] = wg[blk * 256 + i];
-    __syncthreads();
-    const float* x = w + (t & 15) * 16;
-    auto refit16 = [&](float scale, float* out) __attribute__((always_inline)) {
-        double num = 0.0, den = 0.0;
+    __shared__ double2 sums[64];
+    __shared__ uint32_t img[210];  // four blocks
+    __shared__ Team short_team;
+    const int with_short = job.L.n > 0;
+    if (with_short && blockIdx.x == 0) { encode_short_block<TFQ_Q_G_6>(job, short_team); return; }
+    const int t = threadIdx.x, g = t & (ng - 1), first = t & ~(ng - 1);
+    const int64_t mine = (int64_t)(blockIdx.x - with_short) * 4 + t / ng;
+    const int64_t blk = mine < nblocks ? mine : nblocks - 1;  // past the end: the last block again, stored by nobody
+    float x[16];
+    float maxa = 0.0f;
+    uint32_t top_bits = 0;
+#pragma unroll
+    for (int i = 0; i < 16; i += 4) {
+        float4 v;  // (the caller's pointer is aligned to a float only)
+        __builtin_memcpy(&v, wg + blk * 256 + g * 16 + i, 16);
+        x[i] = v.x; x[i + 1] = v.y; x[i + 2] = v.z; x[i + 3] = v.w;
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        maxa = fmaxf(maxa, fabsf(x[i]));
+        top_bits = max(top_bits, __float_as_uint(x[i]) & 0x7FFFFFFFu);
+    }
+    const bool odd = top_bits > 0x71000000u;  // above 2^99, infinite or NaN
+    // use(i, l) for every weight, l (float) = its level for `scale`; `reset` forgets what `use` gathered
+    auto pass = [&](float scale, auto&& reset, auto&& use) __attribute__((always_inline)) {
+        const float r = 1.0f / scale;
+        float far = 0.0f;
+        reset();
+#pragma unroll
         for (int i = 0; i < 16; ++i) {
-            const int l = q6k_level_dev(x[i] / scale);
-            num = __builtin_fma((double)x[i], (double)l, num);
-            den = __builtin_fma((double)l, (double)l, den);
+            const float q = __builtin_amdgcn_fmed3f(x[i] * r, -32.0f, 31.0f);
+            const float n = __builtin_rintf(q);
+            far = fmaxf(far, fabsf(q - n));
+            use(i, n);
         }
+        if (odd || !(far <= 0.5f - 1.52587890625e-5f) || !(fabsf(r) < 1e37f)) {
+            reset();
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                use(i, (float)q6k_level_dev(x[i] / scale));
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    };
+    auto refit16 = [&](float scale, float* out) __attribute__((always_inline)) {
+        double num, den;
+        pass(scale, [&]() __attribute__((always_inline)) { num = 0.0; den = 0.0; },
+             [&](int i, float n) __attribute__((always_inline)) {
+                 const double l = (double)n;
+                 num = __builtin_fma((double)x[i], l, num);
+                 den = __builtin_fma(l, l, den);
+             });
         if (den > 1e-20) *out = (float)(num / den);
     };
-    if (t < ng) {
-        float maxa = 0.0f;
-        for (int i = 0; i < 16; ++i) maxa = fmaxf(maxa, fabsf(x[i]));
-        float sg = (maxa > eps) ? maxa / 32.0f : 0.0f;
-        if (fabsf(sg) <= eps) sg = 0.0f;
-        else {
-            for (int iter = 0; iter < giters; ++iter) refit16(sg, &sg);
-            float best_s = sg;
-            double best = 1e300;
-            for (int k = -polish; k <= polish; ++k) {
-                if (k == 0) continue;
-                const float cs = sg * __builtin_fmaf(0.05f, (float)k, 1.0f);
-                double e = 0.0;
-                for (int i = 0; i < 16; ++i) {
-                    const float d = __builtin_fmaf(cs, (float)q6k_level_dev(x[i] / cs), -x[i]);
-                    e = __builtin_fma((double)d, (double)d, e);
+    float sg = (maxa > eps) ? maxa / 32.0f : 0.0f;
+    if (fabsf(sg) <= eps) sg = 0.0f;
+    else {
+#pragma unroll 1
+        for (int iter = 0; iter <= giters; ++iter) {  // the last one behind the polish
+            if (iter == giters) {
+                float best_s = sg;
+                double best = 1e300;
+#pragma unroll 1
+                for (int k = -polish; k <= polish; ++k) {
+                    if (k == 0) continue;
+                    const float cs = sg * __builtin_fmaf(0.05f, (float)k, 1.0f);
+                    double e;
+                    pass(cs, [&]() __attribute__((always_inline)) { e = 0.0; },
+                         [&](int i, float n) __attribute__((always_inline)) {
+                             const float d = __builtin_fmaf(cs, n, -x[i]);
+                             e = __builtin_fma((double)d, (double)d, e);
+                         });
+                    if (e < best) { best = e; best_s = cs; }
                 }
-                if (e < best) { best = e; best_s = cs; }
+                sg = best_s;
             }
-            sg = best_s;
             refit16(sg, &sg);
         }
-        s_[t] = sg;
-        sc_[t] = 0;
     }
-    __syncthreads();
-    float max_abs = 0.0f;
-    for (int g = 0; g < ng; ++g) max_abs = fmaxf(max_abs, fabsf(s_[g]));
-    if (max_abs <= eps) {
-        if (t == 0) dsh = 0.0f;
-        __syncthreads();
-    } else {
-        const float iscale = -128.0f / max_abs;
-        if (t == 0) dsh = 1.0f / iscale;
-        // the product feeds the rounding add directly: one fused operation in the reference's build
-        if (t < ng) sc_[t] = max(-127, min(127, (int)(__float_as_uint(__builtin_fmaf(iscale, s_[t], 12582912.f)) & 0x007fffffu) - 0x00400000));
-        __syncthreads();
-        for (int iter = 0; iter < joint; ++iter) {
-            const float d = dsh;
-            if (t < ng) {
-                const float eff = d * (float)sc_[t];
-                if (eff != 0.0f) {
-                    float fitted = 0.0f;
-                    refit16(eff, &fitted);
-                    s_[t] = fitted;
-                }
-                sc_[t] = (d == 0.0f) ? 0 : max(-127, min(127, q6k_round_dev(s_[t] / d)));
-            }
-            __syncthreads();
-            if (t == 0) {
-                double num = 0.0, den = 0.0;
-                for (int g = 0; g < ng; ++g) {
-                    num = __builtin_fma((double)s_[g], (double)sc_[g], num);
-                    den = __builtin_fma((double)sc_[g], (double)sc_[g], den);
-                }
-                float nd = (den > 1e-20) ? (float)(num / den) : 0.0f;
-                if (fabsf(nd) <= eps) nd = 0.0f;
-                dsh = nd;
-            }
-            __syncthreads();
-        }
-    }
-    const float d = dsh;
-    if (t < ng) {
-        const float eff = d * (float)sc_[t];
-        for (int i = 0; i < 16; ++i) code[t * 16 + i] = (uint8_t)(((eff == 0.0f) ? 0 : q6k_level_dev(x[i] / eff)) + 32);
-    }
-    __syncthreads();
-    const uint32_t dh = float_to_half_bits(d);
-    uint8_t* p = dst + blk * 210;
-    for (int byte = t; byte < 210; byte += 64) {
-        uint32_t v = 0;
-        if (byte < 192) {
+    float max_abs = fabsf(sg);
 #pragma unroll
-            for (int b = 0; b < 8; ++b) {
-                const int pos = 8 * byte + b;
-                v |= (((uint32_t)code[pos / 6] >> (pos % 6)) & 1u) << b;
-            }
-        } else if (byte < 208) {
-            v = (uint32_t)(uint8_t)(int8_t)sc_[byte - 192];
-        } else {
-            v = (dh >> (8 * (byte - 208))) & 0xFFu;
-        }
-        p[byte] = (uint8_t)v;
+    for (int k = ng / 2; k >= 1; k >>= 1) max_abs = fmaxf(max_abs, __shfl_xor(max_abs, k, 64));
+    const bool dead = max_abs <= eps;
+    float d = 0.0f;
+    int sc = 0;
+    if (!dead) {
+        const float iscale = -128.0f / max_abs;
+        d = 1.0f / iscale;
+        // the product feeds the rounding add directly: one fused operation in the reference's build
+        sc = max(-127, min(127, (int)(__float_as_uint(__builtin_fmaf(iscale, sg, 12582912.f)) & 0x007fffffu) - 0x00400000));
     }
+#pragma unroll 1
+    for (int iter = 0; iter < joint; ++iter) {  // (dead blocks come along for the barriers)
+        const float eff = d * (float)sc;
+        if (eff != 0.0f) {
+            float fitted = 0.0f;
+            refit16(eff, &fitted);
+            sg = fitted;
+        }
+        if (!dead) sc = (d == 0.0f) ? 0 : max(-127, min(127, q6k_round_dev(sg / d)));
+        __syncthreads();
+        sums[t] = double2{(double)sg, (double)sc};
+        __syncthreads();
+        double num = 0.0, den = 0.0;
+#pragma unroll
+        for (int k = 0; k < ng; ++k) {
+            const double2 v = sums[first + k];
+            num = __builtin_fma(v.x, v.y, num);
+            den = __builtin_fma(v.y, v.y, den);
+        }
+        float nd = (den > 1e-20) ? (float)(num / den) : 0.0f;
+        if (fabsf(nd) <= eps) nd = 0.0f;
+        if (!dead) d = nd;
+    }
+    uint32_t packed[3] = {0, 0, 0};
+    auto level_bits = [&](int i, uint32_t c) __attribute__((always_inline)) {
+        packed[i * 6 / 32] |= c << (i * 6 % 32);
+        if (i * 6 % 32 + 6 > 32) packed[i * 6 / 32 + 1] |= c >> (32 - i * 6 % 32);
+    };
+    const float eff = d * (float)sc;
+    if (eff != 0.0f) {
+        pass(eff, [&]() __attribute__((always_inline)) { packed[0] = packed[1] = packed[2] = 0; },
+             [&](int i, float n) __attribute__((always_inline)) { level_bits(i, (uint32_t)((int)n + 32)); });
+    } else {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) level_bits(i, 32u);
+    }
+    // a block is 210 bytes: its parts in the image are aligned to two bytes
+    uint8_t* bytes = reinterpret_cast<uint8_t*>(img) + (t / ng) * 210;
+#pragma unroll
+    for (int i = 0; i < 6; ++i) *reinterpret_cast<uint16_t*>(bytes + 12 * g + 2 * i) = (uint16_t)(packed[i >> 1] >> (16 * (i & 1)));
+    bytes[192 + g] = (uint8_t)(int8_t)sc;
+    if (g == 0) *reinterpret_cast<uint16_t*>(bytes + 208) = (uint16_t)float_to_half_bits(d);
+    __syncthreads();
+    const int64_t b0 = (int64_t)(blockIdx.x - with_short) * 4;
+    const int halves = (int)min((int64_t)4, nblocks - b0) * 105;
+    uint8_t* p = dst + b0 * 210;
+    for (int i = t; i < halves / 2; i += 64) __builtin_memcpy(p + 4 * i, &img[i], 4);
+    if ((halves & 1) && t == 0) __builtin_memcpy(p + 2 * halves - 2, reinterpret_cast<const uint8_t*>(img) + 2 * halves - 2, 2);
 }
 
 // _K_M / _K_H tiers (src/codec/block_codec.cpp:2378-2400, :2551-2665, :2733-2824): a candidate payload replaces
@@ -1443,11 +1515,6 @@ bool block_layout(int fmt, int n, BlockLayout* L) {
     }
 }
 
-int launch_encode_mix(const MixLayout& L, const float* w, uint8_t* dst, hipStream_t s) {
-    hipLaunchKernelGGL(encode_mix_kernel, dim3(1), dim3(64), 0, s, L, w, dst);
-    return hip_fail(hipGetLastError(), "encode launch");
-}
-
 int launch_decode_short(const BlockLayout& L, const uint8_t* src, float* out, hipStream_t s) {
     if (L.n <= 0 || L.n > 256 || L.bytes <= 0) return fail(TFQ_ERR_SHAPE, "decode: bad short-block layout");
     if (L.kind == BK_MIX) {
@@ -1560,7 +1627,7 @@ struct TierTry { int iters; float smult; };
 template <int FMT, class Launch>
 static int encode_tiers(const TierTry* tries, int count, const float* w, int64_t nblocks, uint8_t* dst, hipStream_t s,
                         Launch&& launch) {
-    if (count <= 0) return TFQ_OK;
+    if (count <= 0 || nblocks <= 0) return TFQ_OK;
     constexpr size_t BB = spec_of(FMT).block_bytes;
     uint8_t* cand = nullptr;
     TFQ_HIP(hipMalloc(&cand, (size_t)nblocks * BB));
@@ -1577,67 +1644,126 @@ static int encode_tiers(const TierTry* tries, int count, const float* w, int64_t
 // Lattice and fixed-codebook ids with their tiers: base (iters0, 1.0), _K_M one longer search, _K_H six
 // (src/codec/block_codec.cpp:2551-2665).
 template <int FMT>
-static int encode_lattice_family(int fmt, const float* w, int64_t nblocks, uint8_t* dst, hipStream_t s) {
+static int encode_lattice_family(int fmt, const float* w, int64_t nblocks, uint8_t* dst, const ShortJob& job, hipStream_t s) {
     constexpr bool FIXED = spec_of(FMT).codec == Codec::Fixed;
-    const dim3 grid((unsigned)nblocks);
-    auto launch = [&](uint8_t* out, int iters, float smult) {
-        hipLaunchKernelGGL(encode_lattice_kernel<FMT>, grid, dim3(64), 0, s, w, out, iters, smult);
+    const bool spread = nblocks < 8192;  // eight lanes per block are less than a wavefront per SIMD
+    auto launch = [&](uint8_t* out, int iters, float smult, const ShortJob& job) {
+        const unsigned grid = (unsigned)((spread ? (nblocks + 3) / 4 : (nblocks + 7) / 8) + (job.L.n > 0));
+        if (spread) hipLaunchKernelGGL((encode_lattice_kernel<FMT, 16>), dim3(grid), dim3(64), 0, s, w, out, iters, smult, nblocks, job);
+        else hipLaunchKernelGGL((encode_lattice_kernel<FMT, 8>), dim3(grid), dim3(64), 0, s, w, out, iters, smult, nblocks, job);
     };
-    launch(dst, FIXED ? 3 : 2, 1.0f);
+    launch(dst, FIXED ? 3 : 2, 1.0f, job);
     const int a = FIXED ? 10 : 6, b = FIXED ? 24 : 14;
     const TierTry tries[6] = {{a, 1.0f}, {b, 1.0f}, {b, 0.9f}, {b, 1.1f}, {b, 0.7f}, {b, 1.3f}};
     const int tier = tier_of(fmt);
-    return encode_tiers<FMT>(tries, tier >= 2 ? 6 : tier, w, nblocks, dst, s, launch);
+    return encode_tiers<FMT>(tries, tier >= 2 ? 6 : tier, w, nblocks, dst, s,
+                             [&](uint8_t* out, int iters, float smult) { launch(out, iters, smult, ShortJob{}); });
 }
 
-int launch_encode(int fmt, const float* w, int64_t nblocks, uint8_t* dst, hipStream_t s) {
-    if (nblocks <= 0) return TFQ_OK;
+// The job of a tensor's short last block (behind nblocks full ones); job->L.n = 0 where there is none.
+static int short_job(int fmt, const BlockLayout* L, const float* w, int64_t nblocks, uint8_t* dst, ShortJob* job) {
+    *job = ShortJob{};
+    if (!L || L->n <= 0) return TFQ_OK;
+    if (L->n >= 256 || L->bytes <= 0 || L->bytes > kMaxShortBytes) return fail(TFQ_ERR_SHAPE, "encode: bad short-block layout");
+    job->L = *L;
+    job->w = w + nblocks * 256;
+    job->dst = dst + nblocks * (int64_t)spec_of(fmt).block_bytes;
+    job->tier = tier_of(fmt);
+    if (L->kind == BK_Q1)
+        job->tier = fmt == TFQ_Q_1 ? -1 : (fmt == TFQ_Q_1_K_M || fmt == TFQ_Q_G_1_K_M) ? 1 : (fmt == TFQ_Q_1_K_H || fmt == TFQ_Q_G_1_K_H) ? 2 : 0;
+    if (L->kind == BK_Q6K) job->tier = fmt == TFQ_Q_G_6_K_M ? 1 : fmt == TFQ_Q_G_6_K_H ? 2 : 0;
+    // A short Q_G_8_K_M / _K_H block that still holds an affine header would take the searched affine encoder
+    // of :2775-2785; with their claim of 8.0 bits the header never fits, so this does not occur.
+    if (spec_of(fmt).codec == Codec::Grp8 && L->kind == BK_AFFINE && tier_of(fmt) > 0)
+        return fail(TFQ_ERR_FORMAT, "encode: a short block of this id in the affine layout has no device encoder");
+    return TFQ_OK;
+}
+
+// formats whose full-block encoder takes the short block along as a workgroup
+static bool short_rides_along(int fmt) {
+    switch (spec_of(fmt).codec) {
+        case Codec::Affine: case Codec::Lattice: case Codec::Fixed: case Codec::Grp8: case Codec::Q6K: case Codec::Sym32: return true;
+        default: return false;
+    }
+}
+
+static int launch_encode_short(int fmt, const ShortJob& job, hipStream_t s) {
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(1), dim3(64), 0, s, job); };
+    switch (canonical(fmt)) {
+        case TFQ_Q_32: launch(encode_short_kernel<TFQ_Q_32>); break;
+        case TFQ_Q_G_12: launch(encode_short_kernel<TFQ_Q_G_12>); break;
+        case TFQ_Q_G_2_K_L: launch(encode_short_kernel<TFQ_Q_G_2_K_L>); break;
+        case TFQ_Q_G_3_K_L: launch(encode_short_kernel<TFQ_Q_G_3_K_L>); break;
+        case TFQ_Q_G_4_K_L: launch(encode_short_kernel<TFQ_Q_G_4_K_L>); break;
+        case TFQ_Q_6_5: launch(encode_short_kernel<TFQ_Q_6_5>); break;
+        case TFQ_Q_24: launch(encode_short_kernel<TFQ_Q_24>); break;
+        case TFQ_Q_24_5: launch(encode_short_kernel<TFQ_Q_24_5>); break;
+        case TFQ_Q_G_24: launch(encode_short_kernel<TFQ_Q_G_24>); break;
+        case TFQ_Q_16: launch(encode_short_kernel<TFQ_Q_16>); break;
+        case TFQ_Q_16_5: launch(encode_short_kernel<TFQ_Q_16_5>); break;
+        case TFQ_Q_G_16: launch(encode_short_kernel<TFQ_Q_G_16>); break;
+        case TFQ_Q_1: launch(encode_short_kernel<TFQ_Q_1>); break;
+        default: return fail(TFQ_ERR_FORMAT, "encode: wire id " + std::to_string(fmt) + " has no device encoder in this build");
+    }
+    return hip_fail(hipGetLastError(), "encode launch");
+}
+
+int launch_encode(int fmt, const float* w, int64_t nblocks, uint8_t* dst, hipStream_t s, const BlockLayout* short_block) {
     if (nblocks > 0x7FFFFFFF) return fail(TFQ_ERR_SHAPE, "encode: more than 2^31-1 blocks in one call");
-    const dim3 grid((unsigned)nblocks), block(256);
+    ShortJob job;
+    if (int r = short_job(fmt, short_block, w, nblocks, dst, &job)) return r;
+    if (nblocks <= 0 && job.L.n <= 0) return TFQ_OK;
+    const dim3 grid((unsigned)nblocks), grid4((unsigned)((nblocks + 3) / 4)), block(256);
     if (is_mix(fmt)) {
-        hipLaunchKernelGGL(encode_mix_kernel, grid, dim3(64), 0, s, mix_layout(fmt, 256), w, dst);
+        if (nblocks > 0) hipLaunchKernelGGL(encode_mix_kernel, grid, dim3(64), 0, s, mix_layout(fmt, 256), w, dst);
+        if (job.L.n > 0) hipLaunchKernelGGL(encode_mix_kernel, dim3(1), dim3(64), 0, s, mix_layout(fmt, job.L.n), job.w, job.dst);
         return hip_fail(hipGetLastError(), "encode launch");
+    }
+    if (job.L.n > 0 && !short_rides_along(fmt)) {
+        if (nblocks > 0)
+            if (int r = launch_encode(fmt, w, nblocks, dst, s)) return r;
+        return launch_encode_short(fmt, job, s);
     }
     switch (canonical(fmt)) {
         case TFQ_Q_32: hipLaunchKernelGGL(encode_raw32_kernel, grid, block, 0, s, w, dst); break;
-        case TFQ_B32S4: hipLaunchKernelGGL(encode_sym32_kernel<TFQ_B32S4>, grid, block, 0, s, w, dst); break;
-        case TFQ_B32S8: hipLaunchKernelGGL(encode_sym32_kernel<TFQ_B32S8>, grid, block, 0, s, w, dst); break;
-        case TFQ_Q_G_4: hipLaunchKernelGGL(encode_affine_kernel<TFQ_Q_G_4>, grid, dim3(64), 0, s, w, dst); break;
-        case TFQ_Q_G_3: hipLaunchKernelGGL(encode_affine_kernel<TFQ_Q_G_3>, grid, dim3(64), 0, s, w, dst); break;
-        case TFQ_Q_G_2: hipLaunchKernelGGL(encode_affine_kernel<TFQ_Q_G_2>, grid, dim3(64), 0, s, w, dst); break;
-        case TFQ_SB256A3: hipLaunchKernelGGL(encode_affine_kernel<TFQ_SB256A3>, grid, dim3(64), 0, s, w, dst); break;
-        case TFQ_SB256A2: hipLaunchKernelGGL(encode_affine_kernel<TFQ_SB256A2>, grid, dim3(64), 0, s, w, dst); break;
-        case TFQ_Q_1_5: hipLaunchKernelGGL(encode_affine_kernel<TFQ_Q_1_5>, grid, dim3(64), 0, s, w, dst); break;
+        case TFQ_B32S4: launch_encode_sym32<TFQ_B32S4>(w, nblocks, dst, job.L.n, s); break;
+        case TFQ_B32S8: launch_encode_sym32<TFQ_B32S8>(w, nblocks, dst, job.L.n, s); break;
+        case TFQ_Q_G_4: launch_encode_affine<TFQ_Q_G_4>(w, nblocks, dst, job, s); break;
+        case TFQ_Q_G_3: launch_encode_affine<TFQ_Q_G_3>(w, nblocks, dst, job, s); break;
+        case TFQ_Q_G_2: launch_encode_affine<TFQ_Q_G_2>(w, nblocks, dst, job, s); break;
+        case TFQ_SB256A3: launch_encode_affine<TFQ_SB256A3>(w, nblocks, dst, job, s); break;
+        case TFQ_SB256A2: launch_encode_affine<TFQ_SB256A2>(w, nblocks, dst, job, s); break;
+        case TFQ_Q_1_5: launch_encode_affine<TFQ_Q_1_5>(w, nblocks, dst, job, s); break;
         case TFQ_Q_G_8:
             if (nblocks * 8 > 0x7FFFFFFF) return fail(TFQ_ERR_SHAPE, "encode: too many groups in one call");
-            hipLaunchKernelGGL(encode_comp8_kernel<TFQ_Q_G_8>, dim3((unsigned)(nblocks * 8)), dim3(64), 0, s, w, dst, 1.0f);
+            launch_encode_comp8<TFQ_Q_G_8>(w, nblocks, dst, 1.0f, job, s);
             if (const int tier = tier_of(fmt)) {
                 // :2756-2772: scaled copies of every group's fitted scale, the last two for _K_M, all six for _K_H
                 const TierTry tries[6] = {{0, 0.7f}, {0, 0.9f}, {0, 0.95f}, {0, 1.05f}, {0, 1.1f}, {0, 1.3f}};
                 const int count = tier >= 2 ? 6 : 2;
                 const int rc = encode_tiers<TFQ_Q_G_8>(tries + 6 - count, count, w, nblocks, dst, s, [&](uint8_t* out, int, float smult) {
-                    hipLaunchKernelGGL(encode_comp8_kernel<TFQ_Q_G_8>, dim3((unsigned)(nblocks * 8)), dim3(64), 0, s, w, out, smult);
+                    launch_encode_comp8<TFQ_Q_G_8>(w, nblocks, out, smult, ShortJob{}, s);
                 });
                 if (rc != TFQ_OK) return rc;
             }
             break;
         case TFQ_Q_8:
-            hipLaunchKernelGGL(encode_comp8_kernel<TFQ_Q_8>, grid, dim3(64), 0, s, w, dst, 1.0f);
+            launch_encode_comp8<TFQ_Q_8>(w, nblocks, dst, 1.0f, job, s);
             if (tier_of(fmt) >= 2) {
                 // :2627-2645: the tries with smult 1 repeat the base payload (the 8-bit fit takes no iteration
                 // count), so _K_M equals _K_L and _K_H has four scaled tries
                 const TierTry tries[4] = {{0, 0.9f}, {0, 1.1f}, {0, 0.7f}, {0, 1.3f}};
                 const int rc = encode_tiers<TFQ_Q_8>(tries, 4, w, nblocks, dst, s, [&](uint8_t* out, int, float smult) {
-                    hipLaunchKernelGGL(encode_comp8_kernel<TFQ_Q_8>, grid, dim3(64), 0, s, w, out, smult);
+                    launch_encode_comp8<TFQ_Q_8>(w, nblocks, out, smult, ShortJob{}, s);
                 });
                 if (rc != TFQ_OK) return rc;
             }
             break;
-        case TFQ_Q_4: { const int rc = encode_lattice_family<TFQ_Q_4>(fmt, w, nblocks, dst, s); if (rc != TFQ_OK) return rc; break; }
-        case TFQ_Q_2: { const int rc = encode_lattice_family<TFQ_Q_2>(fmt, w, nblocks, dst, s); if (rc != TFQ_OK) return rc; break; }
-        case TFQ_Q_3: { const int rc = encode_lattice_family<TFQ_Q_3>(fmt, w, nblocks, dst, s); if (rc != TFQ_OK) return rc; break; }
-        case TFQ_Q_6: { const int rc = encode_lattice_family<TFQ_Q_6>(fmt, w, nblocks, dst, s); if (rc != TFQ_OK) return rc; break; }
-        case TFQ_Q_12: { const int rc = encode_lattice_family<TFQ_Q_12>(fmt, w, nblocks, dst, s); if (rc != TFQ_OK) return rc; break; }
+        case TFQ_Q_4: { const int rc = encode_lattice_family<TFQ_Q_4>(fmt, w, nblocks, dst, job, s); if (rc != TFQ_OK) return rc; break; }
+        case TFQ_Q_2: { const int rc = encode_lattice_family<TFQ_Q_2>(fmt, w, nblocks, dst, job, s); if (rc != TFQ_OK) return rc; break; }
+        case TFQ_Q_3: { const int rc = encode_lattice_family<TFQ_Q_3>(fmt, w, nblocks, dst, job, s); if (rc != TFQ_OK) return rc; break; }
+        case TFQ_Q_6: { const int rc = encode_lattice_family<TFQ_Q_6>(fmt, w, nblocks, dst, job, s); if (rc != TFQ_OK) return rc; break; }
+        case TFQ_Q_12: { const int rc = encode_lattice_family<TFQ_Q_12>(fmt, w, nblocks, dst, job, s); if (rc != TFQ_OK) return rc; break; }
         case TFQ_Q_G_12: {
             auto launch = [&](uint8_t* out, int iters, float smult) {
                 hipLaunchKernelGGL(encode_grp12_kernel, grid, dim3(64), 0, s, w, out, iters, smult);
@@ -1657,14 +1783,14 @@ int launch_encode(int fmt, const float* w, int64_t nblocks, uint8_t* dst, hipStr
         case TFQ_Q_G_6:
             // the _K_M / _K_H tiers re-run the search with more effort and keep the better candidate by decoded
             // error (src/codec/block_codec.cpp:2733-2755); that selection is not on the device
-            hipLaunchKernelGGL(encode_q6k_kernel, grid, dim3(64), 0, s, w, dst, 4, 3, 3);
-            if (fmt == TFQ_Q_G_6_K_M || fmt == TFQ_Q_G_6_K_H) {
+            hipLaunchKernelGGL(encode_q6k_kernel, dim3(grid4.x + (job.L.n > 0)), dim3(64), 0, s, w, dst, 4, 3, 3, nblocks, job);
+            if (nblocks > 0 && (fmt == TFQ_Q_G_6_K_M || fmt == TFQ_Q_G_6_K_H)) {
                 // longer searches, each kept only where it decodes strictly better (src/codec/block_codec.cpp:2733-2755)
                 uint8_t* cand = nullptr;
                 TFQ_HIP(hipMalloc(&cand, (size_t)nblocks * 210));
                 const int effort[2][3] = {{8, 5, 6}, {14, 8, 10}};
                 for (int c = 0; c < (fmt == TFQ_Q_G_6_K_H ? 2 : 1); ++c) {
-                    hipLaunchKernelGGL(encode_q6k_kernel, grid, dim3(64), 0, s, w, cand, effort[c][0], effort[c][1], effort[c][2]);
+                    hipLaunchKernelGGL(encode_q6k_kernel, grid4, dim3(64), 0, s, w, cand, effort[c][0], effort[c][1], effort[c][2], nblocks, ShortJob{});
                     hipLaunchKernelGGL(keep_better_kernel<TFQ_Q_G_6>, grid, dim3(64), 0, s, w, dst, (const uint8_t*)cand);
                 }
                 const hipError_t e1 = hipStreamSynchronize(s);

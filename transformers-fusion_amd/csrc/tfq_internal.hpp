@@ -367,9 +367,8 @@ int launch_decode(int fmt, const uint8_t* src, int64_t nblocks, float* out, hipS
 int launch_decode_short(const BlockLayout& L, const uint8_t* src, float* out, hipStream_t s);
 int launch_tile16(int fmt, const uint8_t* wire, uint8_t* tiled, int64_t N, int64_t K, hipStream_t s);
 int launch_decode_tiled(int fmt, const uint8_t* tiled, int64_t N, int64_t K, float* out, hipStream_t s);
-int launch_encode(int fmt, const float* w, int64_t nblocks, uint8_t* dst, hipStream_t s);
-// one block of L.n < 256 weights (the last block of a tensor) in the layout L = block_layout(fmt, L.n)
-int launch_encode_short(int fmt, const BlockLayout& L, const float* w, uint8_t* dst, hipStream_t s);
+// nblocks full blocks, then (short_block given and not empty) the short last block of the tensor behind them
+int launch_encode(int fmt, const float* w, int64_t nblocks, uint8_t* dst, hipStream_t s, const BlockLayout* short_block = nullptr);
 // split_ws (optional, device memory, 256-byte aligned): where the 5..16-row kernel of a single matrix with K above
 // 4096 keeps the partial sums of its K parts (gemv_rows16_split_bytes says how many bytes); without it such a call
 // runs unsplit, every workgroup reading whole activation rows.  A handle owns no scratch memory, so calls on one
