@@ -91,3 +91,59 @@ def test_prefill_full_grid_is_repeatable(tfq, gpu, fmt):
     half = W.gemm(x[:M // 2], out_dtype=torch.float32)
     assert torch.equal(half, ref[:M // 2])
     W.close()
+
+
+EXACT_FMTS = [("Q_G_4", "f32"), ("Q_G_3", "f32"), ("B32S4", "f32"), ("B32S8", "f32"), ("Q_G_8", "f32"), ("Q_8", "f32"),
+              ("Q_G_2", "f32"), ("SB256A3", "f32"), ("SB256A2", "f32"), ("Q_4", "f32"), ("Q_G_6", "f32"), ("Q_4_K_H", "f32"),
+              ("Q_G_2", "bf16"), ("SB256A3", "bf16"), ("SB256A2", "bf16"), ("Q_4", "bf16"), ("Q_G_6", "bf16")]
+
+
+@pytest.mark.parametrize("fmt,dtype", EXACT_FMTS)
+@pytest.mark.parametrize("M,N,K", [(17, 1, 256), (64, 128, 512), (65, 129, 768), (129, 250, 4352), (300, 48, 1024)])
+def test_gemm_integer_operands(O, tfq, gpu, fmt, dtype, M, N, K):
+    """The tile kernel with integer operands against the float64 product with the decoded matrix, at the edges of its
+    tiles (64 / 128 rows of either side), of its K split and of the last block.  Derived bounds on the norm of the
+    error: fp32 activations of the Tiled16 formats keep 16 bits (a part left out is below 2^-18 of a value, 4e-6),
+    everything else is fp32 sums (1e-6); the companded grid is a line within 7.5e-5 of its levels."""
+    import torch
+    print(f"gemm {fmt} {dtype} M={M} N={N} K={K}", flush=True)
+    w = O.rng_normal(42, N * K, 0.02)
+    pay = O.encode_tensor(fmt, w)
+    W = tfq.Weight(fmt, N, K, pay)
+    x = torch.from_numpy(O.rng_normal(43, M * K, 1.0).reshape(M, K)).to(gpu)
+    x = x.bfloat16() if dtype == "bf16" else x
+    dense = torch.from_numpy(O.decode_tensor(fmt, pay, N * K).reshape(N, K)).to(gpu).double()
+    want = x.double() @ dense.T
+    bound = 1.5e-4 if fmt in ("Q_G_8", "Q_8") else 1e-6 if dtype == "bf16" or fmt in ("Q_4", "Q_G_6", "Q_4_K_H") else 1e-5
+    for ws in (True, False):
+        y = W.gemm(x, workspace=ws)
+        assert float((y.double() - want).norm() / want.norm()) <= bound
+    # a row does not depend on the other rows of its tile
+    x2 = x.clone()
+    x2[1:] = 0
+    assert torch.equal(W.gemm(x2, workspace=False)[0], W.gemm(x, workspace=False)[0])
+    yb = W.gemm(x, out_dtype=torch.bfloat16)
+    assert torch.equal(yb, W.gemm(x).bfloat16())
+    W.close()
+
+
+@pytest.mark.parametrize("fmt", ["Q_4", "Q_G_6"])
+def test_gemm_integer_operands_non_finite(O, tfq, gpu, fmt):
+    """Infinite, not-a-number and huge activations give what the fp32 products of the 16-row path give."""
+    import torch
+    M, N, K = 20, 40, 512
+    W = tfq.Weight(fmt, N, K, O.encode_tensor(fmt, O.rng_normal(42, N * K, 0.02)))
+    x = torch.from_numpy(O.rng_normal(43, M * K, 1.0).reshape(M, K)).to(gpu)
+    x[2, 7] = float("inf")
+    x[3, 300] = -float("inf")
+    x[4, 100] = float("nan")
+    x[5] = 0
+    x[5, 9] = 2.0 ** 120  # times an unscaled integer this overflows, times the weight it does not
+    for xt in (x, x.bfloat16()):
+        y = W.gemm(xt)
+        ref = torch.cat([W.gemv(xt[:16].contiguous()), W.gemv(xt[16:].contiguous())])
+        assert torch.equal(torch.isnan(y), torch.isnan(ref)) and torch.equal(torch.isinf(y), torch.isinf(ref))
+        assert torch.equal(y[torch.isinf(y)], ref[torch.isinf(ref)])
+        f = torch.isfinite(ref)
+        assert torch.allclose(y[f], ref[f], rtol=1e-4, atol=1e-5)
+    W.close()
