@@ -712,3 +712,35 @@ def test_paired_gate_up_with_swiglu_epilogue(O, tfq, gpu, fmt, xdt, B, norm, ydt
     ref = O.silu_mul(O.matmul(fmt, pg, F, D, xin).reshape(-1), O.matmul(fmt, pu, F, D, xin).reshape(-1)).reshape(B, F)
     tol = 1e-2 if (xdt == "bf16" or ydt == "bf16") else 1e-3
     assert np.abs(h.float().cpu().numpy() - ref).max() / np.abs(ref).max() <= tol
+
+
+@pytest.mark.parametrize("fmt", ["Q_4", "Q_G_6", "Q_4_K_M"])
+@pytest.mark.parametrize("N,K", [(1, 256), (3, 768), (9, 4096), (33, 4352), (130, 8192)])
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+def test_gemv_sixteen_weight_runs(O, tfq, gpu, fmt, N, K, dtype):
+    """Q_4 and Q_G_6 at one to seven rows against the float64 product with the decoded matrix: row groups of four and
+    passes of sixteen blocks that are not full, infinite and huge activations (the kernel multiplies unscaled codes).
+    Bound: fp32 sums of exact products, 16 in a chain, then one per 16 blocks: 1e-6 of the norm."""
+    import torch
+    pay = O.encode_tensor(fmt, O.rng_normal(42, N * K, 0.02))
+    W = tfq.Weight(fmt, N, K, pay)
+    dense = torch.from_numpy(O.decode_tensor(fmt, pay, N * K).reshape(N, K)).to(gpu).double()
+    for B in (1, 2, 3, 4, 7):
+        print(f"gemv {fmt} {dtype} B={B} N={N} K={K}", flush=True)
+        x = torch.from_numpy(O.rng_normal(43 + B, B * K, 1.0).reshape(B, K)).to(gpu)
+        x = x.bfloat16() if dtype == "bf16" else x
+        y, want = W.gemv(x).double(), x.double() @ dense.T
+        # (a single output may be small beside its terms: the terms' norm bounds it then)
+        terms = (x.double().abs() @ dense.abs().T).norm()
+        assert float((y - want).norm()) <= max(1e-6 * float(want.norm()), 1.2e-7 * float(terms))
+    x = torch.zeros(4, K, device=gpu)
+    x[0] = 1.0
+    x[0, 5] = float("inf")
+    x[1, K - 1] = float("nan")
+    x[2, K // 2] = 3.0e38
+    x = x.bfloat16() if dtype == "bf16" else x
+    y, want = W.gemv(x), (x.double().unsqueeze(1) * dense.unsqueeze(0)).sum(-1).float()
+    assert torch.equal(torch.isnan(y), torch.isnan(want)) and torch.equal(torch.isinf(y), torch.isinf(want))
+    assert torch.equal(y[torch.isinf(y)], want[torch.isinf(want)])
+    assert torch.allclose(y[2:], want[2:], rtol=1e-5, atol=0, equal_nan=True)
+    W.close()

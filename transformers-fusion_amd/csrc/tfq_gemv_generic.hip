@@ -87,15 +87,212 @@ __global__ __launch_bounds__(256) void gemv_generic_kernel(const uint8_t* __rest
     }
 }
 
+// one row times one activation row, weight by weight (the arithmetic of gemv_generic_kernel); the total in lane 63
+template <int FMT, bool XF32>
+__device__ __attribute__((noinline)) float row_sum_lane63(const uint8_t* W, const void* xin, int row, int b, int N, int K, int lane) {
+    constexpr int BB = spec_of(FMT).block_bytes;
+    const int nblk = K >> 8;
+    const uint8_t* limit = W + (size_t)N * (size_t)nblk * BB;
+    float acc = 0.0f;
+    for (int blk = 0; blk < nblk; ++blk) {
+        float w[4];
+        decode_quad<FMT>(W + ((size_t)row * nblk + blk) * BB, (uint32_t)lane, w, limit);
+        const size_t k0 = (size_t)b * K + (size_t)blk * 256 + 4 * lane;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const float xv = XF32 ? static_cast<const float*>(xin)[k0 + t] : __uint_as_float((uint32_t)static_cast<const unsigned short*>(xin)[k0 + t] << 16);
+            acc = __builtin_fmaf(w[t], xv, acc);
+        }
+    }
+    return wave_sum_lane63(acc);
+}
+
+// ---- Q_4 and Q_G_6: four rows per workgroup, sixteen weights per lane
+// Bound by vector issue before the bytes: the wavefront-per-row kernel above spends 12 to 20 instructions per weight
+// on these formats (unpacking one code at a time, the scale per weight, a wavefront-wide sum per row).  Here a lane
+// takes a run of sixteen weights (one scale group of Q_G_6: 96 bits; 63 bits of Q_4), multiplies them unscaled and
+// scales the sum of sixteen; a code becomes a number by one field extract and one conversion (Q_G_6), or two at a
+// time by an 8-byte look-up in LDS (Q_4).  Sixteen lanes cover a block, a wavefront four blocks, the workgroup's four
+// wavefronts sixteen (K = 4096 in one pass, where a lane's activations then stay in registers); four weight rows
+// share every unpacked activation.  The codes of the next rows are fetched before the present ones are multiplied.
+template <int FMT>
+constexpr bool kRun16 = FMT == TFQ_Q_4 || FMT == TFQ_Q_G_6;
+constexpr int kRunRows = 4;
+
+struct Run16 {
+    uint32_t v[3];
+    uint32_t sc;  // Q_G_6: the group's scale byte
+    uint32_t d;   // binary16
+};
+
+template <int FMT, int BT, bool XF32, bool ONE_PASS>
+__global__ __launch_bounds__(256) void gemv_run16_kernel(const uint8_t* __restrict__ W, const void* __restrict__ xin,
+                                                         void* __restrict__ yout, int N, int K, int y_bf16) {
+    constexpr int BB = spec_of(FMT).block_bytes, R = kRunRows;
+    __shared__ float part[2][4][R * BT];
+    __shared__ float2 pair_levels[FMT == TFQ_Q_4 ? 256 : 1];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if constexpr (FMT == TFQ_Q_4) {
+        pair_levels[tid] = float2{kGrid4[tid & 15], kGrid4[tid >> 4]};
+        __syncthreads();
+    }
+    const int nblk = K >> 8, groups = (N + R - 1) / R, passes = (nblk + 15) >> 4;
+    const int c = lane & 15, sub = wave * 4 + (lane >> 4);  // run of a block, block of a pass
+    // where the lane's codes start in its block
+    constexpr int kBits4 = 63;
+    const int bit = FMT == TFQ_Q_4 ? 16 + kBits4 * c : 0;
+    const int at = FMT == TFQ_Q_4 ? 4 * min(bit >> 5, 29) : 12 * c;  // (the last run ends with the block's dword 31)
+    const uint32_t shift = bit & 31;
+
+    auto fetch = [&](int g, int pass, Run16 (&r)[R]) __attribute__((always_inline)) {
+        const int blk = min(pass * 16 + sub, nblk - 1);
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            const uint8_t* p = W + ((size_t)min(g * R + i, N - 1) * nblk + blk) * BB;
+            if constexpr (FMT == TFQ_Q_4) {
+                const uint32_t* q = reinterpret_cast<const uint32_t*>(p + at);
+                r[i].v[0] = q[0]; r[i].v[1] = q[1]; r[i].v[2] = q[2];
+                r[i].d = half_at(p);
+            } else {
+                __builtin_memcpy(r[i].v, __builtin_assume_aligned(p + at, 2), 12);
+                r[i].sc = p[192 + c];
+                r[i].d = half_at(p + 208);
+            }
+        }
+    };
+    float x[BT][16];
+    auto fetch_x = [&](int pass) __attribute__((always_inline)) {
+        const size_t k0 = (size_t)min(pass * 16 + sub, nblk - 1) * 256 + 16 * c;
+#pragma unroll
+        for (int b = 0; b < BT; ++b) {
+            if constexpr (XF32) {
+                const float4* q = reinterpret_cast<const float4*>(static_cast<const float*>(xin) + (size_t)b * K + k0);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const float4 v = q[t];
+                    x[b][4 * t] = v.x; x[b][4 * t + 1] = v.y; x[b][4 * t + 2] = v.z; x[b][4 * t + 3] = v.w;
+                }
+            } else {
+                const uint4* q = reinterpret_cast<const uint4*>(static_cast<const unsigned short*>(xin) + (size_t)b * K + k0);
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const uint4 v = q[t];
+                    const uint32_t u[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        x[b][8 * t + 2 * e] = __uint_as_float(u[e] << 16);
+                        x[b][8 * t + 2 * e + 1] = __uint_as_float(u[e] & 0xFFFF0000u);
+                    }
+                }
+            }
+        }
+    };
+
+    Run16 cur[R], nxt[R];
+    int g = blockIdx.x, parity = 0;
+    fetch(g, 0, nxt);
+    if constexpr (ONE_PASS) fetch_x(0);
+    for (; g < groups; g += gridDim.x) {  // the same trips for the whole workgroup
+        float acc[R][BT];
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+#pragma unroll
+            for (int b = 0; b < BT; ++b) acc[i][b] = 0.0f;
+        for (int pass = 0; pass < (ONE_PASS ? 1 : passes); ++pass) {
+#pragma unroll
+            for (int i = 0; i < R; ++i) cur[i] = nxt[i];
+            const bool last = ONE_PASS || pass == passes - 1;
+            fetch(last ? (g + (int)gridDim.x < groups ? g + (int)gridDim.x : g) : g, last ? 0 : pass + 1, nxt);
+            if constexpr (!ONE_PASS) fetch_x(pass);
+            const bool live = pass * 16 + sub < nblk;
+#pragma unroll
+            for (int i = 0; i < R; ++i) {
+                float w[16], scale;
+                if constexpr (FMT == TFQ_Q_4) {
+                    uint32_t v0 = cur[i].v[0], v1 = cur[i].v[1], v2 = cur[i].v[2];
+                    if (c == 15) { v0 = v1; v1 = v2; v2 = 0; }
+                    const uint32_t lo = __builtin_amdgcn_alignbit(v1, v0, shift);
+                    uint32_t hi = __builtin_amdgcn_alignbit(v2, v1, shift);
+                    hi = (hi & 0x0FFFFFFFu) | ((hi << 1) & 0xE0000000u);  // the sixteenth code has three bits, an even level
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) {
+                        const float2 a = pair_levels[(lo >> (8 * t)) & 255u], b = pair_levels[(hi >> (8 * t)) & 255u];
+                        w[2 * t] = a.x; w[2 * t + 1] = a.y;
+                        w[8 + 2 * t] = b.x; w[8 + 2 * t + 1] = b.y;
+                    }
+                    scale = half_bits_to_float(cur[i].d);
+                } else {
+                    // codes are stored + 32: with the top bit of each turned they are two's complement
+                    const uint32_t v0 = cur[i].v[0] ^ 0x20820820u, v1 = cur[i].v[1] ^ 0x08208208u, v2 = cur[i].v[2] ^ 0x82082082u;
+                    const uint32_t s5 = __builtin_amdgcn_alignbit(v1, v0, 30), s10 = __builtin_amdgcn_alignbit(v2, v1, 28);
+#pragma unroll
+                    for (int t = 0; t < 16; ++t) {
+                        const uint32_t src = t == 5 ? s5 : t == 10 ? s10 : t < 5 ? v0 : t < 10 ? v1 : v2;
+                        const int pos = t == 5 || t == 10 ? 0 : 6 * t - (t < 5 ? 0 : t < 10 ? 32 : 64);
+                        w[t] = (float)((int32_t)(src << (26 - pos)) >> 26);
+                    }
+                    scale = half_bits_to_float(cur[i].d) * (float)(int)(int8_t)cur[i].sc;
+                }
+#pragma unroll
+                for (int b = 0; b < BT; ++b) {
+                    float s = w[0] * x[b][0];
+#pragma unroll
+                    for (int t = 1; t < 16; ++t) s = __builtin_fmaf(w[t], x[b][t], s);
+                    const float a = __builtin_fmaf(scale, s, acc[i][b]);
+                    acc[i][b] = live ? a : acc[i][b];
+                }
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+#pragma unroll
+            for (int b = 0; b < BT; ++b) {
+                const float s = wave_sum_lane63(acc[i][b]);
+                if (lane == 63) part[parity][wave][i * BT + b] = s;
+            }
+        __syncthreads();  // (the next group's sums go to the other half)
+        if (wave == 0) {
+            const int o = lane < R * BT ? lane : 0, row = g * R + o / BT, b = o % BT;
+            const bool mine = lane < R * BT && row < N;
+            float v = (part[parity][0][o] + part[parity][1][o]) + (part[parity][2][o] + part[parity][3][o]);
+            // Where the unscaled sums left the range of fp32, the row is multiplied again weight by weight
+            uint64_t redo = __ballot(mine && (__float_as_uint(v) & 0x7F800000u) == 0x7F800000u);
+            while (redo) {
+                const int src = __builtin_ctzll(redo);
+                redo &= redo - 1;
+                const float again = row_sum_lane63<FMT, XF32>(W, xin, g * R + src / BT, src % BT, N, K, lane);
+                const float all = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(again), 63));
+                if (lane == src) v = all;
+            }
+            if (mine) {
+                if (y_bf16) reinterpret_cast<unsigned short*>(yout)[(size_t)b * N + row] = (unsigned short)bf16_rne(v);
+                else reinterpret_cast<float*>(yout)[(size_t)b * N + row] = v;
+            }
+        }
+        parity ^= 1;
+    }
+}
+
 template <int FMT, int BT>
 int run(const tfq_weight* w, const void* x, int xd, void* y, int yd, hipStream_t s) {
     const int N = (int)w->N, K = (int)w->K;
+    if constexpr (kRun16<FMT>) {
+        // about a thousand workgroups (four per compute unit), each with the same number of row groups
+        const int groups = (N + kRunRows - 1) / kRunRows, per = (groups + 1023) / 1024, grid = (groups + per - 1) / per;
+        const bool one_pass = K <= 4096;
+        using Kernel = void (*)(const uint8_t*, const void*, void*, int, int, int);
+        const Kernel kern = xd == TFQ_F32 ? (one_pass ? gemv_run16_kernel<FMT, BT, true, true> : gemv_run16_kernel<FMT, BT, true, false>)
+                                          : (one_pass ? gemv_run16_kernel<FMT, BT, false, true> : gemv_run16_kernel<FMT, BT, false, false>);
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, s, w->dev, x, y, N, K, yd == TFQ_BF16);
+        return hip_fail(hipGetLastError(), "gemv launch");
+    } else {
     const int grid = (N + 3) / 4 < 4096 ? (N + 3) / 4 : 4096;
     if (xd == TFQ_F32)
         hipLaunchKernelGGL((gemv_generic_kernel<FMT, BT, true>), dim3(grid), dim3(256), 0, s, w->dev, x, y, N, K, yd == TFQ_BF16);
     else
         hipLaunchKernelGGL((gemv_generic_kernel<FMT, BT, false>), dim3(grid), dim3(256), 0, s, w->dev, x, y, N, K, yd == TFQ_BF16);
     return hip_fail(hipGetLastError(), "gemv launch");
+    }
 }
 
 template <int FMT>
