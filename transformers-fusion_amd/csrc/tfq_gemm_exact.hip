@@ -21,10 +21,15 @@
 //
 // A workgroup of four wavefronts owns 128 tokens x 128 weight rows and walks K in steps of 32, both operands staged
 // in LDS (two buffers, one barrier per step); a wavefront multiplies 64 x 64.  What bounds it is vector issue next
-// to the MFMAs (splitting activations, decoding codes, the scale's multiply-adds: 1.2-1.4 vector cycles per MFMA
-// cycle), so two workgroups share a compute unit (LDS <= 80 KB, <= 256 registers): one's staging runs under the
-// other's MFMAs.  256-row tiles with one workgroup per unit would stage less per product, but a ragged prompt (333
-// rows) then pads to 512 rows instead of 384.
+// to the MFMAs (splitting activations, decoding codes, the scale's multiply-adds; counted on 333 fp32 rows of Q_G_4
+// 4096 x 14336: 260 vector instructions and 38 MFMAs per wavefront and step, vector issue busy for 66 % of the cycles,
+// the matrix cores for 34 %, LDS for 44 %), so two workgroups share a compute unit (LDS <= 80 KB, <= 256 registers):
+// one's staging runs under the other's MFMAs.  256-row tiles with one workgroup per unit would stage less per product,
+// but a ragged prompt (333 rows) then pads to 512 rows instead of 384.  Activations are fetched two steps ahead, codes
+// three.  Few rows take 64-row tiles, three workgroups per unit.
+// Measured, before (slices of 4 to 16 rows through the decode kernels) and now: Q_G_4 fp32 333 rows 4096 x 14336
+// 657 -> 171 us, B32S8 the same 700 -> 133 us; 512 bf16 rows of 14336 x 4096: Q_4 7580 -> 155 us, Q_G_6 5360 -> 164 us,
+// SB256A3 789 -> 135 us.  Below 17 rows the decode kernels stay.
 
 #include <algorithm>
 #include <atomic>
@@ -155,7 +160,7 @@ constexpr int lds_uint4s() {
 }
 
 template <int FMT, int XP, int TM>
-__global__ __launch_bounds__(THREADS, XP == 3 && TM == 128 ? 1 : TM == 128 || XP == 3 ? 2 : 3) void gemm_exact_kernel(ExactArgs args) {
+__global__ __launch_bounds__(THREADS, TM == 128 || XP == 3 ? 2 : 3) void gemm_exact_kernel(ExactArgs args) {
     using F = Form<FMT>;
     constexpr int WP = F::WP, OG = F::OG, UB = F::WIRE ? spec_of(FMT).block_bytes : tiled_unit_bytes(FMT);
     constexpr int MI = TM / 32, NJ = 4, XPL = TM * 4;  // XPL: 16-byte pieces of an activation part in LDS
@@ -191,8 +196,8 @@ __global__ __launch_bounds__(THREADS, XP == 3 && TM == 128 ? 1 : TM == 128 || XP
     const uint8_t* const wbase = args.W + (size_t)(F::WIRE ? n0 : n0 >> 4) * nblocks * UB;
     const uint32_t woffs = (uint32_t)wtile * (uint32_t)nblocks * UB;  // below 4 GiB: K is at most 2^22
     const int r16 = (n0 + row) & 15;
-    // staging of the activations: 16-byte pieces, adjacent threads take adjacent pieces of a row (a piece of another row
-    // per thread kept the address unit busy four times as long: 183 us against 118 us, Q_G_4 4096 x 14336 x 333 rows).
+    // staging of the activations: 16-byte pieces, adjacent threads take adjacent pieces of a row (64 bytes of
+    // a row per thread, every lane on a line of its own: B32S8 fp32 333 x 4096 x 14336 144 us against 133 us).
     // LDS slot of (row, piece of eight values): row * 4 + (piece ^ row / 2 % 4), free of bank conflicts both ways.
     constexpr int XE = XP == 1 ? 2 : 4, TPR = XP == 1 ? 4 : 8, RPP = THREADS / TPR, XC = TM / RPP;
     const int xrow0 = tid / TPR, xpiece = tid % TPR;
@@ -326,9 +331,7 @@ __global__ __launch_bounds__(THREADS, XP == 3 && TM == 128 ? 1 : TM == 128 || XP
                 wd[512 + 8 * h] = uint4{el[0], el[1], ol[0], ol[1]};
             }
             // the scale takes 10^-4 in one rounding
-            if constexpr (U == 0) {
-                if (half == 0) wscale[par * 128 + row] = (float)((double)half_bits_to_float(hdd) * 1e-4);
-            }
+            if constexpr (U == 0) wscale[par * 128 + row] = (float)((double)half_bits_to_float(hdd) * 1e-4);
         } else if constexpr (FMT == TFQ_Q_G_6) {
             const uint32_t scw = U < 4 ? hdr.x : hdr.y;
             const float sc = (float)((int32_t)(scw << (24 - 8 * (U & 3))) >> 24), c = -32.0f * sc;
@@ -350,9 +353,7 @@ __global__ __launch_bounds__(THREADS, XP == 3 && TM == 128 ? 1 : TM == 128 || XP
             wd[8] = uint4{hi[4], hi[5], hi[6], hi[7]};
             wd[512] = uint4{lo[0], lo[1], lo[2], lo[3]};
             wd[520] = uint4{lo[4], lo[5], lo[6], lo[7]};
-            if constexpr (U == 0) {
-                if (half == 0) wscale[par * 128 + row] = half_bits_to_float(hdd);
-            }
+            if constexpr (U == 0) wscale[par * 128 + row] = half_bits_to_float(hdd);
         } else if constexpr (F::BYTES) {
             const uint32_t scw = (U >> 1) == 0 ? hdr.x : (U >> 1) == 1 ? hdr.y : (U >> 1) == 2 ? hdr.z : hdr.w;
             const float sc = (float)((scw >> (16 * (U & 1) + 8 * half)) & 255u);
@@ -378,10 +379,8 @@ __global__ __launch_bounds__(THREADS, XP == 3 && TM == 128 ? 1 : TM == 128 || XP
                 };
                 mcs[par * 256 + half * 128 + row] = ints(half ? hmc.z : hmc.x, half ? hmc.w : hmc.y, bias, -1.0f);
                 if constexpr (F::SC_OFFSET) scs[par * 256 + half * 128 + row] = ints(half ? hdr.z : hdr.x, half ? hdr.w : hdr.y, 0.0f, 4.0f);
-                if (half == 0) {
-                    wscale[par * 128 + row] = half_fast(hdd & 0xFFFFu) * (sp.bits == 3 ? 1.0f / 7.0f : 1.0f / 3.0f);
-                    woff[par * 128 + row] = half_fast(hdd >> 16);
-                }
+                wscale[par * 128 + row] = half_fast(hdd & 0xFFFFu) * (sp.bits == 3 ? 1.0f / 7.0f : 1.0f / 3.0f);
+                woff[par * 128 + row] = half_fast(hdd >> 16);
             }
         } else {
             float a, c;
@@ -396,7 +395,9 @@ __global__ __launch_bounds__(THREADS, XP == 3 && TM == 128 ? 1 : TM == 128 || XP
                 wd[8] = decode8x2(r[1], r[3], s, c0);
                 if constexpr (FMT != TFQ_B32S8) a *= 0.5f;
             }
-            if (half == 0) wscale[(U & 1) * 128 + row] = a;
+            // (the halves hold the same value; without the offsets' longer step one write of it is the faster form:
+            // B32S8 133 against 137 us, Q_G_4 172 against 171 us, fp32 333 x 4096 x 14336)
+            if (OG > 0 || half == 0) wscale[(U & 1) * 128 + row] = a;
             if constexpr (U == 0 && OG == 8) {
                 // the 6-bit offset codes of the eight groups, 32 - code
                 const uint64_t mw = (uint64_t)(hdr.y >> 16) | ((uint64_t)hdr.z << 16);
@@ -404,10 +405,8 @@ __global__ __launch_bounds__(THREADS, XP == 3 && TM == 128 ? 1 : TM == 128 || XP
 #pragma unroll
                 for (int t = 0; t < 4; ++t)
                     o[t] = pk(32.0f - (float)(uint32_t)((mw >> (12 * t)) & 63u), 32.0f - (float)(uint32_t)((mw >> (12 * t + 6)) & 63u));
-                if (half == 0) {
-                    mcs[par * 128 + row] = uint4{o[0], o[1], o[2], o[3]};
-                    woff[par * 128 + row] = half_fast(hdr.w >> 16);
-                }
+                mcs[par * 128 + row] = uint4{o[0], o[1], o[2], o[3]};
+                woff[par * 128 + row] = half_fast(hdr.w >> 16);
             }
         }
     };
@@ -490,16 +489,15 @@ __global__ __launch_bounds__(THREADS, XP == 3 && TM == 128 ? 1 : TM == 128 || XP
                 f32x4_t v4 = zero4;
 #pragma unroll
                 for (int p = XP - 1; p >= 0; --p) v4 = mm(xb[p * XPL + i * 64], ones, v4);
-                const int e = OG == 16 ? fr >> 1 : fr;
-                const float v = e == 0 ? v4[0] : e == 1 ? v4[1] : e == 2 ? v4[2] : v4[3];
+                // (lanes beyond the four rows write what those write: no branch in the middle of the step)
+                const int e = (OG == 16 ? fr >> 1 : fr) & 3;
+                const float v01 = e & 1 ? v4[1] : v4[0], v23 = e & 1 ? v4[3] : v4[2], v = e & 2 ? v23 : v01;
                 const uint32_t p0 = pk(v, 0.0f), p1 = pk(v - bf_lo(p0), 0.0f), p2 = pk(v - bf_lo(p0) - bf_lo(p1), 0.0f);
-                if (e < 4) {
-                    const int r = wm * (TM / 2) + i * 16 + 4 * fk + e;
-                    unsigned short* const sd = reinterpret_cast<unsigned short*>(sums) + (OG == 16 ? r * 48 + 2 * U + (fr & 1) : r * 24 + U);
-                    sd[0] = (unsigned short)p0;
-                    sd[OG] = (unsigned short)p1;
-                    sd[2 * OG] = (unsigned short)p2;
-                }
+                const int r = wm * (TM / 2) + i * 16 + 4 * fk + e;
+                unsigned short* const sd = reinterpret_cast<unsigned short*>(sums) + (OG == 16 ? r * 48 + 2 * U + (fr & 1) : r * 24 + U);
+                sd[0] = (unsigned short)p0;
+                sd[OG] = (unsigned short)p1;
+                sd[2 * OG] = (unsigned short)p2;
             }
         }
         if constexpr (U == 7) {
@@ -620,28 +618,30 @@ __global__ __launch_bounds__(256) void reduce_exact_kernel(ExactArgs args) {
     else reinterpret_cast<float*>(args.Y)[i] = v;
 }
 
-// Tile height, K split and time (us) of M rows by a model of measurements: two workgroups of 128 rows or three of 64
-// run on a compute unit at once; a step takes `full` us with the units full and `alone` us with one workgroup on each;
-// the partials' traffic at 5 TB/s.
+// Tile height, K split and time (us) of M rows by a model of measurements (14336 x 4096): two workgroups of 128 rows
+// or three of 64 run on a compute unit at once; a step takes t[n - 1] us with n workgroups on every unit.  Rows are the
+// operand products per weight: one (bf16 activations, 16-weight groups), two (fp32 activations, or bf16 ones on the
+// wire formats) or six (fp32 on the wire formats, whose 128-row tile fits a unit only once and lost: 1.7 us against
+// 1.44 us for two of 64).  The partials' traffic at 5 TB/s.
 struct ExactPlan {
     int tm, ksplit;
     double us;
 };
 ExactPlan plan_exact(int64_t N, int64_t K, int M, int planes, size_t scratch_bytes) {
-    const int nblocks = (int)(K >> 8);
-    ExactPlan best{128, 1, 1e30};
-    for (int tm = 64; tm <= 128; tm *= 2) {
+    static constexpr double kStep64[3][3] = {{0.50, 0.78, 1.05}, {0.56, 0.93, 1.30}, {0.84, 1.44, 0.0}}, kStep128[2][2] = {{0.75, 1.00}, {0.85, 1.30}};
+    const int nblocks = (int)(K >> 8), kind = planes == 1 ? 0 : planes == 2 ? 1 : 2;
+    ExactPlan best{64, 1, 1e30};
+    for (int tm = 64; tm <= (kind == 2 ? 64 : 128); tm *= 2) {
         const long tiles = (long)((M + tm - 1) / tm) * (long)((N + TN - 1) / TN);
-        const int per_cu = planes == 6 ? (tm == 64 ? 2 : 1) : tm == 64 ? 3 : 2;
-        const double alone = tm == 64 ? 0.22 + 0.06 * planes : 0.25 + 0.12 * planes;
-        const double full = per_cu == 1 ? alone : (tm == 64 ? 0.36 + 0.14 * planes : 0.30 + 0.22 * planes);
+        const int per_cu = tm == 128 || kind == 2 ? 2 : 3;
+        const double* t = tm == 64 ? kStep64[kind] : kStep128[kind];
         const long slots = 256L * per_cu;
         for (int S = 1; S <= 16 && S <= nblocks; ++S) {
             const double part_bytes = (double)S * (double)M * (double)N * 4.0;
             if (S > 1 && (tiles * S > 2 * slots || part_bytes > (double)scratch_bytes)) continue;
             const long wgs = tiles * S, rest = wgs % slots;
             const double steps = 8.0 * (double)((nblocks + S - 1) / S);
-            double us = 4.0 + steps * ((double)(wgs / slots) * full + (rest > 256 ? full : rest ? alone : 0.0));
+            double us = 4.0 + steps * ((double)(wgs / slots) * t[per_cu - 1] + (rest ? t[(rest + 255) / 256 - 1] : 0.0));
             if (S > 1) us += 3.0 + part_bytes * (1.0 + 1.0 / S) / 5e6;
             if (us < best.us) best = {tm, S, us};
         }
@@ -670,7 +670,8 @@ int run_exact_tm(ExactArgs a, hipStream_t s) {
 
 template <int FMT, int XP>
 int run_exact(const ExactArgs& a, int tm, hipStream_t s) {
-    return tm == 64 ? run_exact_tm<FMT, XP, 64>(a, s) : run_exact_tm<FMT, XP, 128>(a, s);
+    if constexpr (XP == 3) return run_exact_tm<FMT, XP, 64>(a, s);
+    else return tm == 64 ? run_exact_tm<FMT, XP, 64>(a, s) : run_exact_tm<FMT, XP, 128>(a, s);
 }
 
 int planes_of(const tfq_weight* w, int x_dtype) {
@@ -686,10 +687,6 @@ bool gemm_exact_serves(const tfq_weight* w, int x_dtype, int M) {
     const int f = canonical(w->fmt);
     if (w->layout == TFQ_LAYOUT_WIRE) return f == TFQ_Q_4 || f == TFQ_Q_G_6;
     return w->layout == TFQ_LAYOUT_TILED16 && (x_dtype == TFQ_F32 || tiled_header_bytes(w->fmt) == 48);
-}
-
-double gemm_exact_us(const tfq_weight* w, int x_dtype, int M, size_t scratch_bytes) {
-    return plan_exact(w->N, w->K, M, planes_of(w, x_dtype), scratch_bytes).us;
 }
 
 size_t gemm_exact_scratch_bytes(const tfq_weight* w, int x_dtype, int M) {

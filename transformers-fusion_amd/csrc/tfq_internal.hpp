@@ -490,9 +490,8 @@ int launch_gemm(const tfq_weight* w, const void* x, int x_dtype, int M, void* y,
                 hipStream_t s, void* scratch = nullptr, size_t scratch_bytes = 0);
 size_t gemm_scratch_bytes(const tfq_weight* w, int x_dtype, int M);
 // The tile kernel with integer operands (tfq_gemm_exact.hip), reached through launch_gemm: products that may not round
-// their weights.  Any scratch size is served (less scratch, fewer K parts); gemm_exact_us is its modelled time.
+// their weights.  Any scratch size is served (less scratch, fewer K parts).
 bool gemm_exact_serves(const tfq_weight* w, int x_dtype, int M);
-double gemm_exact_us(const tfq_weight* w, int x_dtype, int M, size_t scratch_bytes);
 size_t gemm_exact_scratch_bytes(const tfq_weight* w, int x_dtype, int M);
 int launch_gemm_exact(const tfq_weight* w, const void* x, int x_dtype, int M, void* y, int y_dtype, hipStream_t s, void* scratch,
                       size_t scratch_bytes);
