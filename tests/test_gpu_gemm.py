@@ -139,9 +139,14 @@ def test_gemm_integer_operands_non_finite(O, tfq, gpu, fmt):
     x[4, 100] = float("nan")
     x[5] = 0
     x[5, 9] = 2.0 ** 120  # times an unscaled integer this overflows, times the weight it does not
+    x[6] = 0
+    x[6, 500] = 3.4e38    # its bf16 is infinite
+    x[7] = float("inf")
+    x[8] = float("nan")
     for xt in (x, x.bfloat16()):
-        y = W.gemm(xt)
         ref = torch.cat([W.gemv(xt[:16].contiguous()), W.gemv(xt[16:].contiguous())])
+        y = W.gemm(xt)
+        assert torch.equal(torch.isnan(W.gemm(xt, workspace=False)), torch.isnan(ref))
         assert torch.equal(torch.isnan(y), torch.isnan(ref)) and torch.equal(torch.isinf(y), torch.isinf(ref))
         assert torch.equal(y[torch.isinf(y)], ref[torch.isinf(ref)])
         f = torch.isfinite(ref)

@@ -14,6 +14,7 @@
 //   SB256A3               I = sc (code - 4),   scale d / 7 per 256,             offset 4 sc d / 7 - dm mc per 16
 //   Q_4                   I = 10^4 level (14 bits and sign, two bf16), scale per 256
 //   Q_G_6                 I = sc (code - 32)   (13 bits, two bf16),    scale d per 256
+// (of the last two the operands are I 2^-23 and I 2^-20, so that no sum of 256 leaves the range before its scale)
 // bf16 activations are exact operands.  fp32 activations go in as a bf16 high part and the bf16 of the rest (two
 // operands, the 16 bits that the decode kernels keep too), for the wire formats, whose other kernel multiplies in
 // fp32, as three (24 bits).  The offsets times the activations' group sums are a product of their own, one MFMA per
@@ -73,14 +74,14 @@ __device__ __forceinline__ float bf_hi(uint32_t v) { return __uint_as_float(v & 
 struct Q4Table {
     uint32_t hi_b[2], hi_t[2], lo_b[2], lo_t[2];  // low / high bytes of the two parts, entry m in byte m % 4 of word m / 4
 };
-constexpr uint32_t bf16_of_int(int v) {  // exact: at most eight significant bits
+constexpr uint32_t bf16_of_int(int v) {  // v 2^-23, exact: at most eight significant bits
     if (v == 0) return 0;
     const uint32_t sign = v < 0 ? 0x8000u : 0u;
     uint32_t m = v < 0 ? (uint32_t)-v : (uint32_t)v;
     int e = 0;
     while ((m >> e) > 1) ++e;
     const uint32_t frac = e >= 7 ? (m >> (e - 7)) : (m << (7 - e));
-    return sign | ((uint32_t)(127 + e) << 7) | (frac & 0x7Fu);
+    return sign | ((uint32_t)(127 - 23 + e) << 7) | (frac & 0x7Fu);
 }
 constexpr Q4Table make_q4_table() {
     constexpr int L[8] = {1260, 3976, 6508, 9275, 12392, 15995, 20522, 27178};
@@ -133,25 +134,60 @@ __device__ __forceinline__ void decode16x2(uint32_t v, float sc, uint32_t C, uin
     o1 = uint4{o[4], o[5], o[6], o[7]};
 }
 
-// The product of one output in fp32, weight by weight, as the wavefront-per-row kernel forms it: where a sum of the
-// two-part integers is not finite (an infinite activation gives inf - inf, a huge one overflows the unscaled sum)
-// the output is formed again this way.
+__device__ __forceinline__ bool finite_f32(float v) { return (__float_as_uint(v) & 0x7F800000u) != 0x7F800000u; }
+
+// An infinite activation meets two parts of a weight here, which may differ in sign or be zero, and gives a NaN where
+// the fp32 product gives an infinity.  Where outputs of the wire formats (whose other kernel multiplies in fp32) are
+// not finite, the wavefront looks the activation row over: a NaN makes the output a NaN; else the infinities alone
+// decide, by the signs of their weights (and stop as soon as every output is a NaN); fp32 values that round to an
+// infinite bf16 part have their outputs formed again weight by weight.  All 64 lanes call this together.
 template <int FMT, int XP>
-__device__ __attribute__((noinline)) float exact_output(const uint8_t* W, const void* X, int K, int m, int n) {
-    const int nblk = K >> 8;
+__device__ __attribute__((noinline)) float repair_non_finite(const uint8_t* W, const void* X, int K, int m, int col, bool valid, float v) {
+    const int nblk = K >> 8, lane = threadIdx.x & 63;
     constexpr int BB = spec_of(FMT).block_bytes;
-    float v = 0.0f;
-    for (int blk = 0; blk < nblk; ++blk) {
-        const uint8_t* p = W + ((size_t)n * nblk + blk) * BB;
-        for (int i = 0; i < 256; ++i) {
-            const size_t k = (size_t)m * K + (size_t)blk * 256 + i;
-            const float xv = XP == 1 ? __uint_as_float((uint32_t)static_cast<const unsigned short*>(X)[k] << 16) : static_cast<const float*>(X)[k];
-            v = __builtin_fmaf(decode_weight<FMT>(p, (uint32_t)i), xv, v);
+    const bool flag = valid && !finite_f32(v);
+    auto value = [&](int row, int k) {
+        return XP == 1 ? __uint_as_float((uint32_t)static_cast<const unsigned short*>(X)[(size_t)row * K + k] << 16)
+                       : static_cast<const float*>(X)[(size_t)row * K + k];
+    };
+    auto weight = [&](int k) { return decode_weight<FMT>(W + ((size_t)col * nblk + (k >> 8)) * BB, (uint32_t)(k & 255)); };
+    uint64_t todo = __ballot(flag);
+    while (todo) {
+        const int row = __builtin_amdgcn_readlane(m, __builtin_ctzll(todo));
+        const bool mine = flag && m == row;
+        todo &= ~__ballot(mine);
+        bool nan = false, inf = false, huge = false;
+        for (int k = lane; k < K; k += 64) {
+            const uint32_t u = __float_as_uint(value(row, k)) & 0x7FFFFFFFu;
+            nan |= u > 0x7F800000u;
+            inf |= u == 0x7F800000u;
+            huge |= u >= 0x7F7F8000u && u < 0x7F800000u;
+        }
+        if (__ballot(nan)) {
+            if (mine) v = __uint_as_float(0x7FC00000u);
+        } else if (__ballot(inf)) {
+            float r = 0.0f;
+            for (int k0 = 0; k0 < K && __ballot(mine && r == r); k0 += 64) {
+                const float xv = value(row, k0 + lane);
+                uint64_t at = __ballot(!finite_f32(xv));
+                while (at) {
+                    const int p = __builtin_ctzll(at);
+                    at &= at - 1;
+                    const float xi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(xv), p));
+                    if (mine) r += weight(k0 + p) * xi;
+                }
+            }
+            if (mine) v = r;
+        } else if (__ballot(huge)) {
+            if (mine) {
+                float r = 0.0f;
+                for (int k = 0; k < K; ++k) r = __builtin_fmaf(weight(k), value(row, k), r);
+                v = r;
+            }
         }
     }
     return v;
 }
-__device__ __forceinline__ bool finite_f32(float v) { return (__float_as_uint(v) & 0x7F800000u) != 0x7F800000u; }
 
 template <int FMT, int XP, int TM>
 constexpr int lds_uint4s() {
@@ -331,10 +367,10 @@ __global__ __launch_bounds__(THREADS, TM == 128 || XP == 3 ? 2 : 3) void gemm_ex
                 wd[512 + 8 * h] = uint4{el[0], el[1], ol[0], ol[1]};
             }
             // the scale takes 10^-4 in one rounding
-            if constexpr (U == 0) wscale[par * 128 + row] = (float)((double)half_bits_to_float(hdd) * 1e-4);
+            if constexpr (U == 0) wscale[par * 128 + row] = (float)((double)half_bits_to_float(hdd) * (8388608.0 * 1e-4));
         } else if constexpr (FMT == TFQ_Q_G_6) {
             const uint32_t scw = U < 4 ? hdr.x : hdr.y;
-            const float sc = (float)((int32_t)(scw << (24 - 8 * (U & 3))) >> 24), c = -32.0f * sc;
+            const float sc = (float)((int32_t)(scw << (24 - 8 * (U & 3))) >> 24) * (1.0f / 1048576.0f), c = -32.0f * sc;
             uint32_t hi[8], lo[8];
 #pragma unroll
             for (int t = 0; t < 8; ++t) {
@@ -353,7 +389,7 @@ __global__ __launch_bounds__(THREADS, TM == 128 || XP == 3 ? 2 : 3) void gemm_ex
             wd[8] = uint4{hi[4], hi[5], hi[6], hi[7]};
             wd[512] = uint4{lo[0], lo[1], lo[2], lo[3]};
             wd[520] = uint4{lo[4], lo[5], lo[6], lo[7]};
-            if constexpr (U == 0) wscale[par * 128 + row] = half_bits_to_float(hdd);
+            if constexpr (U == 0) wscale[par * 128 + row] = half_bits_to_float(hdd) * 1048576.0f;
         } else if constexpr (F::BYTES) {
             const uint32_t scw = (U >> 1) == 0 ? hdr.x : (U >> 1) == 1 ? hdr.y : (U >> 1) == 2 ? hdr.z : hdr.w;
             const float sc = (float)((scw >> (16 * (U & 1) + 8 * half)) & 255u);
@@ -588,17 +624,16 @@ __global__ __launch_bounds__(THREADS, TM == 128 || XP == 3 ? 2 : 3) void gemm_ex
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int m = m0 + wm * (TM / 2) + i * 16 + 4 * fk + e;
-                if (m < M && col < N) {
-                    const size_t o = (size_t)m * N + col;
-                    float v = acc[i][j][e];
+                const bool valid = m < M && col < N;
+                const size_t o = (size_t)m * N + col;
+                float v = acc[i][j][e];
+                if constexpr (F::WIRE) {
+                    if (S == 1 && __ballot(valid && !finite_f32(v))) v = repair_non_finite<FMT, XP>(args.W, args.X, K, m, col, valid, v);
+                }
+                if (valid) {
                     if (S > 1) args.partial[(size_t)split * M * N + o] = v;
-                    else {
-                        if constexpr (F::WIRE) {
-                            if (!finite_f32(v)) v = exact_output<FMT, XP>(args.W, args.X, K, m, col);
-                        }
-                        if (args.y_bf16) reinterpret_cast<unsigned short*>(args.Y)[o] = (unsigned short)bf16_rne(v);
-                        else reinterpret_cast<float*>(args.Y)[o] = v;
-                    }
+                    else if (args.y_bf16) reinterpret_cast<unsigned short*>(args.Y)[o] = (unsigned short)bf16_rne(v);
+                    else reinterpret_cast<float*>(args.Y)[o] = v;
                 }
             }
         }
@@ -608,12 +643,14 @@ __global__ __launch_bounds__(THREADS, TM == 128 || XP == 3 ? 2 : 3) void gemm_ex
 template <int FMT, int XP>
 __global__ __launch_bounds__(256) void reduce_exact_kernel(ExactArgs args) {
     const size_t n = (size_t)args.M * args.N, i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    float v = args.partial[i];
-    for (int sp = 1; sp < args.ksplit; ++sp) v += args.partial[(size_t)sp * n + i];
+    const bool valid = i < n;
+    float v = 0.0f;
+    for (int sp = 0; sp < args.ksplit; ++sp) v += valid ? args.partial[(size_t)sp * n + i] : 0.0f;
     if constexpr (Form<FMT>::WIRE) {
-        if (!finite_f32(v)) v = exact_output<FMT, XP>(args.W, args.X, args.K, (int)(i / args.N), (int)(i % args.N));
+        if (__ballot(valid && !finite_f32(v)))
+            v = repair_non_finite<FMT, XP>(args.W, args.X, args.K, (int)(i / args.N), (int)(i % args.N), valid, v);
     }
+    if (!valid) return;
     if (args.y_bf16) reinterpret_cast<unsigned short*>(args.Y)[i] = (unsigned short)bf16_rne(v);
     else reinterpret_cast<float*>(args.Y)[i] = v;
 }
