@@ -29,7 +29,7 @@
 // but a ragged prompt (333 rows) then pads to 512 rows instead of 384.  Activations are fetched two steps ahead, codes
 // three.  Few rows take 64-row tiles, three workgroups per unit.
 // Measured, before (slices of 4 to 16 rows through the decode kernels) and now: Q_G_4 fp32 333 rows 4096 x 14336
-// 657 -> 171 us, B32S8 the same 700 -> 133 us; 512 bf16 rows of 14336 x 4096: Q_4 7580 -> 155 us, Q_G_6 5360 -> 164 us,
+// 657 -> 171 us, B32S8 the same 700 -> 133 us; 512 bf16 rows of 14336 x 4096: Q_4 7580 -> 150-195 us, Q_G_6 5360 -> 165-185 us,
 // SB256A3 789 -> 135 us.  Below 17 rows the decode kernels stay.
 
 #include <algorithm>
@@ -49,7 +49,7 @@ template <int FMT>
 struct Form {
     static constexpr bool WIRE = FMT == TFQ_Q_4 || FMT == TFQ_Q_G_6;
     static constexpr bool BYTES = tiled_header_in_bytes(FMT);  // sixteen groups of 16, header one code per byte
-    static constexpr bool BLOCK_SCALE = WIRE || BYTES;         // one scale per 256 weights: the sums of a block stay unscaled
+    static constexpr bool BLOCK_SCALE = WIRE || BYTES;         // the sums of a block of 256 stay unscaled until its end
     static constexpr int WP = WIRE ? 2 : 1;                    // bf16 operands per weight
     static constexpr int OG = BYTES ? 16 : (FMT == TFQ_Q_G_4 || FMT == TFQ_Q_G_3) ? 8 : 0;  // offset groups per block
     static constexpr bool SC_OFFSET = FMT == TFQ_SB256A3;      // the centred codes bring a second offset product
@@ -89,7 +89,7 @@ constexpr Q4Table make_q4_table() {
     for (int m = 0; m < 8; ++m) {
         int e = 0;
         while ((L[m] >> e) > 1) ++e;
-        const int hi = (L[m] >> (e - 7)) << (e - 7), lo = L[m] - hi;  // lo < 2^(e - 7) <= 2^7
+        const int hi = ((L[m] + (1 << (e - 8))) >> (e - 7)) << (e - 7), lo = L[m] - hi;  // |lo| <= 2^(e - 8) <= 2^6
         const uint32_t h = bf16_of_int(hi), l = bf16_of_int(lo);
         t.hi_b[m / 4] |= (h & 255u) << (8 * (m % 4));
         t.hi_t[m / 4] |= (h >> 8) << (8 * (m % 4));
@@ -477,12 +477,13 @@ __global__ __launch_bounds__(THREADS, TM == 128 || XP == 3 ? 2 : 3) void gemm_ex
             for (int p = 0; p < WP; ++p) bf[p][j] = wb[p * 512 + j * 64];
             if constexpr (!F::BLOCK_SCALE) sc[j] = wscale[(U & 1) * 128 + wn_ * 64 + j * 16 + fr];
         }
-        f32x4_t t[2][NJ];
+        constexpr int TS = F::WIRE ? 1 : 2;  // (the wire formats' registers are full)
+        f32x4_t t[TS][NJ];
         auto apply = [&](int i) __attribute__((always_inline)) {  // the step's scale
 #pragma unroll
             for (int j = 0; j < NJ; ++j) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) acc[i][j][e] = __builtin_fmaf(sc[j], t[i & 1][j][e], acc[i][j][e]);
+                for (int e = 0; e < 4; ++e) acc[i][j][e] = __builtin_fmaf(sc[j], t[i % TS][j][e], acc[i][j][e]);
                 // (the optimizer would otherwise keep a block's eight sums and add them at its end, out of registers)
                 f32x4_t& done = acc[i][j];
                 asm volatile("" : "+v"(done));
@@ -493,21 +494,21 @@ __global__ __launch_bounds__(THREADS, TM == 128 || XP == 3 ? 2 : 3) void gemm_ex
             uint4 af[XP];
 #pragma unroll
             for (int p = 0; p < XP; ++p) af[p] = xb[p * XPL + i * 64];
-            // The small parts first.  Three-part activations: the five small products of a step meet in a sum of their
-            // own, so that the block's sum is rounded twice per step and not six times (error 2.2e-7 -> 1.2e-7).
+            // The small parts first.  The wire formats add a step's products to the block's sum in fp32: kept in the matrix
+            // cores over its 16 products its error was up to 1.45 times the fp32 kernel's.
 #pragma unroll
             for (int p = XP - 1; p >= 0; --p)
 #pragma unroll
                 for (int q = WP - 1; q >= 0; --q)
 #pragma unroll
                     for (int j = 0; j < NJ; ++j) {
-                        const bool first = p == XP - 1 && q == WP - 1, apart = XP == 3 && (p || q);
-                        if (F::BLOCK_SCALE && !apart) blk_acc[i][j] = mm(af[p], bf[q][j], (first || XP == 3) && U == 0 ? zero4 : blk_acc[i][j]);
-                        else t[i & 1][j] = mm(af[p], bf[q][j], first ? zero4 : t[i & 1][j]);
+                        const bool first = p == XP - 1 && q == WP - 1;
+                        if constexpr (F::BYTES) blk_acc[i][j] = mm(af[p], bf[q][j], first && U == 0 ? zero4 : blk_acc[i][j]);
+                        else t[i % TS][j] = mm(af[p], bf[q][j], first ? zero4 : t[i % TS][j]);
                     }
-            if constexpr (XP == 3) {
+            if constexpr (F::WIRE) {
 #pragma unroll
-                for (int j = 0; j < NJ; ++j) blk_acc[i][j] += t[i & 1][j];
+                for (int j = 0; j < NJ; ++j) blk_acc[i][j] = U == 0 ? t[i % TS][j] : blk_acc[i][j] + t[i % TS][j];
             }
             // one row of tiles behind the matrix instructions, which then have no result to wait for
             if constexpr (!F::BLOCK_SCALE) {
