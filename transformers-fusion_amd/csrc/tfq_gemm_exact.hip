@@ -29,7 +29,7 @@
 // but a ragged prompt (333 rows) then pads to 512 rows instead of 384.  Activations are fetched two steps ahead, codes
 // three.  Few rows take 64-row tiles, three workgroups per unit.
 // Measured, before (slices of 4 to 16 rows through the decode kernels) and now: Q_G_4 fp32 333 rows 4096 x 14336
-// 657 -> 171 us, B32S8 the same 700 -> 133 us; 512 bf16 rows of 14336 x 4096: Q_4 7580 -> 150-195 us, Q_G_6 5360 -> 165-185 us,
+// 657 -> 171 us, B32S8 the same 700 -> 133 us; 512 bf16 rows of 14336 x 4096: Q_4 7580 -> 197 us, Q_G_6 5360 -> 184 us,
 // SB256A3 789 -> 135 us.  Below 17 rows the decode kernels stay.
 
 #include <algorithm>

@@ -1,4 +1,4 @@
-// Dequant-fused GEMV for the formats that have no matrix-core kernel (plain 2- and 4-bit lattice,
+// Dequant-fused GEMV for the formats that have no matrix-core decode kernel (plain 2- and 4-bit lattice,
 // Q_G_6, the grouped-lattice fallback ids and raw fp32 blocks), on the wire layout:
 //   y[b][n] = sum_k x[b][k] * W[n][k]
 // Replaces Qwen35Engine::gemm (src/adapters/tools/qwen35_engine.cpp:54-101) for
