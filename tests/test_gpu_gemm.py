@@ -152,3 +152,27 @@ def test_gemm_integer_operands_non_finite(O, tfq, gpu, fmt):
         f = torch.isfinite(ref)
         assert torch.allclose(y[f], ref[f], rtol=1e-4, atol=1e-5)
     W.close()
+
+
+@pytest.mark.parametrize("fmt,dtype,M,N,K,workspace,slices", [
+    ("Q_G_4", "f32", 17, 1024, 4096, False, True), ("Q_G_4", "f32", 200, 1024, 4096, False, False),
+    ("B32S8", "f32", 33, 512, 14336, False, True), ("Q_G_3", "f32", 24, 512, 4096, False, True),
+    ("SB256A3", "bf16", 40, 1024, 4096, False, True), ("Q_G_2", "f32", 32, 256, 14336, False, True),
+    ("Q_G_6", "bf16", 17, 256, 4096, False, True), ("Q_4", "f32", 20, 14336, 1024, False, False),
+    ("B32S4", "f32", 18, 28672, 4096, True, True), ("Q_G_4", "f32", 64, 28672, 4096, True, False)])
+def test_gemm_rows_in_slices_or_tiles(tfq, gpu, fmt, dtype, M, N, K, workspace, slices):
+    """Where a matrix makes few tiles and there is no scratch to split K, and for a few fp32 rows on a tall matrix, the
+    rows go through the decode kernels 16 at a time, bit for bit; both ways are the product (float64, the decoded matrix)."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(11)
+    W = tfq.Weight(fmt, N, K, tfq.encode(fmt, torch.randn(N * K, device=gpu, generator=g) * 0.02))
+    x = torch.randn(M, K, device=gpu, generator=g)
+    x = x.bfloat16() if dtype == "bf16" else x
+    y = W.gemm(x, workspace=workspace)
+    rows = torch.cat([W.gemv(x[m:m + 16].contiguous()) for m in range(0, M, 16)])
+    if K <= 4096:  # (a longer K is split by gemv's own workspace, which the slices of a call without one do not have)
+        assert torch.equal(y, rows) == slices
+    want = x.double() @ W.decode().reshape(N, K).double().T
+    for v in (y, rows):
+        assert float((v.double() - want).norm() / want.norm()) <= 1e-5  # 16 bits of an fp32 activation, as above
+    W.close()

@@ -583,8 +583,47 @@ static size_t slice_split_bytes(const tfq_weight* w) {
     return w->layout == TFQ_LAYOUT_TILED16 ? gemv_rows16_split_bytes(w->fmt, w->N, w->K) : 0;
 }
 
+// The same question for the integer tile kernel: its plan with the scratch there is against M rows in 16-row slices
+// through the decode kernels.  Without scratch it cannot split K, and a matrix of few row tiles then leaves most compute
+// units idle (1024 x 4096, 17 fp32 rows of Q_G_4: 84 us against 21 us in slices; 4096 x 14336: 281 against 52 us); with
+// scratch the slices win below about 20 fp32 rows of the 4-bit formats on tall matrices (28672 x 4096: 61 against 48 us).
+// A pass of the decode kernels over the matrix costs (us) about 3 + the staging of its activation slots (two per fp32
+// row) + the weights, fitted to passes of 256 x 1024 to 28672 x 4096 and 4096 x 14336 within 20 %.  The slices have to be
+// 8 % below.  Of 3068 measured cases (16 format / type pairs, 17 to 200 rows, with and without scratch) 52 are then more
+// than 3 % slower than the faster side, nine of those through a wrong choice of the slices, at most 15 %; without the
+// comparison 728 were more than 5 % slower.
+static bool exact_cheaper(const tfq_weight* w, int x_dtype, int M, size_t scratch_bytes, bool split_scratch) {
+    // (a taller matrix takes the decode kernels more than one round of workgroups: 128256 x 4096 at 32 fp32 rows 328 us
+    // in slices, 205 us here; a longer K leaves the formats without a sixteen-row kernel room for fewer and fewer staged
+    // rows, and in the end refuses a bf16 y)
+    if (w->N > 32768 || (w->layout == TFQ_LAYOUT_TILED16 && !gemv_rows16_supported(w->fmt) && w->K > 14336)) return true;
+    const int f = canonical(w->fmt);
+    const double mw = (double)w->N * (double)w->K * 1e-6, kk = (double)w->K / 1024.0;
+    const bool f32 = x_dtype == TFQ_F32;
+    int rows;     // of a pass
+    double pass;  // its time, us
+    if (w->layout == TFQ_LAYOUT_WIRE) {
+        rows = 4;
+        pass = 3.5 + std::max(0.30 * mw, 0.0013 * (double)w->N);
+    } else if (gemv_rows16_supported(w->fmt)) {  // fp32 rows: eight per pass
+        rows = 8;
+        pass = 3.2 + (f == TFQ_B32S4 ? 0.066 : f == TFQ_Q_G_4 ? 0.085 : 0.13) * mw;
+        pass += split_scratch && w->K > 4096 ? 0.95 * 4.0 + 3.5 : 0.95 * kk;
+    } else {
+        // four fp32 or eight bf16 rows in eight slots, half of them where eight staged ones do not fit in LDS
+        const int slots = w->K <= (f == TFQ_Q_G_3 ? 8192 : 7168) ? 8 : 4;
+        rows = f32 ? slots / 2 : slots;
+        if (f == TFQ_Q_G_3) pass = 3.0 + 0.08 * slots * kk + 0.075 * mw;
+        else if (!f32) pass = 3.0 + 0.07 * slots * kk + 0.105 * mw;
+        else pass = 3.0 + (slots == 8 ? 1.02 : 0.1 * slots) * kk + (slots == 8 ? 0.115 : 0.09) * mw;
+    }
+    const int passes = M / 16 * ((16 + rows - 1) / rows) + (M % 16 + rows - 1) / rows;
+    return passes * pass >= 0.92 * gemm_exact_us(w, x_dtype, M, scratch_bytes);
+}
+
 size_t gemm_scratch_bytes(const tfq_weight* w, int x_dtype, int M) {
-    if (gemm_exact_serves(w, x_dtype, M)) return gemm_exact_scratch_bytes(w, x_dtype, M);
+    if (gemm_exact_serves(w, x_dtype, M))
+        return exact_cheaper(w, x_dtype, M, ~(size_t)0, true) ? gemm_exact_scratch_bytes(w, x_dtype, M) : slice_split_bytes(w);
     if (!tile_kernel_serves(w, x_dtype, M)) return M > 4 ? slice_split_bytes(w) : 0;
     const GemmPlan p = plan_for(w, M, ~(size_t)0);
     if (slices_cheaper(w, M, p.us, true)) return slice_split_bytes(w);
@@ -594,9 +633,10 @@ size_t gemm_scratch_bytes(const tfq_weight* w, int x_dtype, int M) {
 
 int launch_gemm(const tfq_weight* w, const void* x, int x_dtype, int M, void* y, int y_dtype, hipStream_t s, void* scratch,
                 size_t scratch_bytes) {
-    if (gemm_exact_serves(w, x_dtype, M)) return launch_gemm_exact(w, x, x_dtype, M, y, y_dtype, s, scratch, scratch_bytes);
     const size_t slice_ws = slice_split_bytes(w);
     const bool slices_split = scratch && slice_ws && scratch_bytes >= slice_ws;
+    if (gemm_exact_serves(w, x_dtype, M) && exact_cheaper(w, x_dtype, M, scratch ? scratch_bytes : 0, slices_split))
+        return launch_gemm_exact(w, x, x_dtype, M, y, y_dtype, s, scratch, scratch_bytes);
     if (tile_kernel_serves(w, x_dtype, M) && !slices_cheaper(w, M, plan_for(w, M, scratch ? scratch_bytes : 0).us, slices_split)) {
         if (w->N > 0x7FFFFFF0 || w->K > 0x7FFFFFF0 || w->dev_bytes >= 0xFFFFF000ull) return fail(TFQ_ERR_SHAPE, "gemm: matrix too large");
         switch (canonical(w->fmt)) {

@@ -30,7 +30,10 @@
 // three.  Few rows take 64-row tiles, three workgroups per unit.
 // Measured, before (slices of 4 to 16 rows through the decode kernels) and now: Q_G_4 fp32 333 rows 4096 x 14336
 // 657 -> 171 us, B32S8 the same 700 -> 133 us; 512 bf16 rows of 14336 x 4096: Q_4 7580 -> 197 us, Q_G_6 5360 -> 184 us,
-// SB256A3 789 -> 135 us.  Below 17 rows the decode kernels stay.
+// SB256A3 789 -> 135 us.  Up to 16 rows tfq_gemv's kernels serve every format, above that the
+// faster of the two by a model (exact_cheaper).  For the wire formats the step at 17 rows is where the entry points part,
+// not where the kernels cross: 14336 x 4096 bf16 Q_4 takes 93 us at 16 rows (four passes) and 40 us at 17 to 24 rows here,
+// Q_G_6 90 and 45 us; at 1024 x 4096 the two meet (16 us).  The Tiled16 formats cross between 16 and 20 rows.
 
 #include <algorithm>
 #include <atomic>
@@ -730,6 +733,22 @@ bool gemm_exact_serves(const tfq_weight* w, int x_dtype, int M) {
 size_t gemm_exact_scratch_bytes(const tfq_weight* w, int x_dtype, int M) {
     const ExactPlan p = plan_exact(w->N, w->K, M, planes_of(w, x_dtype), ~(size_t)0);
     return p.ksplit > 1 ? (size_t)p.ksplit * (size_t)M * (size_t)w->N * 4 : 0;
+}
+
+// What a call with this much scratch takes (us): the plan's model, which prices every format of a kind alike, times
+// about the median of measured over modelled (17 to 200 rows, 256 x 1024 to 128256 x 4096; nine tenths within 25 % of it).
+double gemm_exact_us(const tfq_weight* w, int x_dtype, int M, size_t scratch_bytes) {
+    const bool f32 = x_dtype == TFQ_F32;
+    double fit = 1.0;
+    switch (canonical(w->fmt)) {
+        case TFQ_B32S4: fit = 0.86; break;
+        case TFQ_B32S8: case TFQ_Q_G_8: case TFQ_Q_8: fit = 0.9; break;
+        case TFQ_Q_G_4: case TFQ_Q_G_3: fit = 1.05; break;
+        case TFQ_SB256A3: fit = f32 ? 1.1 : 0.95; break;
+        case TFQ_Q_G_2: case TFQ_SB256A2: fit = f32 ? 1.0 : 0.89; break;
+        default: fit = f32 ? 1.1 : 1.25; break;
+    }
+    return fit * plan_exact(w->N, w->K, M, planes_of(w, x_dtype), scratch_bytes).us;
 }
 
 int launch_gemm_exact(const tfq_weight* w, const void* x, int x_dtype, int M, void* y, int y_dtype, hipStream_t s, void* scratch,

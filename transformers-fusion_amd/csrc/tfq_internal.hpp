@@ -485,14 +485,16 @@ int launch_moe_ffn_capacity(const tfq_weight* const* gate, const tfq_weight* con
                             size_t workspace_bytes, int64_t* dropped, hipStream_t s);
 // `scratch` (optional, device memory) lets the tile kernel split K over several workgroups per output tile when
 // the tiles alone do not fill the GPU; gemm_scratch_bytes says how much a call would use, gemm_scratch_bound is
-// an upper bound for any matrix with at most `rows` x `cols` outputs (a split never makes more than 256 tiles).
+// what the feed-forward calls set aside for any matrix with at most `rows` x `cols` outputs: all the bf16 tile kernel
+// would use (at most eight parts, 256 tiles); the integer one may plan more parts and makes do with what there is.
 int launch_gemm(const tfq_weight* w, const void* x, int x_dtype, int M, void* y, int y_dtype,
                 hipStream_t s, void* scratch = nullptr, size_t scratch_bytes = 0);
 size_t gemm_scratch_bytes(const tfq_weight* w, int x_dtype, int M);
 // The tile kernel with integer operands (tfq_gemm_exact.hip), reached through launch_gemm: products that may not round
-// their weights.  Any scratch size is served (less scratch, fewer K parts).
+// their weights.  Any scratch size is served (less scratch, fewer K parts); gemm_exact_us says how long it would take.
 bool gemm_exact_serves(const tfq_weight* w, int x_dtype, int M);
 size_t gemm_exact_scratch_bytes(const tfq_weight* w, int x_dtype, int M);
+double gemm_exact_us(const tfq_weight* w, int x_dtype, int M, size_t scratch_bytes);
 int launch_gemm_exact(const tfq_weight* w, const void* x, int x_dtype, int M, void* y, int y_dtype, hipStream_t s, void* scratch,
                       size_t scratch_bytes);
 // Grouped form of the prefill tile kernel: several products over matrices of one format and one N x K, each with
