@@ -154,6 +154,40 @@ def test_gemm_integer_operands_non_finite(O, tfq, gpu, fmt):
     W.close()
 
 
+@pytest.mark.parametrize("fmt,dtype", [f for f in EXACT_FMTS if f[0] not in ("Q_4", "Q_G_6", "Q_4_K_H")])
+def test_gemm_tiled_operands_range(O, tfq, gpu, fmt, dtype):
+    """Infinite, not-a-number, huge and tiny activations on the formats of the tiled layout: the same outputs are NaN as
+    with the decode kernels, and what is finite there is finite and the same to fp32 rounding (an fp32 activation keeps
+    16 bits).  A whole row of the largest power of two whose group sums the decode kernels hold: the tile kernel leaves
+    more than a group's sum unscaled."""
+    import torch
+    M, N, K = 64, 40, 768
+    top = {"B32S8": 111, "Q_G_8": 111, "Q_8": 111, "SB256A3": 113, "SB256A2": 114, "Q_G_2": 116}.get(fmt, 115)
+    W = tfq.Weight(fmt, N, K, O.encode_tensor(fmt, O.rng_normal(42, N * K, 0.02)))
+    x = torch.from_numpy(O.rng_normal(43, M * K, 1.0).reshape(M, K)).to(gpu)
+    x[2, 7] = float("inf")
+    x[3, 300] = -float("inf")
+    x[4, 700] = float("nan")
+    x[5] = 0
+    x[5, 9] = 2.0 ** 120
+    x[6] = 2.0 ** top
+    x[7] = -(2.0 ** top)
+    x[8] *= 2.0 ** (top - 3)
+    x[9] *= 2.0 ** -100
+    x = x.bfloat16() if dtype == "bf16" else x
+    ref = torch.cat([W.gemv(x[m:m + 16].contiguous()) for m in range(0, M, 16)])
+    for ws in (True, False):
+        y = W.gemm(x, workspace=ws)
+        assert torch.equal(torch.isnan(y), torch.isnan(ref)), (torch.isnan(y) != torch.isnan(ref)).any(1).nonzero().flatten().tolist()
+        f = torch.isfinite(ref)
+        assert f[6:10].all()
+        assert torch.isfinite(y[f]).all(), (torch.isfinite(y) != f).any(1).nonzero().flatten().tolist()
+        for m in range(M):
+            if f[m].all():
+                assert float((y[m].double() - ref[m].double()).norm() / ref[m].double().norm()) <= 1e-5, m
+    W.close()
+
+
 @pytest.mark.parametrize("fmt,dtype,M,N,K,workspace,slices", [
     ("Q_G_4", "f32", 17, 1024, 4096, False, True), ("Q_G_4", "f32", 200, 1024, 4096, False, False),
     ("B32S8", "f32", 33, 512, 14336, False, True), ("Q_G_3", "f32", 24, 512, 4096, False, True),

@@ -14,7 +14,9 @@
 //   SB256A3               I = sc (code - 4),   scale d / 7 per 256,             offset 4 sc d / 7 - dm mc per 16
 //   Q_4                   I = 10^4 level (14 bits and sign, two bf16), scale per 256
 //   Q_G_6                 I = sc (code - 32)   (13 bits, two bf16),    scale d per 256
-// (of the last two the operands are I 2^-23 and I 2^-20, so that no sum of 256 leaves the range before its scale)
+// (of the last two the operands are I 2^-23 and I 2^-20, so that no sum of 256 leaves the range before its scale; of
+// the three formats above them, and of their offsets, the integers times 2^-6: as plain integers the sums of 256 left
+// the range one power of two before those of the decode kernels, which scale sums of 16; now 3 to 7 powers after them)
 // bf16 activations are exact operands.  fp32 activations go in as a bf16 high part and the bf16 of the rest (two
 // operands, the 16 bits that the decode kernels keep too), for the wire formats, whose other kernel multiplies in
 // fp32, as three (24 bits).  The offsets times the activations' group sums are a product of their own, one MFMA per
@@ -46,6 +48,7 @@ namespace tfq {
 
 namespace {
 
+constexpr float kSumScale = 64.0f;  // the 16-weight-group formats' operands are divided by it (see above), their scales multiplied
 constexpr int TN = 128, THREADS = 256;  // tokens of a tile: a template parameter, 128 or 64
 
 template <int FMT>
@@ -117,9 +120,9 @@ __device__ __forceinline__ void q4_levels(uint32_t q, uint32_t (&hi)[2], uint32_
     lo[1] = __builtin_amdgcn_perm(lt, lb, 0x07030602u);
 }
 
-// sixteen 2-bit codes of the true-width layout -> I = sc * code as bf16, in order
+// sixteen 2-bit codes of the true-width layout -> I = sc * code / kSumScale as bf16, in order (C: see f16_bias)
 __device__ __forceinline__ void decode16x2(uint32_t v, float sc, uint32_t C, uint4& o0, uint4& o1) {
-    const float c2 = -1024.0f * sc;
+    const float c2 = -16.0f * sc;
     uint32_t o[8];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -298,7 +301,10 @@ __global__ __launch_bounds__(THREADS, TM == 128 || XP == 3 ? 2 : 3) void gemm_ex
             hnext = *reinterpret_cast<const uint4*>(p + tiled_header_offset(FMT, r16, 0));
         }
     };
-    uint32_t nib_mask = 0x000F000Fu, f16_bias = 0x64006400u;
+    // f16_bias: OR-ed under a code n it makes the binary16 number 1024 + n, of the 16-weight-group formats 16 + n / 64,
+    // which divides their operands without an operation (a multiplication of sc: SB256A3 142 -> 144 us, 512 x 14336 x 4096)
+    static_assert(kSumScale == 64.0f);
+    uint32_t nib_mask = 0x000F000Fu, f16_bias = F::BYTES ? 0x4C004C00u : 0x64006400u;
     float one = 1.0f;
     asm volatile("" : "+v"(nib_mask), "+v"(f16_bias), "+v"(one));  // kept in registers (see decode8); a literal 1 would split its mixed multiply-add
 
@@ -402,8 +408,9 @@ __global__ __launch_bounds__(THREADS, TM == 128 || XP == 3 ? 2 : 3) void gemm_ex
                 wd[0] = o0;
                 wd[8] = o1;
             } else {
-                wd[0] = decode8(r[0], sc, -4.0f * sc, nib_mask, f16_bias);
-                wd[8] = decode8(r[1], sc, -4.0f * sc, nib_mask, f16_bias);
+                // decode8 takes 1024 sc off its addend: -(16 + 4 / 64) sc is left, exactly
+                wd[0] = decode8(r[0], sc, (1024.0f - 16.0f - 4.0f / kSumScale) * sc, nib_mask, f16_bias);
+                wd[8] = decode8(r[1], sc, (1024.0f - 16.0f - 4.0f / kSumScale) * sc, nib_mask, f16_bias);
             }
             if constexpr (U == 0) {
                 constexpr Spec sp = spec_of(FMT);
@@ -416,10 +423,10 @@ __global__ __launch_bounds__(THREADS, TM == 128 || XP == 3 ? 2 : 3) void gemm_ex
                     o.w = pk(__builtin_fmaf(s, (float)((w1 >> 16) & 255u), b), __builtin_fmaf(s, (float)(w1 >> 24), b));
                     return o;
                 };
-                mcs[par * 256 + half * 128 + row] = ints(half ? hmc.z : hmc.x, half ? hmc.w : hmc.y, bias, -1.0f);
-                if constexpr (F::SC_OFFSET) scs[par * 256 + half * 128 + row] = ints(half ? hdr.z : hdr.x, half ? hdr.w : hdr.y, 0.0f, 4.0f);
-                wscale[par * 128 + row] = half_fast(hdd & 0xFFFFu) * (sp.bits == 3 ? 1.0f / 7.0f : 1.0f / 3.0f);
-                woff[par * 128 + row] = half_fast(hdd >> 16);
+                mcs[par * 256 + half * 128 + row] = ints(half ? hmc.z : hmc.x, half ? hmc.w : hmc.y, bias / kSumScale, -1.0f / kSumScale);
+                if constexpr (F::SC_OFFSET) scs[par * 256 + half * 128 + row] = ints(half ? hdr.z : hdr.x, half ? hdr.w : hdr.y, 0.0f, 4.0f / kSumScale);
+                wscale[par * 128 + row] = half_fast(hdd & 0xFFFFu) * (sp.bits == 3 ? 1.0f / 7.0f : 1.0f / 3.0f) * kSumScale;
+                woff[par * 128 + row] = half_fast(hdd >> 16) * kSumScale;
             }
         } else {
             float a, c;
