@@ -256,9 +256,11 @@ int tfq_gemm_ws(const tfq_weight_t* w, const void* x, int x_dtype, int M, void* 
 /* tfq_gemm_ws for callers that cannot allocate or bring a workspace: code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc.  The K-split scratch is a fixed array of
  * tfq_gemm_static_scratch_bytes() = 32 MiB in the library's device image (every GPU the library runs on holds
- * its copy until the process ends); the call itself allocates nothing.  A product whose split would use more
- * (tfq_gemm_workspace_bytes above that size) is refused with TFQ_ERR_SHAPE.  Same results as tfq_gemm_ws with
- * a workspace of tfq_gemm_workspace_bytes.  All calls on one GPU share the array: calls that overlap in time
+ * its copy until the process ends); the call itself allocates nothing.  Same results, bit for bit, as tfq_gemm_ws
+ * with a workspace of tfq_gemm_workspace_bytes.  Where that is more than the array holds, a product of the bf16 tile
+ * kernel (bf16 x on B32S4, B32S8, Q_G_4, Q_G_8, Q_8, Q_G_3) is refused with TFQ_ERR_SHAPE; one of the integer tile
+ * kernel (more than 16 rows: fp32 x on a tiled format, any x on Q_G_2, SB256A2, SB256A3, Q_4, Q_G_6) is served, its
+ * rows in several runs.  All calls on one GPU share the array: calls that overlap in time
  * on one GPU race (issue them on one stream).  The first call on a device resolves the array's address and
  * raises the kernel's LDS limit, which a capturing stream does not allow: make one call of the same shape
  * before a capture starts.  No counterpart in the reference: it is for callers that cannot allocate. */

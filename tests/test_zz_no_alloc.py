@@ -54,3 +54,26 @@ def test_gemm_static_refuses_what_does_not_fit(O, tfq, gpu):
     torch.cuda.synchronize()
     assert bool((y == 3.0).all())
     W.close()
+
+
+@pytest.mark.parametrize("fmt,dtype,M,N,K,fits", [
+    ("Q_G_4", "f32", 333, 1024, 4096, True), ("SB256A3", "bf16", 100, 1000, 4096, True), ("Q_4", "bf16", 65, 512, 4096, True),
+    ("B32S4", "f32", 18, 1000, 4096, True), ("Q_G_4", "f32", 333, 14336, 4096, False), ("SB256A2", "bf16", 400, 10001, 5376, False)])
+def test_gemm_static_integer_operands(tfq, gpu, fmt, dtype, M, N, K, fits):
+    """The products of the integer tile kernel are served whatever their K split needs, with the sums of tfq_gemm_ws
+    and a workspace of tfq_gemm_workspace_bytes, bit for bit: past 32 MiB the rows go through in several runs."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(12)
+    W = tfq.Weight(fmt, N, K, tfq.encode(fmt, torch.randn(N * K, device=gpu, generator=g) * 0.02))
+    x = torch.randn(M, K, device=gpu, generator=g)
+    x = x.bfloat16() if dtype == "bf16" else x
+    lib, code = tfq.lib(), tfq.BF16 if dtype == "bf16" else tfq.F32
+    need = int(lib.tfq_gemm_workspace_bytes(W.handle, code, M))
+    assert need > 0 and (need <= 32 << 20) == fits, need
+    for out, oc in ((torch.float32, tfq.F32), (torch.bfloat16, tfq.BF16)):
+        y_ws = W.gemm(x, out_dtype=out, workspace=True)
+        y_st = torch.full((M, N), float("nan"), device=gpu, dtype=out)
+        rc = lib.tfq_gemm_static(W.handle, x.data_ptr(), code, M, y_st.data_ptr(), oc, C.c_void_p(torch.cuda.current_stream().cuda_stream))
+        assert rc == 0, lib.tfq_last_error().decode()
+        assert torch.equal(y_ws, y_st)
+    W.close()

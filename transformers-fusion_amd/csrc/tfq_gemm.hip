@@ -687,8 +687,11 @@ int launch_gemm_static(const tfq_weight* w, const void* x, int x_dtype, int M, v
         g_static_scratch_ptr[dev].store(p, std::memory_order_release);  // the same address whichever thread resolves it
         scratch = p;
     }
-    // (the integer tile kernel takes whatever scratch there is)
-    const size_t need = gemm_exact_serves(w, x_dtype, M) ? slice_split_bytes(w) : gemm_scratch_bytes(w, x_dtype, M);
+    const size_t need = gemm_scratch_bytes(w, x_dtype, M);
+    // The integer tile kernel's products are not refused: where their parts need more than there is, the rows go through
+    // in as many runs as the area holds, with the K split of the whole, so that every sum is the one tfq_gemm_ws forms.
+    if (need > kStaticScratchBytes && gemm_exact_serves(w, x_dtype, M) && exact_cheaper(w, x_dtype, M, ~(size_t)0, true))
+        return launch_gemm_exact(w, x, x_dtype, M, y, y_dtype, s, scratch, kStaticScratchBytes, true);
     if (need > kStaticScratchBytes)
         return fail(TFQ_ERR_SHAPE, "tfq_gemm_static: this product would use " + std::to_string(need) +
                                        " bytes of scratch memory, the static area holds " + std::to_string(kStaticScratchBytes) +

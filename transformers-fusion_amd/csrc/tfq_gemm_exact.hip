@@ -722,6 +722,23 @@ int run_exact(const ExactArgs& a, int tm, hipStream_t s) {
     else return tm == 64 ? run_exact_tm<FMT, XP, 64>(a, s) : run_exact_tm<FMT, XP, 128>(a, s);
 }
 
+int run_exact_fmt(int fmt, const ExactArgs& a, bool f32, int tm, hipStream_t s) {
+    switch (canonical(fmt)) {
+        case TFQ_Q_G_4: return run_exact<TFQ_Q_G_4, 2>(a, tm, s);
+        case TFQ_Q_G_3: return run_exact<TFQ_Q_G_3, 2>(a, tm, s);
+        case TFQ_B32S4: return run_exact<TFQ_B32S4, 2>(a, tm, s);
+        case TFQ_B32S8: return run_exact<TFQ_B32S8, 2>(a, tm, s);
+        case TFQ_Q_G_8: return run_exact<TFQ_Q_G_8, 2>(a, tm, s);
+        case TFQ_Q_8: return run_exact<TFQ_Q_8, 2>(a, tm, s);
+        case TFQ_Q_G_2: return f32 ? run_exact<TFQ_Q_G_2, 2>(a, tm, s) : run_exact<TFQ_Q_G_2, 1>(a, tm, s);
+        case TFQ_SB256A3: return f32 ? run_exact<TFQ_SB256A3, 2>(a, tm, s) : run_exact<TFQ_SB256A3, 1>(a, tm, s);
+        case TFQ_SB256A2: return f32 ? run_exact<TFQ_SB256A2, 2>(a, tm, s) : run_exact<TFQ_SB256A2, 1>(a, tm, s);
+        case TFQ_Q_4: return f32 ? run_exact<TFQ_Q_4, 3>(a, tm, s) : run_exact<TFQ_Q_4, 1>(a, tm, s);
+        case TFQ_Q_G_6: return f32 ? run_exact<TFQ_Q_G_6, 3>(a, tm, s) : run_exact<TFQ_Q_G_6, 1>(a, tm, s);
+        default: return fail(TFQ_ERR_FORMAT, "gemm: no tile kernel for this format");
+    }
+}
+
 int planes_of(const tfq_weight* w, int x_dtype) {
     const bool wire = w->layout == TFQ_LAYOUT_WIRE;
     return (x_dtype == TFQ_BF16 ? 1 : wire ? 3 : 2) * (wire ? 2 : 1);
@@ -758,35 +775,35 @@ double gemm_exact_us(const tfq_weight* w, int x_dtype, int M, size_t scratch_byt
     return fit * plan_exact(w->N, w->K, M, planes_of(w, x_dtype), scratch_bytes).us;
 }
 
+// keep_split: the K split is the one that a scratch of any size would give; where its partial tiles need more than there
+// is, the rows go through in runs of whole tiles (a split has at most two rounds of workgroups, so 32 MiB hold the parts
+// of 42 rows or more; a row's sums do not depend on the tile it is in).
 int launch_gemm_exact(const tfq_weight* w, const void* x, int x_dtype, int M, void* y, int y_dtype, hipStream_t s, void* scratch,
-                      size_t scratch_bytes) {
-    ExactArgs a{};
-    a.W = w->dev;
-    a.X = x;
-    a.Y = y;
-    a.M = M;
-    a.N = (int)w->N;
-    a.K = (int)w->K;
-    a.y_bf16 = y_dtype == TFQ_BF16;
-    a.tiles_n = (int)((w->N + TN - 1) / TN);
-    const ExactPlan p = plan_exact(w->N, w->K, M, planes_of(w, x_dtype), scratch ? scratch_bytes : 0);
-    a.ksplit = p.ksplit;
-    a.partial = reinterpret_cast<float*>(scratch);
-    const bool f32 = x_dtype == TFQ_F32;
-    switch (canonical(w->fmt)) {
-        case TFQ_Q_G_4: return run_exact<TFQ_Q_G_4, 2>(a, p.tm, s);
-        case TFQ_Q_G_3: return run_exact<TFQ_Q_G_3, 2>(a, p.tm, s);
-        case TFQ_B32S4: return run_exact<TFQ_B32S4, 2>(a, p.tm, s);
-        case TFQ_B32S8: return run_exact<TFQ_B32S8, 2>(a, p.tm, s);
-        case TFQ_Q_G_8: return run_exact<TFQ_Q_G_8, 2>(a, p.tm, s);
-        case TFQ_Q_8: return run_exact<TFQ_Q_8, 2>(a, p.tm, s);
-        case TFQ_Q_G_2: return f32 ? run_exact<TFQ_Q_G_2, 2>(a, p.tm, s) : run_exact<TFQ_Q_G_2, 1>(a, p.tm, s);
-        case TFQ_SB256A3: return f32 ? run_exact<TFQ_SB256A3, 2>(a, p.tm, s) : run_exact<TFQ_SB256A3, 1>(a, p.tm, s);
-        case TFQ_SB256A2: return f32 ? run_exact<TFQ_SB256A2, 2>(a, p.tm, s) : run_exact<TFQ_SB256A2, 1>(a, p.tm, s);
-        case TFQ_Q_4: return f32 ? run_exact<TFQ_Q_4, 3>(a, p.tm, s) : run_exact<TFQ_Q_4, 1>(a, p.tm, s);
-        case TFQ_Q_G_6: return f32 ? run_exact<TFQ_Q_G_6, 3>(a, p.tm, s) : run_exact<TFQ_Q_G_6, 1>(a, p.tm, s);
-        default: return fail(TFQ_ERR_FORMAT, "gemm: no tile kernel for this format");
+                      size_t scratch_bytes, bool keep_split) {
+    const size_t have = scratch ? scratch_bytes : 0;
+    const ExactPlan p = plan_exact(w->N, w->K, M, planes_of(w, x_dtype), keep_split ? ~(size_t)0 : have);
+    int rows = M;
+    if (keep_split && p.ksplit > 1) {
+        const size_t fit = have / ((size_t)p.ksplit * (size_t)w->N * 4);
+        if (fit < (size_t)M) rows = (int)(fit < (size_t)p.tm ? fit : fit / p.tm * p.tm);
+        if (rows < 1) return fail(TFQ_ERR_SHAPE, "gemm: no scratch for the K split");
     }
+    const size_t xe = x_dtype == TFQ_F32 ? 4 : 2, ye = y_dtype == TFQ_F32 ? 4 : 2;
+    for (int m0 = 0; m0 < M; m0 += rows) {
+        ExactArgs a{};
+        a.W = w->dev;
+        a.X = static_cast<const uint8_t*>(x) + (size_t)m0 * (size_t)w->K * xe;
+        a.Y = static_cast<uint8_t*>(y) + (size_t)m0 * (size_t)w->N * ye;
+        a.M = std::min(rows, M - m0);
+        a.N = (int)w->N;
+        a.K = (int)w->K;
+        a.y_bf16 = y_dtype == TFQ_BF16;
+        a.tiles_n = (int)((w->N + TN - 1) / TN);
+        a.ksplit = p.ksplit;
+        a.partial = reinterpret_cast<float*>(scratch);
+        if (int rc = run_exact_fmt(w->fmt, a, x_dtype == TFQ_F32, p.tm, s)) return rc;
+    }
+    return TFQ_OK;
 }
 
 }  // namespace tfq

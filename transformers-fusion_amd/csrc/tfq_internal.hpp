@@ -496,7 +496,7 @@ bool gemm_exact_serves(const tfq_weight* w, int x_dtype, int M);
 size_t gemm_exact_scratch_bytes(const tfq_weight* w, int x_dtype, int M);
 double gemm_exact_us(const tfq_weight* w, int x_dtype, int M, size_t scratch_bytes);
 int launch_gemm_exact(const tfq_weight* w, const void* x, int x_dtype, int M, void* y, int y_dtype, hipStream_t s, void* scratch,
-                      size_t scratch_bytes);
+                      size_t scratch_bytes, bool keep_split = false);
 // Grouped form of the prefill tile kernel: several products over matrices of one format and one N x K, each with
 // its own bf16 X, its own Y and row count, in one grid (the experts of a mixture layer at prefill sizes).  Entry
 // table and workgroup map are built on the host (fill_gemm_group) and copied to the device by the caller.
