@@ -262,8 +262,9 @@ int tfq_gemm_ws(const tfq_weight_t* w, const void* x, int x_dtype, int M, void* 
  * kernel (more than 16 rows: fp32 x on a tiled format, any x on Q_G_2, SB256A2, SB256A3, Q_4, Q_G_6) is served, its
  * rows in several runs.  All calls on one GPU share the array: calls that overlap in time
  * on one GPU race (issue them on one stream).  The first call on a device resolves the array's address and
- * raises the kernel's LDS limit, which a capturing stream does not allow: make one call of the same shape
- * before a capture starts.  No counterpart in the reference: it is for callers that cannot allocate. */
+ * raises the kernel's LDS limit.  ROCm 7.2 accepts both while a stream is being captured; where a runtime does
+ * not, make one call of the same shape before a capture starts (the same holds for the first use of the other
+ * kernels of a tiled format; those of the wire formats raise no limit).  No counterpart in the reference: it is for callers that cannot allocate. */
 int tfq_gemm_static(const tfq_weight_t* w, const void* x, int x_dtype, int M, void* y, int y_dtype,
                     tfq_stream_t stream);
 size_t tfq_gemm_static_scratch_bytes(void);

@@ -210,3 +210,35 @@ def test_gemm_rows_in_slices_or_tiles(tfq, gpu, fmt, dtype, M, N, K, workspace, 
     for v in (y, rows):
         assert float((v.double() - want).norm() / want.norm()) <= 1e-5  # 16 bits of an fp32 activation, as above
     W.close()
+
+
+COLD_CAPTURE = """
+import importlib, sys
+import torch
+tfq = importlib.import_module("transformers-fusion_amd")
+tfq.init(0)
+for fmt, dtype, M in (("Q_4", "bf16", 20), ("Q_G_6", "f32", 40), ("Q_4", "f32", 300), ("Q_G_4", "f32", 200), ("SB256A3", "f32", 300), ("SB256A3", "bf16", 40)):
+    W = tfq.Weight(fmt, 1024, 1024, tfq.encode(fmt, torch.randn(1024 * 1024, device="cuda") * 0.02))
+    x = torch.randn(M, 1024, device="cuda").to(torch.bfloat16 if dtype == "bf16" else torch.float32)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = W.gemm(x)
+    for r in range(3):
+        y.zero_()
+        graph.replay()
+        x2 = x + 0  # the program's own work between the replays
+        torch.cuda.synchronize()
+        assert torch.equal(y, W.gemm(x2)), (fmt, dtype, M, r)
+print("captured")
+"""
+
+
+def test_first_call_inside_a_capture(gpu):
+    """The first prefill call of a process may be one that is being captured, for each kernel of the integer tile route."""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", COLD_CAPTURE], cwd=root, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "captured" in r.stdout, r.stderr[-2000:]

@@ -368,7 +368,7 @@ int run_tiles(GemmArgs a, hipStream_t s) {
     constexpr size_t lds = (size_t)(4 * BM * 8 + 2 * (BN > 128 ? 256 : 128) * 4) * 16;  // 160 KB or 144 KB
     using Kernel = void (*)(GemmArgs);
     const Kernel kern = pp ? gemm4_kernel<FMT, BN, NT, true> : gemm4_kernel<FMT, BN, NT, false>;
-    static std::atomic<bool> lds_limit_raised[2] = {};  // once: not allowed while a stream is being captured
+    static std::atomic<bool> lds_limit_raised[2] = {};  // once, not per launch: a runtime may refuse the call during a capture
     if (!lds_limit_raised[pp]) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute");

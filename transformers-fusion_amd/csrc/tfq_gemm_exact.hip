@@ -700,11 +700,13 @@ ExactPlan plan_exact(int64_t N, int64_t K, int M, int planes, size_t scratch_byt
 template <int FMT, int XP, int TM>
 int run_exact_tm(ExactArgs a, hipStream_t s) {
     constexpr size_t lds = (size_t)lds_uint4s<FMT, XP, TM>() * 16;
-    static std::atomic<bool> lds_limit_raised = false;  // once: not allowed while a stream is being captured
-    if (!lds_limit_raised) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_exact_kernel<FMT, XP, TM>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute");
-        lds_limit_raised = true;
+    if constexpr (lds > 64 * 1024) {  // (two fp32 parts of 128 rows beside the byte headers' offsets: 70 or 78 KB)
+        static std::atomic<bool> lds_limit_raised = false;  // once per kernel, as for the other tile kernel
+        if (!lds_limit_raised) {
+            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_exact_kernel<FMT, XP, TM>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute");
+            lds_limit_raised = true;
+        }
     }
     a.tiles_m = (a.M + TM - 1) / TM;
     const long items = (long)a.tiles_m * a.tiles_n * a.ksplit;

@@ -1519,8 +1519,8 @@ int run_gemv4(GemvArgs a, const void* x, hipStream_t s) {
             slot = wd == 2 ? 21 : 20;
         }
     }
-    // Raise the dynamic-LDS limit once per kernel (not per launch: the call is
-    // not allowed while a stream is being captured into a graph).
+    // Raise the dynamic-LDS limit once per kernel, not per launch: a runtime may
+    // refuse the call while a stream is being captured into a graph.
     static std::atomic<bool> lds_limit_raised[22] = {};
     if (!lds_limit_raised[slot]) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
