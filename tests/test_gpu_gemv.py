@@ -744,3 +744,37 @@ def test_gemv_sixteen_weight_runs(O, tfq, gpu, fmt, N, K, dtype):
     assert torch.equal(y[torch.isinf(y)], want[torch.isinf(want)])
     assert torch.allclose(y[2:], want[2:], rtol=1e-5, atol=0, equal_nan=True)
     W.close()
+
+
+def test_multi_calls_refuse_what_the_c_call_refuses(O, tfq, gpu):
+    """Counts of matrices and outputs that do not fit: the C call's error, or an IndexError where an output has no matrix."""
+    import torch
+    N, K = 32, 512
+    W = tfq.Weight("B32S4", N, K, O.encode_tensor("B32S4", O.rng_normal(5, N * K, 0.02)))
+    x = torch.zeros(1, K, device=gpu)
+    ys = [torch.zeros(1, N, device=gpu) for _ in range(5)]
+    for call in (tfq.gemv_multi, tfq.gemv_multi_fused):
+        with pytest.raises(tfq.TfqError):
+            call([W] * 5, x, ys)  # four matrices at most
+        with pytest.raises(tfq.TfqError):
+            call([W] * 3, x, ys[:2])  # an output is missing
+        with pytest.raises(IndexError):
+            call([W] * 2, x, ys[:3])
+        with pytest.raises(IndexError):
+            call([], x, ys[:1])
+        with pytest.raises(IndexError):
+            call([W], x, [])
+        call([W] * 4, x, ys[:4])
+    with pytest.raises(IndexError):
+        tfq.gemv_multi_fused([W], x, ys[:1], pair_swiglu=True)
+    tfq.gemv_multi_fused([W] * 2, x, ys[:1], pair_swiglu=True)
+    idx, wts = [[0, 1]], [[0.5, 0.5]]
+    xs = torch.zeros(1, K, device=gpu)
+    S = tfq.Weight("B32S4", K, K, O.encode_tensor("B32S4", O.rng_normal(6, K * K, 0.02)))
+    with pytest.raises(tfq.TfqError):
+        tfq.moe_ffn([S] * 2, [S], [S] * 2, idx, wts, xs)
+    with pytest.raises(IndexError):
+        tfq.moe_ffn([S] * 2, [S] * 3, [S] * 2, idx, wts, xs)
+    tfq.moe_ffn([S] * 2, [S] * 2, [S] * 2, idx, wts, xs)
+    W.close()
+    S.close()

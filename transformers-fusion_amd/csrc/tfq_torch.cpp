@@ -78,6 +78,11 @@ double number(PyObject* o) {
     if (v == -1.0 && PyErr_Occurred()) throw PyFail{};
     return v;
 }
+bool truth(PyObject* o) {
+    const int v = PyObject_IsTrue(o);
+    if (v < 0) throw PyFail{};
+    return v != 0;
+}
 const tfq_weight_t* weight_of(PyObject* w) {
     PyObject* h = PyObject_GetAttr(w, g_handle_name);
     if (!h) throw PyFail{};
@@ -146,7 +151,7 @@ PyObject* gemm(PyObject* const* a, Py_ssize_t n) {
     const int M = (int)(x.numel() / K), xd = dtype_code(x);
     at::Tensor y = empty({M, N}, dtype_or(a[4], at::kFloat), x);
     const int yd = dtype_code(y);
-    const size_t need = PyObject_IsTrue(a[5]) ? tfq_gemm_workspace_bytes(w, xd, M) : 0;
+    const size_t need = truth(a[5]) ? tfq_gemm_workspace_bytes(w, xd, M) : 0;
     if (need == 0) {
         const tfq_stream_t s = stream();
         call([&] { return tfq_gemm(w, x.data_ptr(), xd, M, y.data_ptr(), yd, s); });
@@ -159,25 +164,23 @@ PyObject* gemm(PyObject* const* a, Py_ssize_t n) {
 }
 
 struct Outs {
-    void* p[4];
-    int n, dtype;
+    std::vector<void*> p;  // one per matrix; null where there are fewer outputs
+    int dtype = 0;
 };
-Outs outs_of(PyObject* seq, size_t count_w) {
+// What the matrices' count allows is the C call's to say (TfqError), as is a missing output; outputs without a matrix
+// are an IndexError, as for a fixed-size array.
+Outs outs_of(PyObject* seq, size_t matrices, bool repeat_single = false) {
     PyObject* f = PySequence_Fast(seq, "expected a sequence of tensors");
     if (!f) throw PyFail{};
-    Outs o{};
-    o.n = (int)PySequence_Fast_GET_SIZE(f);
-    const char* bad = o.n < 1 || o.n > 4 || count_w > 4 ? "one to four matrices and outputs" : nullptr;
-    if (!bad)
-        for (int i = 0; i < o.n; ++i) {
-            PyObject* t = PySequence_Fast_GET_ITEM(f, i);
-            if (!THPVariable_Check(t)) { bad = "expected torch.Tensor outputs"; break; }
-            o.p[i] = THPVariable_Unpack(t).data_ptr();
-        }
-    PyObject* first = bad ? nullptr : PySequence_Fast_GET_ITEM(f, 0);
+    Outs o;
     try {
-        if (bad) raise(PyExc_ValueError, bad);
-        o.dtype = dtype_code(THPVariable_Unpack(first));
+        const Py_ssize_t n = PySequence_Fast_GET_SIZE(f);
+        o.p.reserve(4);
+        for (Py_ssize_t i = 0; i < n; ++i) o.p.push_back(tensor(PySequence_Fast_GET_ITEM(f, i)).data_ptr());
+        if (repeat_single && n == 1) o.p.push_back(o.p[0]);
+        if (o.p.empty() || o.p.size() > matrices) raise(PyExc_IndexError, "no matrices or outputs, or more outputs than matrices");
+        o.p.resize(matrices, nullptr);
+        o.dtype = dtype_code(THPVariable_Unpack(PySequence_Fast_GET_ITEM(f, 0)));
     } catch (...) {
         Py_DECREF(f);
         throw;
@@ -192,12 +195,11 @@ PyObject* gemv_multi(PyObject* const* a, Py_ssize_t n) {
     const auto ws = weights_of(a[0]);
     const at::Tensor& x = tensor(a[1]);
     const Outs o = outs_of(a[2], ws.size());
-    if (ws.empty() || (size_t)o.n != ws.size()) raise(PyExc_ValueError, "as many outputs as matrices");
     int64_t K = 0;
     tfq_weight_info(ws[0], nullptr, nullptr, &K, nullptr);
     const int B = K ? (int)(x.numel() / K) : 0, xd = dtype_code(x);
     const tfq_stream_t s = stream();
-    call([&] { return tfq_gemv_multi(ws.data(), (int)ws.size(), x.data_ptr(), xd, B, o.p, o.dtype, s); });
+    call([&] { return tfq_gemv_multi(ws.data(), (int)ws.size(), x.data_ptr(), xd, B, o.p.data(), o.dtype, s); });
     Py_INCREF(a[2]);
     return a[2];
 }
@@ -208,22 +210,18 @@ PyObject* gemv_multi_fused(PyObject* const* a, Py_ssize_t n) {
     const auto ws = weights_of(a[0]);
     const at::Tensor& x = tensor(a[1]);
     require(x.is_contiguous() && x.dim() > 0, "x must be contiguous");
-    Outs o = outs_of(a[2], ws.size());
     tfq_prologue_t pro{};
-    pro.accumulate = PyObject_IsTrue(a[8]);
-    pro.pair_swiglu = PyObject_IsTrue(a[9]);
-    if (pro.pair_swiglu && o.n == 1) {  // the second output is not written; the C call still wants two pointers
-        o.p[1] = o.p[0];
-        o.n = 2;
-    }
-    if (ws.empty() || (size_t)o.n < ws.size()) raise(PyExc_ValueError, "as many outputs as matrices");
+    pro.accumulate = truth(a[8]);
+    pro.pair_swiglu = truth(a[9]);
+    // (the second output of a pair is not written; the C call still wants two pointers)
+    const Outs o = outs_of(a[2], ws.size(), pro.pair_swiglu);
     if (a[3] != Py_None) {
         const at::Tensor& g = tensor(a[3]);
         require(g.scalar_type() == at::kFloat, "rmsnorm must be float32");
         pro.op = TFQ_PRO_RMSNORM;
         pro.gamma = static_cast<const float*>(g.data_ptr());
         pro.eps = (float)number(a[5]);
-        pro.gamma_plus_one = PyObject_IsTrue(a[6]);
+        pro.gamma_plus_one = truth(a[6]);
     } else if (a[4] != Py_None) {
         const at::Tensor& up = tensor(a[4]);
         require(up.scalar_type() == at::kFloat && up.sizes() == x.sizes() && up.is_contiguous(), "swiglu_up must be a contiguous float32 tensor of x's shape");
@@ -233,7 +231,7 @@ PyObject* gemv_multi_fused(PyObject* const* a, Py_ssize_t n) {
     }
     const int B = (int)x.size(0), xd = dtype_code(x);
     const tfq_stream_t s = stream();
-    call([&] { return tfq_gemv_multi_fused(ws.data(), (int)ws.size(), x.data_ptr(), xd, B, o.p, o.dtype, &pro, s); });
+    call([&] { return tfq_gemv_multi_fused(ws.data(), (int)ws.size(), x.data_ptr(), xd, B, o.p.data(), o.dtype, &pro, s); });
     Py_INCREF(a[2]);
     return a[2];
 }
@@ -294,11 +292,14 @@ struct Buffer {  // a C-contiguous host array
 // gate, up, down, idx (int64 array [T][k]), weights (float32 array [T][k]), T, k, x, out_dtype, mid_dtype
 PyObject* moe_ffn(PyObject* const* a, Py_ssize_t n) {
     count(n, 10);
-    const auto g = weights_of(a[0]), u = weights_of(a[1]), d = weights_of(a[2]);
-    if (g.empty() || u.size() != g.size() || d.size() != g.size()) raise(PyExc_ValueError, "as many up and down matrices as gate matrices");
+    const auto g = weights_of(a[0]);
+    auto u = weights_of(a[1]), d = weights_of(a[2]);
+    if (g.empty() || u.size() > g.size() || d.size() > g.size()) raise(PyExc_IndexError, "no experts, or more up or down matrices than gate matrices");
+    u.resize(g.size(), nullptr);  // a missing one is the C call's to refuse
+    d.resize(g.size(), nullptr);
     const int T = (int)integer(a[5]), k = (int)integer(a[6]);
     const Buffer idx(a[3]), wts(a[4]);
-    require(idx.b.len == (Py_ssize_t)T * k * 8 && wts.b.len == (Py_ssize_t)T * k * 4, "routing arrays of int64 and float32 [T][k]");
+    require(idx.b.len >= (Py_ssize_t)T * k * 8 && wts.b.len >= (Py_ssize_t)T * k * 4, "routing arrays of int64 and float32 [T][k]");
     int64_t F = 0, D = 0;
     tfq_weight_info(g[0], nullptr, &F, &D, nullptr);
     const at::Tensor x = tensor(a[7]).contiguous();
