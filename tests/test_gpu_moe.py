@@ -484,6 +484,27 @@ def test_mlp_step_matches_the_oracle(O, tfq, gpu, fmt, B, xdt, mid):
         W.close()
 
 
+@pytest.mark.parametrize("fmt", ["B32S4", "Q_G_8", "Q_G_3", "SB256A3", "Q_G_6"])
+@pytest.mark.parametrize("B", [2, 3, 8, 9, 16, 17])
+def test_mlp_step_fp32_rows_match_the_oracle(O, tfq, gpu, fmt, B):
+    """The same with fp32 activations throughout, at the row counts where the launches change: the paired launch up to
+    two, the SwiGLU prologue up to sixteen, the prefill entry above.  Three products of 16-bit activations are within
+    3 x 2^-17 of a value, the companded grid's line within 7.5e-5 of its levels (on the norm; SiLU's slope is below 1.1)."""
+    import torch
+    D, F = 512, 768
+    print(f"mlp_step {fmt} B={B} f32", flush=True)
+    pays = [O.encode_tensor(fmt, O.rng_normal(70 + i, n * k, 0.02)) for i, (n, k) in enumerate(((F, D), (F, D), (D, F)))]
+    x = O.rng_normal(9, B * D, 1.0).reshape(B, D)
+    g = O.matmul(fmt, pays[0], F, D, x)
+    u = O.matmul(fmt, pays[1], F, D, x)
+    want = O.matmul(fmt, pays[2], D, F, O.silu_mul(g.reshape(-1), u.reshape(-1)).reshape(B, F)).astype(np.float64)
+    Ws = [tfq.Weight(fmt, n, k, p) for p, (n, k) in zip(pays, ((F, D), (F, D), (D, F)))]
+    y = tfq.mlp_step(Ws[0], Ws[1], Ws[2], torch.from_numpy(x).to(gpu)).cpu().numpy()
+    assert np.linalg.norm(y - want) <= (3e-4 if fmt == "Q_G_8" else 3e-5) * np.linalg.norm(want)
+    for W in Ws:
+        W.close()
+
+
 def test_capacity_dispatch_matches_oracle(O, tfq, gpu):
     """moe_engine::plan_dispatch / gather / combine (engines/trainer/moe/dispatch.cpp:9-78) through the C ABI."""
     import torch

@@ -579,7 +579,7 @@ int moe_run(const tfq_weight* const* gate, const tfq_weight* const* up, const tf
     }
     for (int e = 0; e < E && !grouped && !tall_grouped; ++e) {
         const int p0 = first[e], nt = first[e + 1] - first[e];
-        if (nt > 16) {  // the prefill entry: matrix cores for bf16 rows, 16-row slices otherwise
+        if (nt > 16) {  // the prefill entry: a tile kernel, or 16-row slices where those are faster
             if (int rc = launch_gemm(gate[e], ws.xe + (size_t)p0 * D * xe_bytes, x_dtype, nt, ws.g + (size_t)p0 * F, TFQ_F32, s, ws.scratch, ws.scratch_bytes)) return rc;
             if (int rc = launch_gemm(up[e], ws.xe + (size_t)p0 * D * xe_bytes, x_dtype, nt, ws.u + (size_t)p0 * F, TFQ_F32, s, ws.scratch, ws.scratch_bytes)) return rc;
             continue;
@@ -1008,7 +1008,8 @@ int launch_mlp_step(const tfq_weight* gate, const tfq_weight* up, const tfq_weig
     if (B <= 16 && gemv_prologue_supported(down) && (B <= 2 || mid_dtype == TFQ_F32)) {
         // silu(gate) * up happens while the down kernel stages its activations.  The prologue reads fp32 rows, two
         // per pass over the matrix: with bf16 mid activations and more rows the elementwise kernel below and one
-        // pass of the sixteen-row kernel are cheaper (fp32 mid activations take two rows per pass either way)
+        // pass of the sixteen-row kernel are cheaper.  fp32 mid activations take the prologue at every row count, so
+        // three rows read the down matrix twice and sixteen read it eight times.
         tfq_prologue_t pro{};
         pro.op = TFQ_PRO_SWIGLU;
         pro.up = u;

@@ -4,7 +4,7 @@
 // Why: a decode-sized product runs 3 to 15 us on the GPU, and the same steps through ctypes and the tensors' Python
 // attributes took longer, so the host, not the kernel, set the rate of a loop of such calls.  Host time per call, ctypes
 // and here: gemv 10.7 and 4.2 us (1024 x 4096, one bf16 row), with a workspace 12.3 and 5.1, one fused product 9.0 and
-// 3.2, router and routed mixture (two calls, six to eight launches) 40 and 25; the launch itself is about 2 us of each.
+// 3.2, router and routed mixture (two calls, five launches) 40 and 25; the launch itself is about 2 us of each.
 //
 // The C calls run without the GIL, as they do under ctypes.  Nothing is kept between calls.
 #include <Python.h>
