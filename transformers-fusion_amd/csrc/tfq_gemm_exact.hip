@@ -25,15 +25,15 @@
 // A workgroup of four wavefronts owns 128 tokens x 128 weight rows and walks K in steps of 32, both operands staged
 // in LDS (two buffers, one barrier per step); a wavefront multiplies 64 x 64.  What bounds it is vector issue next
 // to the MFMAs (splitting activations, decoding codes, the scale's multiply-adds; counted on 333 fp32 rows of Q_G_4
-// 4096 x 14336: 260 vector instructions and 38 MFMAs per wavefront and step, vector issue busy for 66 % of the cycles,
-// the matrix cores for 34 %, LDS for 44 %), so two workgroups share a compute unit (LDS <= 80 KB, <= 256 registers):
-// one's staging runs under the other's MFMAs.  256-row tiles with one workgroup per unit would stage less per product,
+// 4096 x 14336: 245 vector instructions, 38 of them MFMAs, per wavefront and step, vector issue busy for 52 % of the
+// cycles, the matrix cores for 33 %, LDS for 34 %; SB256A3 with bf16 rows 123 / 26, 39, 33 and 38 %), so two workgroups
+// share a compute unit (LDS <= 80 KB, <= 256 registers): one's staging runs under the other's MFMAs.  256-row tiles with one workgroup per unit would stage less per product,
 // but a ragged prompt (333 rows) then pads to 512 rows instead of 384.  Activations are fetched two steps ahead, codes
 // three.  Few rows take 64-row tiles, three workgroups per unit.
 // Measured, before (slices of 4 to 16 rows through the decode kernels) and now: Q_G_4 fp32 333 rows 4096 x 14336
-// 657 -> 171 us, B32S8 the same 700 -> 133 us; 512 bf16 rows of 14336 x 4096: Q_4 7580 -> 197 us, Q_G_6 5360 -> 184 us,
-// SB256A3 789 -> 135 us.  Up to 16 rows tfq_gemv's kernels serve every format, above that the
-// faster of the two by a model (exact_cheaper).  For the wire formats the step at 17 rows is where the entry points part,
+// 657 -> 146 us, B32S8 the same 700 -> 133 us; 512 bf16 rows of 14336 x 4096: Q_4 7580 -> 189 us, Q_G_6 5360 -> 184 us,
+// SB256A3 789 -> 141 us.  Up to 16 rows tfq_gemv's kernels serve every format, above that the faster of the two
+// by a model (exact_cheaper).  For the wire formats the step at 17 rows is where the entry points part,
 // not where the kernels cross: 14336 x 4096 bf16 Q_4 takes 93 us at 16 rows (four passes) and 40 us at 17 to 24 rows here,
 // Q_G_6 90 and 45 us; at 1024 x 4096 the two meet (16 us).  The Tiled16 formats cross between 16 and 20 rows.
 
