@@ -311,10 +311,11 @@ int tfq_matmul_host(const tfq_weight_t* w, const float* X, float* Y, int B);
  * Qwen35Engine::mlp_step (src/adapters/tools/qwen35_engine.cpp:662-672) for B rows:
  *   y[b] = down( silu(gate x[b]) * (up x[b]) ),  silu(v) = v / (1 + exp(-v))
  * (src/math/math.cpp:117-126).  gate and up are F x D matrices of one format, down is D x F;
- * x is [B][D], y is [B][D], device pointers.  Up to 16 rows and a format with a tiled kernel: two
- * launches: gate and up in one whose epilogue writes silu(gate x) * (up x) (up to four bf16 / two fp32 rows,
- * formats B32S4, B32S8, Q_G_4, Q_G_8) or, failing that, down with the elementwise step applied while it stages
- * its activations; otherwise gate / up, the elementwise step and down are launches of their own.
+ * x is [B][D], y is [B][D], device pointers.  Up to four bf16 / two fp32 rows in a format with the paired kernel
+ * (B32S4, B32S8, Q_G_4, Q_G_8) are two launches: gate and up in one whose epilogue writes silu(gate x) * (up x),
+ * and down.  Otherwise, up to 16 rows in a tiled format, gate and up share a launch and, with fp32 mid activations
+ * or at most two rows, down applies the elementwise step while it stages its activations, two rows per launch;
+ * in all other cases gate / up, the elementwise step and down are launches of their own.
  * mid_dtype is the type the SwiGLU product is rounded to before
  * the down projection: TFQ_F32 keeps it in fp32 like the reference, TFQ_BF16 feeds the matrix
  * cores.  workspace is device memory of at least tfq_mlp_workspace_bytes(B, F) bytes, 256-byte

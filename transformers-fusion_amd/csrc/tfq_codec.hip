@@ -1,8 +1,10 @@
 // Block codec on the device: bit-exact decode of every supported wire format
 // (per-weight arithmetic in tfq_decode.hpp), the closed-form encoders, the wire ->
-// Tiled16 layout conversion and the decode from that layout.  Decode and encode use one workgroup of
-// 256 lanes per 256-weight block, one lane per weight; the payload of a block is
-// at most 1 KB, so these kernels are bound by the fp32 side (4 B per weight).
+// Tiled16 layout conversion and the decode from that layout, the iterative encoders.  Decode: a wavefront takes
+// four blocks, a lane four weights of each.  The closed-form encoders of the benchmark formats are laid out the same
+// way, the others have a workgroup per block; the iterative ones give a scale group (or a run of weights with one
+// scale) to a lane or a small team of lanes.  Decode and the closed forms are bound by the fp32 side (4 B per
+// weight), the iterative encoders by vector instructions.
 
 #include "tfq_decode.hpp"
 #include "tfq_encode_short.hpp"
@@ -284,7 +286,7 @@ __global__ __launch_bounds__(256) void encode_q1_kernel(const float* __restrict_
 // reference's value before the rounding by less than `2^-24 (128 + 4 |m top / s|)`, and remembers how close any weight
 // of the group came to a rounding boundary; where that is closer than the bound (4 % of the wavefronts and passes)
 // the lane repeats the pass with the reference's own arithmetic.  The payload is therefore the reference's in every
-// case.  58.7 M weights of Q_G_4: 7.46 ms with one block per wavefront and the division, 450 us.
+// case.  58.7 M weights of Q_G_4: 7.46 ms with one block per wavefront and the division, 360 to 400 us.
 __device__ __forceinline__ uint32_t unit_nearest_dev(float value, int bits) {
     const float v = fmaxf(0.0f, fminf(1.0f, value));
     const float top = bits == 1 ? 1.0f : bits == 4 ? 15.0f : bits == 3 ? 7.0f : bits == 6 ? 63.0f : bits == 8 ? 255.0f : 3.0f;
@@ -797,8 +799,7 @@ __global__ __launch_bounds__(64) void encode_grp12_kernel(const float* __restric
 }
 
 // Grouped-lattice fallback encoder (quant_grp16 with grp16_fit_scale, src/codec/block_codec.cpp:739-914) for
-// the ids that use that layout for full blocks, and the Q_G_6 encoder (quant_6k, :1070-1238).  Same shape as
-// the affine encoder: a wavefront per block, lane g owns group g (32 groups of 8, or 16 groups of 16), lane 0
+// the ids that use that layout for full blocks: a wavefront per block, lane g owns group g (32 groups of 8), lane 0
 // the sums over groups; fused operations where GCC's Release build fuses.
 template <int FMT>
 __global__ __launch_bounds__(64) void encode_grp16_kernel(const float* __restrict__ wg, uint8_t* __restrict__ dst) {
