@@ -746,6 +746,29 @@ def test_gemv_sixteen_weight_runs(O, tfq, gpu, fmt, N, K, dtype):
     W.close()
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("fmt,N,K,per_row", [("Q_4", 301, 256, (1, 2, 4)), ("Q_4", 64, 768, (1, 2, 4)), ("Q_4", 301, 1024, (4,)), ("Q_4", 301, 1280, ()),
+                                             ("Q_G_6", 301, 512, (1, 2, 4)), ("Q_G_6", 77, 1280, (1, 2, 4)), ("Q_G_6", 77, 1536, ()),
+                                             ("Q_G_6", 2050, 1536, (1, 2, 4)), ("Q_G_6", 2050, 1792, ())])
+def test_short_rows_of_the_wire_formats(O, tfq, gpu, fmt, N, K, per_row, dtype):
+    """Short rows, where the sixteen-weights-per-lane kernel would leave most of its lanes idle, take the wavefront-per-row
+    kernel: the bits of the mixed-format kernel, which has the same arithmetic.  Either way the float64 product with the
+    decoded matrix, to the rounding of fp32 sums and weights."""
+    import torch
+    pay = O.encode_tensor(fmt, O.rng_normal(21, N * K, 0.02))
+    W = tfq.Weight(fmt, N, K, pay)
+    M = tfq.Weight.mixed(N, K, [fmt] * (N * K // 256), pay)
+    dense = torch.from_numpy(O.decode_tensor(fmt, pay, N * K).reshape(N, K)).to(gpu).double()
+    for B in (1, 2, 4):
+        x = torch.from_numpy(O.rng_normal(22 + B, B * K, 1.0).reshape(B, K)).to(gpu)
+        x = x.bfloat16() if dtype == "bf16" else x
+        y, want = W.gemv(x), x.double() @ dense.T
+        assert float((y.double() - want).norm() / want.norm()) <= 1e-6
+        assert torch.equal(y, M.gemv(x)) == (B in per_row), B
+    W.close()
+    M.close()
+
+
 def test_multi_calls_refuse_what_the_c_call_refuses(O, tfq, gpu):
     """Counts of matrices and outputs that do not fit: the C call's error, or an IndexError where an output has no matrix."""
     import torch

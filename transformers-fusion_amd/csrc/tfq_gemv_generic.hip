@@ -273,10 +273,22 @@ __global__ __launch_bounds__(256) void gemv_run16_kernel(const uint8_t* __restri
     }
 }
 
+// A pass of gemv_run16_kernel covers sixteen blocks of K and takes its time also where the row has fewer; the
+// wavefront-per-row kernel's time is proportional to K.  They cross at three blocks for Q_4 (four with four rows), at
+// five for Q_G_6 (six on many rows).  Runs of sixteen against a wavefront per row, us: Q_G_6 14336 rows of 512 14.6 / 6.6
+// (sixteen bf16 activation rows 89 / 32), of 1280 14.0 / 10.3, of 2048 14.4 / 15.1; Q_4 of 512 11.8 / 8.5, of 768
+// 11.7 / 11.1, of 1024 11.8 / 12.9 (sixteen rows 86 / 71).
+template <int FMT, int BT>
+bool run16_pays(int N, int K) {
+    const int nblk = K >> 8;
+    return FMT == TFQ_Q_4 ? nblk > (BT == 4 ? 4 : 3) : nblk > (N >= 2048 ? 6 : 5);
+}
+
 template <int FMT, int BT>
 int run(const tfq_weight* w, const void* x, int xd, void* y, int yd, hipStream_t s) {
     const int N = (int)w->N, K = (int)w->K;
     if constexpr (kRun16<FMT>) {
+        if (run16_pays<FMT, BT>(N, K)) {
         // about a thousand workgroups (four per compute unit), each with the same number of row groups
         const int groups = (N + kRunRows - 1) / kRunRows, per = (groups + 1023) / 1024, grid = (groups + per - 1) / per;
         const bool one_pass = K <= 4096;
@@ -285,14 +297,14 @@ int run(const tfq_weight* w, const void* x, int xd, void* y, int yd, hipStream_t
                                           : (one_pass ? gemv_run16_kernel<FMT, BT, false, true> : gemv_run16_kernel<FMT, BT, false, false>);
         hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, s, w->dev, x, y, N, K, yd == TFQ_BF16);
         return hip_fail(hipGetLastError(), "gemv launch");
-    } else {
+        }
+    }
     const int grid = (N + 3) / 4 < 4096 ? (N + 3) / 4 : 4096;
     if (xd == TFQ_F32)
         hipLaunchKernelGGL((gemv_generic_kernel<FMT, BT, true>), dim3(grid), dim3(256), 0, s, w->dev, x, y, N, K, yd == TFQ_BF16);
     else
         hipLaunchKernelGGL((gemv_generic_kernel<FMT, BT, false>), dim3(grid), dim3(256), 0, s, w->dev, x, y, N, K, yd == TFQ_BF16);
     return hip_fail(hipGetLastError(), "gemv launch");
-    }
 }
 
 template <int FMT>
