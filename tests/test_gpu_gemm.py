@@ -146,6 +146,33 @@ def test_gemm_few_bf16_rows_integer_operands(O, tfq, gpu, fmt, M, N, K):
     W.close()
 
 
+@pytest.mark.parametrize("fmt,dtype,N,K,bound", [
+    ("B32S4", "f32", 2000, 4096, 3.0e-6), ("Q_G_4", "f32", 2000, 4096, 3.0e-6), ("Q_G_3", "f32", 2000, 4096, 3.0e-6), ("SB256A3", "f32", 2000, 4096, 3.0e-6),
+    ("Q_G_4", "bf16", 2000, 4096, 1.0e-6), ("Q_G_3", "bf16", 2000, 4096, 1.0e-6), ("Q_4", "f32", 1500, 14336, 1.3e-7), ("Q_G_6", "f32", 1500, 14336, 1.3e-7)])
+@pytest.mark.parametrize("mean", [0.0, 1.0])
+def test_gemm_integer_operands_error_with_a_mean(tfq, gpu, fmt, dtype, N, K, bound, mean):
+    """Activations N(0, 1) and 1 + 0.1 N(0, 1), 9 to 333 rows, against the float64 product.  Two bf16 parts of an fp32 value
+    leave out 2.5e-6 of it in the mean (uniform in the second part's half unit, 2^-17 of the value at most); a level times
+    its scale is rounded once in the decoded matrix, which a mean of the activations adds up over a group, 32 of them against
+    the 26 or so steps of the centred codes' sum: 9 times 2^-24, 0.5e-6 to 0.9e-6.  sqrt(2.5^2 + 0.9^2) = 2.7e-6, and 0.9e-6 without
+    the parts, and a tenth for the fp32 sums.  Three parts leave nothing out: fp32 sums of 14336 terms in blocks, 1.3e-7."""
+    import torch
+    print(f"gemm mean {fmt} {dtype} N={N} K={K} mean={mean}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(21)
+    W = tfq.Weight(fmt, N, K, tfq.encode(fmt, torch.randn(N * K, device=gpu, generator=g) * 0.02))
+    dense = W.decode().reshape(N, K).double()
+    for M in (9, 16, 17, 64, 333):
+        if dtype == "bf16" and M not in (17, 64):
+            continue  # (other kernels' rows, whose rounding is their own)
+        x = torch.randn(M, K, device=gpu, generator=g)
+        x = x * 0.1 + mean if mean else x
+        x = x.bfloat16() if dtype == "bf16" else x
+        want = x.double() @ dense.T
+        y = W.gemv(x) if M <= 16 else W.gemm(x, out_dtype=torch.float32)
+        assert float((y.double() - want).norm() / want.norm()) <= bound, M
+    W.close()
+
+
 @pytest.mark.parametrize("fmt,dtype", [("Q_G_4", "f32"), ("B32S8", "bf16"), ("B32S4", "f32"), ("SB256A3", "f32"), ("SB256A2", "bf16"),
                                        ("Q_4", "f32"), ("Q_4", "bf16"), ("Q_G_6", "bf16"), ("Q_G_8", "f32")])
 @pytest.mark.parametrize("M,N,K", [(40, 384, 2048), (300, 700, 1280), (257, 4100, 768)])
