@@ -232,6 +232,30 @@ def test_gemm_integer_operands_non_finite(O, tfq, gpu, fmt):
     W.close()
 
 
+@pytest.mark.parametrize("fmt", ["Q_G_4", "Q_G_3", "B32S4", "B32S8", "Q_G_8", "Q_8"])
+@pytest.mark.parametrize("M,N,K", [(64, 1000, 2048), (80, 16400, 512), (48, 4100, 4352)])
+def test_gemm_infinite_bf16_activations(tfq, gpu, fmt, M, N, K):
+    """An infinite bf16 activation gives the infinity (or, where the weight is zero, the NaN) of its fp32 product, whichever
+    tile kernel serves the rows: with K in parts and whole."""
+    import torch
+    print(f"gemm inf {fmt} M={M} N={N} K={K}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(31)
+    W = tfq.Weight(fmt, N, K, tfq.encode(fmt, torch.randn(N * K, device=gpu, generator=g) * 0.02))
+    x = torch.randn(M, K, device=gpu, generator=g).bfloat16()
+    x[2, 7] = float("inf")
+    x[3, 300] = -float("inf")
+    x[35, 11] = x[35, K - 1] = float("inf")
+    x[40, 100] = float("nan")
+    want = x.double() @ W.decode().reshape(N, K).double().T
+    for out in (torch.float32, torch.bfloat16):
+        y = W.gemm(x, out_dtype=out).double()
+        assert torch.equal(torch.isnan(y), torch.isnan(want)), (torch.isnan(y) != torch.isnan(want)).any(1).nonzero().flatten().tolist()
+        assert torch.equal(torch.isposinf(y), torch.isposinf(want)) and torch.equal(torch.isneginf(y), torch.isneginf(want))
+        f = torch.isfinite(want)
+        assert float((y[f] - want[f]).norm() / want[f].norm()) <= TOL
+    W.close()
+
+
 @pytest.mark.parametrize("fmt,dtype", [f for f in EXACT_FMTS if f[0] not in ("Q_4", "Q_G_6", "Q_4_K_H")])
 def test_gemm_tiled_operands_range(O, tfq, gpu, fmt, dtype):
     """Infinite, not-a-number, huge and tiny activations on the formats of the tiled layout: the same outputs are NaN as
