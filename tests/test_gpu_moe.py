@@ -78,8 +78,8 @@ def test_router_linear_then_route(O, tfq, gpu, xdt):
 @pytest.mark.parametrize("T,D,E,K,bias", [(1, 64, 1, 1, False), (3, 1023, 3, 2, True), (17, 1024, 16, 4, False), (5, 4097, 17, 8, True),
                                           (2, 2112, 130, 6, False), (2, 256, 1100, 3, True)])
 def test_router_in_one_launch(O, tfq, gpu, T, D, E, K, bias):
-    """The router Linear and the route of its logits over the edges of the one-launch kernel (rounds of sixteen experts, D off
-    its steps of 1024, more experts than it takes): logits against float64, and the route equal to tfq_moe_route's of those
+    """The router Linear and the route of its logits over the edges of both its forms (one and two launches, D off the
+    steps of 1024, more experts than a wavefront routes): logits against float64, and the route equal to tfq_moe_route's of those
     very logits."""
     import torch
     x = torch.from_numpy(O.rng_normal(48, T * D, 1.0).reshape(T, D)).to(gpu)
@@ -91,6 +91,25 @@ def test_router_in_one_launch(O, tfq, gpu, T, D, E, K, bias):
         assert float((logits.double() - ref).abs().max()) <= 1e-5 * float(ref.abs().max())
         p2, i2, w2 = tfq.moe_route(logits, K)
         assert torch.equal(probs, p2) and torch.equal(idx, i2) and torch.equal(w, w2)
+
+
+@pytest.mark.parametrize("E,T", [(12, 1), (13, 153), (13, 154), (24, 175), (24, 176), (64, 255), (64, 256), (65, 258)])
+def test_router_one_launch_or_two(tfq, gpu, E, T):
+    """Few experts, or many tokens, take the one-launch kernel and everything else two launches: on both sides of the line a
+    token's logits and route are, bit for bit, those of a call with that token alone (two launches from thirteen experts on),
+    and the route is tfq_moe_route's of the logits."""
+    import torch
+    D, K = 1088, 3
+    gen = torch.Generator().manual_seed(E * 1000 + T)
+    x = torch.randn(T, D, generator=gen).to(gpu)
+    Wr = (torch.randn(E, D, generator=gen) * 0.05).to(gpu)
+    got = tfq.moe_router(x, Wr, K)
+    ref = x.double() @ Wr.double().T
+    assert float((got[0].double() - ref).abs().max()) <= 1e-5 * float(ref.abs().max())
+    assert all(torch.equal(a, b) for a, b in zip(got[1:], tfq.moe_route(got[0], K)))
+    for t in (0, T // 2, T - 1):
+        alone = tfq.moe_router(x[t:t + 1].contiguous(), Wr, K)
+        assert all(torch.equal(a[t:t + 1], b) for a, b in zip(got, alone))
 
 
 def _experts(O, tfq, fmt, E, D, F, seed):

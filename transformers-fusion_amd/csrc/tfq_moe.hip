@@ -306,19 +306,20 @@ template <bool XBF16>
 __global__ __launch_bounds__(256) void router_logits_kernel(const void* __restrict__ xv, const float* __restrict__ Wr, const float* __restrict__ bias,
                                                             float* __restrict__ logits, int T, int E, int D) {
     const int lane = threadIdx.x & 63;
-    const long long pair = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (pair >= (long long)T * E) return;
-    const int t = (int)(pair / E), e = (int)(pair - (long long)t * E);
-    const float s = router_logit<XBF16>(xv, (size_t)t * D, Wr + (size_t)e * D, D, lane);
-    if (lane == 0) logits[pair] = bias ? s + bias[e] : s;
+    for (long long pair = (long long)blockIdx.x * 4 + (threadIdx.x >> 6); pair < (long long)T * E; pair += (long long)gridDim.x * 4) {
+        const int t = (int)(pair / E), e = (int)(pair - (long long)t * E);
+        const float s = router_logit<XBF16>(xv, (size_t)t * D, Wr + (size_t)e * D, D, lane);
+        if (lane == 0) logits[pair] = bias ? s + bias[e] : s;
+    }
 }
-// A token per workgroup: its logits, a wavefront per expert and round, then the route by the first wavefront.  As launches of
-// their own the route waited for the last logit of all tokens (16 tokens, 8 experts of 4096: 10.6 + 6.7 us, here 6.8).
+constexpr int kRouterMaxE = 64;
+// A token per workgroup: its logits, a wavefront per expert and round, then the route by the first wavefront.  A workgroup
+// reads the whole router matrix through one compute unit, sixteen experts of it at a time.
 template <bool XBF16>
 __global__ __launch_bounds__(1024) void router_kernel(const void* __restrict__ xv, const float* __restrict__ Wr, const float* __restrict__ bias,
                                                       float* __restrict__ logits, int E, int D, int k, float* __restrict__ probs,
                                                       int* __restrict__ idx, float* __restrict__ wts) {
-    __shared__ float s_l[kRouteMaxE], s_p[kRouteMaxE];
+    __shared__ float s_l[kRouterMaxE], s_p[kRouterMaxE];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const size_t t = blockIdx.x;
     for (int e = wave; e < E; e += (int)(blockDim.x >> 6)) {
@@ -331,17 +332,26 @@ __global__ __launch_bounds__(1024) void router_kernel(const void* __restrict__ x
 }
 }  // namespace
 
+// One launch for few experts, a round of wavefronts, and for more of them where the tokens fill the compute units several
+// workgroups deep; otherwise a launch of logits, a wavefront per (token, expert), and one of routes.  The same bits.  us a call,
+// one launch and two, D = 4096: 8 experts, 1 token 5.8 and 6.1, 16 tokens 6.3 and 6.9, 1024 tokens 11.6 and 13.7; 12
+// experts, 1 to 256 tokens 8.5 to 9.0 and 8.1 to 10.9; 16 experts, 1 token 7.8 and 6.5, 128 tokens 9.8 and 9.5, 160 tokens 9.8
+// and 10.5; 32 experts, 1 token 16.4 and 11.5, 192 tokens 13.8 and 13.4, 256 tokens 13.8 and 15.3; 64 experts, 1 token 24.5
+// and 12.2, 256 tokens 21.8 and 22.8; 256 experts, 1 token 75 and 17, 1024 tokens 243 and 243.  The line moves little with
+// D (1024 to 7168 measured).
+static bool router_in_one_launch(int T, int E) { return E <= 12 || (E <= kRouterMaxE && T >= 128 + 2 * E); }
+
 int launch_moe_router(const void* x, int x_dtype, const float* Wr, const float* bias, float* logits, int T, int E, int D, int k, float* probs,
                       int* idx, float* wts, hipStream_t s) {
-    if (E <= kRouteMaxE) {
+    if (router_in_one_launch(T, E)) {
         const dim3 block(64 * (E < 16 ? E : 16));
         if (x_dtype == TFQ_BF16) hipLaunchKernelGGL(router_kernel<true>, dim3(T), block, 0, s, x, Wr, bias, logits, E, D, k, probs, idx, wts);
         else hipLaunchKernelGGL(router_kernel<false>, dim3(T), block, 0, s, x, Wr, bias, logits, E, D, k, probs, idx, wts);
         return hip_fail(hipGetLastError(), "router launch");
     }
-    const long long pairs = (long long)T * E;
-    if ((pairs + 3) / 4 > 0x7FFFFFFF) return fail(TFQ_ERR_SHAPE, "router: too many (token, expert) pairs");
-    const dim3 grid((unsigned)((pairs + 3) / 4));
+    const long long quads = ((long long)T * E + 3) / 4;
+    if (E > kRouteMaxE && quads > 0x7FFFFFFF) return fail(TFQ_ERR_SHAPE, "router: too many (token, expert) pairs");
+    const dim3 grid((unsigned)std::min(quads, 1LL << 22));
     if (x_dtype == TFQ_BF16) hipLaunchKernelGGL(router_logits_kernel<true>, grid, dim3(256), 0, s, x, Wr, bias, logits, T, E, D);
     else hipLaunchKernelGGL(router_logits_kernel<false>, grid, dim3(256), 0, s, x, Wr, bias, logits, T, E, D);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return hip_fail(e, "router launch");
