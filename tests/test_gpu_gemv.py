@@ -785,6 +785,27 @@ def test_gemv_sixteen_weight_runs(O, tfq, gpu, fmt, N, K, dtype):
     W.close()
 
 
+@pytest.mark.parametrize("fmt", ["Q_4", "Q_G_6"])
+@pytest.mark.parametrize("N,K", [(3072, 2048), (3079, 1792), (4097, 2048), (6149, 1792)])
+def test_sixteen_weight_runs_over_the_grid(O, tfq, gpu, fmt, N, K):
+    """Rows around the counts at which a workgroup takes one more group of four rows (3072 or 4096): every output against the float64 product with the decoded matrix (bound as above, per
+    output against its terms), none written behind the last."""
+    import torch
+    w = torch.randn(N * K, generator=torch.Generator().manual_seed(N)).to(gpu) * 0.02
+    pay = tfq.encode(fmt, w)
+    W = tfq.Weight(fmt, N, K, pay)
+    dense = tfq.decode(fmt, pay, N * K).reshape(N, K).double()
+    for B in (1, 2, 4):
+        for dt in (torch.float32, torch.bfloat16):
+            x = torch.randn(B, K, generator=torch.Generator().manual_seed(B)).to(gpu).to(dt)
+            out = torch.full((B * N + 64,), 7.0, device=gpu)
+            W.gemv(x, out=out[:B * N].view(B, N))
+            want, terms = x.double() @ dense.T, x.double().abs() @ dense.abs().T
+            assert bool(((out[:B * N].view(B, N).double() - want).abs() <= 1e-6 * terms).all()), (B, dt)
+            assert bool((out[B * N:] == 7.0).all())
+    W.close()
+
+
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("fmt,N,K,per_row", [("Q_4", 301, 256, (1, 2, 4)), ("Q_4", 64, 768, (1, 2, 4)), ("Q_4", 301, 1024, (4,)), ("Q_4", 301, 1280, ()),
                                              ("Q_G_6", 301, 512, (1, 2, 4)), ("Q_G_6", 77, 1280, (1, 2, 4)), ("Q_G_6", 77, 1536, ()),

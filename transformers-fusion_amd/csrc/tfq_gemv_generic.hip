@@ -116,7 +116,7 @@ __device__ __attribute__((noinline)) float row_sum_lane63(const uint8_t* W, cons
 // wavefronts sixteen (K = 4096 in one pass, where a lane's activations then stay in registers); four weight rows
 // share every unpacked activation.  The codes of the next rows are fetched before the present ones are multiplied.
 // Before (a field extract and a conversion per code, a wavefront-wide sum per row, addresses per lane) and now, us: 128256 x 4096
-// Q_G_6 94 and 85 (two rows 110 and 113: 136 registers), Q_4 73 and 57, four rows 157 and 107; 14336 x 4096 13.3 and 11.5, 11.1 and 8.9.
+// Q_G_6 94 and 85, Q_4 73 and 57, four rows 157 and 107; 14336 x 4096 13.3 and 11.5, 11.1 and 8.9.
 template <int FMT>
 constexpr bool kRun16 = FMT == TFQ_Q_4 || FMT == TFQ_Q_G_6;
 constexpr int kRunRows = 4;
@@ -132,8 +132,14 @@ __device__ __forceinline__ float lane_move(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
 }
 
+// Workgroups that share a compute unit, by the registers: the grid is that many on each, or the last of them start when the
+// others end.  Two rows, and four of the 6-bit format, keep their activations in 120 to 168 registers where a pass covers K
+// (us, four on a unit and three: Q_G_6 4096 x 4096 two fp32 rows 8.1 and 6.4, four 10.2 and 8.8; Q_4 4096 x 2048 two fp32 rows
+// 6.6 and 5.6, 14336 x 4096 12.8 and 12.1; held to 128 registers two rows of Q_G_6 128256 x 4096 spill: 126 for 119).
+constexpr int run_share(int fmt, int bt, bool one_pass) { return one_pass && (bt == 2 || (bt == 4 && fmt == TFQ_Q_G_6)) ? 3 : 4; }
+
 template <int FMT, int BT, bool XF32, bool ONE_PASS>
-__global__ __launch_bounds__(256, BT == 4 ? 2 : FMT == TFQ_Q_G_6 && BT == 2 && ONE_PASS ? 3 : 4) void gemv_run16_kernel(const uint8_t* __restrict__ W, const void* __restrict__ xin,
+__global__ __launch_bounds__(256, BT != 4 ? run_share(FMT, BT, ONE_PASS) : FMT == TFQ_Q_G_6 ? 3 : 2) void gemv_run16_kernel(const uint8_t* __restrict__ W, const void* __restrict__ xin,
                                                          void* __restrict__ yout, int N, int K, int y_bf16) {
     constexpr int BB = spec_of(FMT).block_bytes, R = kRunRows;
     static_assert(R == 4);
@@ -328,9 +334,10 @@ int run(const tfq_weight* w, const void* x, int xd, void* y, int yd, hipStream_t
     const int N = (int)w->N, K = (int)w->K;
     if constexpr (kRun16<FMT>) {
         if (run16_pays<FMT, BT>(N, K)) {
-        // about a thousand workgroups (four per compute unit), each with the same number of row groups
-        const int groups = (N + kRunRows - 1) / kRunRows, per = (groups + 1023) / 1024, grid = (groups + per - 1) / per;
+        // as many workgroups as the compute units hold, each with the same number of row groups
         const bool one_pass = K <= 4096;
+        const int room = 256 * run_share(FMT, BT, one_pass);
+        const int groups = (N + kRunRows - 1) / kRunRows, per = (groups + room - 1) / room, grid = (groups + per - 1) / per;
         using Kernel = void (*)(const uint8_t*, const void*, void*, int, int, int);
         const Kernel kern = xd == TFQ_F32 ? (one_pass ? gemv_run16_kernel<FMT, BT, true, true> : gemv_run16_kernel<FMT, BT, true, false>)
                                           : (one_pass ? gemv_run16_kernel<FMT, BT, false, true> : gemv_run16_kernel<FMT, BT, false, false>);
