@@ -378,6 +378,41 @@ def test_moe_ffn_routed_shapes(O, tfq, gpu, T, Ktop, E):
         wl.close()
 
 
+@pytest.mark.parametrize("E,T,busy,exact", [(16, 512, 0, True), (16, 512, 512, True), (16, 1280, 0, False), (16, 1280, 900, False), (4, 256, 0, True)])
+def test_moe_ffn_rows_of_each_expert_choose_the_kernel(tfq, gpu, E, T, busy, exact):
+    """Prefill-sized calls with the lists on the host, `busy` tokens on expert 0 and the rest spread: up to 1024 pairs go through
+    the integer tile kernel, which does not round weights, however they are spread; 160 rows an expert on average through the
+    bf16 tile kernel, whose rounded weights show as 1e-3 of the output's norm.  Against float64 with the mid activations in bf16."""
+    import torch
+    D, F = 1024, 2816
+    gen = torch.Generator().manual_seed(E + T + busy)
+    ws, dense = [], []
+    for n, k in ((F, D), (F, D), (D, F)):
+        pays = [tfq.encode("B32S4", torch.randn(n * k, generator=gen).to(gpu) * 0.03) for _ in range(E)]
+        ws.append([tfq.Weight("B32S4", n, k, p) for p in pays])
+        dense.append([tfq.decode("B32S4", p, n * k).reshape(n, k).double() for p in pays])
+    idx = torch.stack([torch.randperm(E, generator=gen)[:2] for _ in range(T)])
+    for t in range(busy):
+        idx[t] = torch.tensor([0, 1 + t % (E - 1)])
+    w = torch.rand(T, 2, generator=gen) * 0.5 + 0.25
+    x = torch.randn(T, D, generator=gen).to(gpu).bfloat16()
+    want = torch.zeros(T, D, dtype=torch.float64, device=gpu)
+    for e in range(E):
+        t, j = (idx == e).nonzero(as_tuple=True)
+        if len(t) == 0:
+            continue
+        xe = x[t.to(gpu)].double()
+        mid = (torch.nn.functional.silu(xe @ dense[0][e].T) * (xe @ dense[1][e].T)).float().bfloat16().double()
+        want.index_add_(0, t.to(gpu), (mid @ dense[2][e].T) * w[t, j].to(gpu).double()[:, None])
+    y = tfq.moe_ffn(*ws, idx.numpy(), w.numpy(), x, mid_dtype=torch.bfloat16).double()
+    err = float((y - want).norm() / want.norm())
+    assert err <= 1e-2
+    assert (err <= 3e-4) == exact, err
+    for wl in ws:
+        for W in wl:
+            W.close()
+
+
 def test_moe_ffn_routed_refuses_what_it_does_not_serve(O, tfq, gpu):
     """More than 1024 pairs, or a format without the grouped kernels: no workspace size, and the call fails."""
     gate, up, down, _, _, _ = _experts(O, tfq, "B32S4", 2, 256, 512, 860)

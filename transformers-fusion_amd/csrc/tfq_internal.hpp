@@ -516,6 +516,8 @@ struct GemmExactGroups {
     size_t partial_bytes;
 };
 GemmExactGroups plan_gemm_exact_groups(const tfq_weight* w, int rows, int groups, size_t partial_bytes, bool pair);
+// about how long its launches take where the groups' first rows are `first` (host array, `groups` + 1 entries), up to a factor
+double gemm_exact_groups_us(const tfq_weight* w, const GemmExactGroups& g, const int* first, int groups, bool pair);
 int launch_gemm_exact_groups(const tfq_weight* w, const GemmExactGroups& g, const int* first, int groups, int rows, const uint8_t* const* mats,
                              const uint8_t* const* mats2, const void* x, void* y, int y_dtype, hipStream_t s, void* partial);
 // Whether the pair form is the faster side of two products, by whatever kernel, and the elementwise launch (with ample scratch)
@@ -526,6 +528,7 @@ bool gemm_pair_pays(const tfq_weight* w, int x_dtype, int M);
 struct GemmGroupPlan {
     int bn, grid;
     bool pp;
+    double us;  // about how long its launch takes, up to a factor
 };
 bool gemm_grouped_supported(const tfq_weight* w);
 size_t gemm_group_entry_bytes();

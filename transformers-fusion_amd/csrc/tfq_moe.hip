@@ -440,10 +440,12 @@ namespace {
 // Experts of some sixteen pairs each on average and more: the decode kernels read an expert's matrices once per eight or
 // sixteen of its rows and the bf16 tile kernel fills tiles of 256, the integer tile kernel's grouped form reads them once per
 // 32 or 64 rows, gate and up with the SwiGLU step in one launch and down in another.  us per call, 4096 / 14336, top-2 of 8
-// experts, before and here: 64 tokens B32S4 318 and 254, Q_G_8 560 and 335; 128 tokens 569 and 387, 653 and 467; below the line 32
-// tokens B32S4 210 and 265, Q_G_8 362 and 349.  (The 8-bit formats have twice the bytes for the same decode.)  At 160 rows an
-// expert and more the bf16 tile kernel's tiles are full.  By (T, k, E) alone, so that calls whose lists are on the host, on the
-// device or in a graph take the same kernels.
+// experts, decode kernels and here: 64 tokens B32S4 317 and 222, Q_G_8 537 and 336; 128 tokens 557 and 352, 985 and 446; below
+// the line 32 tokens B32S4 210 and 265, Q_G_8 362 and 349.  (The 8-bit formats have twice the bytes for the same decode.)  At
+// 160 rows an expert and more the bf16 tile kernel's tiles are full.  This is a rule of (T, k, E), as a call whose lists are on
+// the device has to have it, and the same for host lists up to the 1024 pairs that such a call takes: the same bits, of
+// weights that are not rounded.  Beyond, the rows of each expert decide as well (tall_is_faster).
+constexpr int kRoutedMaxPairs = 1024;  // T * k of a routed call (one workgroup builds the lists in LDS)
 struct ExpertGroups {
     bool use;
     GemmExactGroups up, down;
@@ -467,6 +469,19 @@ int launch_expert_groups(const tfq_weight* gate, const tfq_weight* down, const E
                          const uint8_t* const* ptrs, const void* xe, void* h, float* o, void* partial, hipStream_t s) {
     if (int rc = launch_gemm_exact_groups(gate, g.up, first, E, P, ptrs, ptrs + E, xe, h, TFQ_BF16, s, nullptr)) return rc;
     return launch_gemm_exact_groups(down, g.down, first, E, P, ptrs + 2 * E, nullptr, h, o, TFQ_F32, s, partial);
+}
+
+// Whether the bf16 tile kernel's grouped launches (gate and up in one, the elementwise one, down) are the faster side for
+// these rows of each expert: from some 70 rows an expert on, later where an expert's rows spill into another tile of 256.  Both
+// sides' launches by their models, fitted to 318 calls (eight kinds of experts, 13 to 160 rows each on average, evenly and
+// unevenly spread) within 8 and 6 %; three of those are then 5 % above the better side (us per call, here and there: 8 experts
+// 4096 / 14336 of B32S4, 144 rows each 988 and 731, 400 rows on one of 160 on average 1005 and 829; 16 experts 2048 / 5632 of
+// Q_G_8, 80 rows each 409 and 384, 640 on one of them 360 and 464; 145 rows each 546 and 417).
+bool tall_is_faster(const tfq_weight* const* gate, const tfq_weight* const* down, const ExpertGroups& eg, const GemmGroupPlan& tall_up,
+                    const GemmGroupPlan& tall_down, const std::vector<int>& first, int E) {
+    const double mids = 1e-6 * (double)first[E] * (double)gate[0]->N;
+    const double here = 14.0 + 1.10 * (gemm_exact_groups_us(gate[0], eg.up, first.data(), E, true) + gemm_exact_groups_us(down[0], eg.down, first.data(), E, false)) + 9.76 * mids;
+    return 36.0 + 0.78 * (tall_up.us + tall_down.us) + 7.26 * mids < here;
 }
 
 int moe_run(const tfq_weight* const* gate, const tfq_weight* const* up, const tfq_weight* const* down, int E,
@@ -493,15 +508,48 @@ int moe_run(const tfq_weight* const* gate, const tfq_weight* const* up, const tf
     // the expert's weights again: those calls go expert by expert through the prefill GEMM instead.
     int most_rows = 0;
     for (int e = 0; e < E; ++e) most_rows = std::max(most_rows, first[e + 1] - first[e]);
-    const ExpertGroups eg = plan_expert_groups(gate, up, down, E, T, Ktop, x_dtype, mid_dtype);
-    const bool tall = most_rows > 32 && !eg.use;
-    const bool grouped = P > 0 && !tall && !eg.use && gemv_grouped_supported(gate[0]->fmt) && gemv_grouped_supported(down[0]->fmt) &&
-                         canonical(gate[0]->fmt) == canonical(up[0]->fmt);
-    GemvGroupPlan planA{}, planB{};
-    bool down16 = false;  // the down stage through the sixteen-row kernel
+    ExpertGroups eg = plan_expert_groups(gate, up, down, E, T, Ktop, x_dtype, mid_dtype);
     std::vector<const tfq_weight*> wA, wA2, wB;
     std::vector<const void*> xA, xB;
     std::vector<void*> yA, yB;
+    // A prefill-sized call with bf16 rows and bf16 mid activations: the experts' gate and up products are ONE grouped
+    // launch of the tile kernel and their down products another, instead of three launches per expert, each of
+    // which fills a fraction of the compute units (512 rows x 14336 weight rows are 128 tiles of 224).
+    bool tall_grouped = most_rows > 32 && x_dtype == TFQ_BF16 && mid_dtype == TFQ_BF16;
+    for (int e = 0; e < E && tall_grouped; ++e)
+        tall_grouped = gemm_grouped_supported(gate[e]) && gemm_grouped_supported(up[e]) && gemm_grouped_supported(down[e]) &&
+                       canonical(gate[e]->fmt) == canonical(gate[0]->fmt) && canonical(up[e]->fmt) == canonical(gate[0]->fmt) &&
+                       canonical(down[e]->fmt) == canonical(down[0]->fmt);
+    GemmGroupPlan gplanA{}, gplanB{};
+    std::vector<int> mA, mB;
+    if (tall_grouped) {
+        for (int e = 0; e < E; ++e) {
+            const int p0 = first[e], nt = first[e + 1] - first[e];
+            if (nt <= 0) continue;
+            for (int half = 0; half < 2; ++half) {
+                wA.push_back(half ? up[e] : gate[e]);
+                xA.push_back(ws.xe + (size_t)p0 * D * xe_bytes);
+                yA.push_back((half ? ws.u : ws.g) + (size_t)p0 * F);
+                mA.push_back(nt);
+            }
+            wB.push_back(down[e]);
+            xB.push_back(ws.h + (size_t)p0 * F * he);
+            yB.push_back(ws.o + (size_t)p0 * D);
+            mB.push_back(nt);
+        }
+        int rc = plan_gemm_grouped(gate[0]->fmt, mA.data(), (int)mA.size(), F, D, &gplanA);
+        if (!rc) rc = plan_gemm_grouped(down[0]->fmt, mB.data(), (int)mB.size(), D, F, &gplanB);
+        if (rc && !eg.use) return rc;
+        if (!rc && eg.use && (int64_t)T * Ktop > kRoutedMaxPairs && tall_is_faster(gate, down, eg, gplanA, gplanB, first, E)) eg.use = false;
+        if (eg.use) {
+            tall_grouped = false;
+            wA.clear(); wB.clear(); xA.clear(); xB.clear(); yA.clear(); yB.clear();
+        }
+    }
+    const bool grouped = P > 0 && most_rows <= 32 && !eg.use && gemv_grouped_supported(gate[0]->fmt) && gemv_grouped_supported(down[0]->fmt) &&
+                         canonical(gate[0]->fmt) == canonical(up[0]->fmt);
+    GemvGroupPlan planA{}, planB{};
+    bool down16 = false;  // the down stage through the sixteen-row kernel
     std::vector<int> nA, nB, rA, rB, pB;  // pB: first pair of a down problem
     if (grouped) {
         int max_nt = 1;
@@ -564,34 +612,6 @@ int moe_run(const tfq_weight* const* gate, const tfq_weight* const* up, const tf
         } else if (int rc = plan_gemv_grouped(down[0]->fmt, (int)F, mid_dtype == TFQ_F32, nB.data(), rB.data(), (int)nB.size(), &planB)) {
             return rc;
         }
-    }
-    // A prefill-sized call with bf16 rows and bf16 mid activations: the experts' gate and up products are ONE grouped
-    // launch of the tile kernel and their down products another, instead of three launches per expert, each of
-    // which fills a fraction of the compute units (512 rows x 14336 weight rows are 128 tiles of 224).
-    bool tall_grouped = tall && x_dtype == TFQ_BF16 && mid_dtype == TFQ_BF16;
-    for (int e = 0; e < E && tall_grouped; ++e)
-        tall_grouped = gemm_grouped_supported(gate[e]) && gemm_grouped_supported(up[e]) && gemm_grouped_supported(down[e]) &&
-                       canonical(gate[e]->fmt) == canonical(gate[0]->fmt) && canonical(up[e]->fmt) == canonical(gate[0]->fmt) &&
-                       canonical(down[e]->fmt) == canonical(down[0]->fmt);
-    GemmGroupPlan gplanA{}, gplanB{};
-    std::vector<int> mA, mB;
-    if (tall_grouped) {
-        for (int e = 0; e < E; ++e) {
-            const int p0 = first[e], nt = first[e + 1] - first[e];
-            if (nt <= 0) continue;
-            for (int half = 0; half < 2; ++half) {
-                wA.push_back(half ? up[e] : gate[e]);
-                xA.push_back(ws.xe + (size_t)p0 * D * xe_bytes);
-                yA.push_back((half ? ws.u : ws.g) + (size_t)p0 * F);
-                mA.push_back(nt);
-            }
-            wB.push_back(down[e]);
-            xB.push_back(ws.h + (size_t)p0 * F * he);
-            yB.push_back(ws.o + (size_t)p0 * D);
-            mB.push_back(nt);
-        }
-        if (int rc = plan_gemm_grouped(gate[0]->fmt, mA.data(), (int)mA.size(), F, D, &gplanA)) return rc;
-        if (int rc = plan_gemm_grouped(down[0]->fmt, mB.data(), (int)mB.size(), D, F, &gplanB)) return rc;
     }
     const size_t eb = tall_grouped ? gemm_group_entry_bytes() : gemv_group_entry_bytes();
     const size_t gridA = tall_grouped ? (size_t)gplanA.grid : (size_t)planA.grid, gridB = tall_grouped ? (size_t)gplanB.grid : (size_t)planB.grid;
@@ -729,7 +749,6 @@ int moe_run(const tfq_weight* const* gate, const tfq_weight* const* up, const tf
 // host fixes from (T, k, E) alone, so the call can be captured into a graph.  Workgroups beyond the problems a
 // call turns out to have find -1 in their map and leave.  (Lists and tables come from one kernel of one workgroup.)
 namespace {
-constexpr int kRoutedMaxPairs = 1024;  // T * k of a routed call (one workgroup builds the lists in LDS)
 
 struct RoutedShape {
     int E, T, Ktop;
