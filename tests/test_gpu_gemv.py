@@ -499,6 +499,33 @@ def test_gemv_rows_on_integer_operands(O, tfq, gpu, fmt, dtype, B, N, K):
     W.close()
 
 
+@pytest.mark.parametrize("fmt,dtype,B,N,K,parts", [("Q_4", "bf16", 16, 14336, 4096, 4), ("Q_4", "f32", 12, 1100, 4096, 16), ("Q_G_6", "bf16", 9, 2000, 2048, 16),
+                                                   ("SB256A3", "f32", 16, 4096, 4096, 8)])
+def test_gemv_workspace_is_what_the_call_uses(tfq, gpu, fmt, dtype, B, N, K, parts):
+    """Five to sixteen rows on the integer tile kernel: the workspace asked for is at most `parts` partial results and a
+    whole number of them (none: unsplit), and one many times as large gives the same bits."""
+    import ctypes as C
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(16)
+    W = tfq.Weight(fmt, N, K, tfq.encode(fmt, torch.randn(N * K, device=gpu, generator=g) * 0.02))
+    x = torch.randn(B, K, device=gpu, generator=g)
+    x = x.bfloat16() if dtype == "bf16" else x
+    code = tfq.BF16 if dtype == "bf16" else tfq.F32
+    need = W.gemv_workspace_bytes(code, B)
+    print(f"workspace {need}", flush=True)
+    assert need % (B * N * 4) == 0 and need <= parts * B * N * 4
+    stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    got = []
+    for size in (need, 64 << 20):
+        ws = torch.empty(max(size, 256), device=gpu, dtype=torch.uint8)
+        y = torch.empty(B, N, device=gpu)
+        assert tfq.lib().tfq_gemv_ws(W.handle, C.c_void_p(x.data_ptr()), code, B, C.c_void_p(y.data_ptr()), tfq.F32,
+                                     C.c_void_p(ws.data_ptr()) if size else None, size, stream) == 0
+        got.append(y)
+    assert torch.equal(*got) and torch.equal(W.gemv(x), got[0])
+    W.close()
+
+
 def test_gemv_one_handle_on_two_streams(O, tfq, gpu):
     """Qwen35Engine::gemm is const and may run concurrently on one matrix (qwen35_engine.cpp:54-75): calls on
     one handle overlap on two streams, each with a workspace of its own, and give the bits of the serial
