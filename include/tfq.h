@@ -326,8 +326,8 @@ int tfq_matmul_host(const tfq_weight_t* w, const float* X, float* Y, int B);
  * mid_dtype is the type the SwiGLU product is rounded to before
  * the down projection: TFQ_F32 keeps it in fp32 like the reference, TFQ_BF16 feeds the matrix
  * cores.  workspace is device memory of at least tfq_mlp_workspace_bytes(B, F) bytes, 256-byte
- * aligned (the gate and up products, the SwiGLU product and, from three to sixteen rows, the partial sums of down's K
- * parts live there; the three products' areas alone, 3 B F fp32 each rounded up to 256 bytes, are accepted too). */
+ * aligned: the gate and up products, the SwiGLU product and the products' scratch live there.  (Up to sixteen rows the three
+ * products' areas alone, 3 B F fp32 each rounded up to 256 bytes, are accepted too: down's K parts are then fewer.) */
 size_t tfq_mlp_workspace_bytes(int B, int64_t F);
 int tfq_mlp_step(const tfq_weight_t* gate, const tfq_weight_t* up, const tfq_weight_t* down, const void* x,
                  int x_dtype, int B, void* y, int y_dtype, int mid_dtype, void* workspace, size_t workspace_bytes,

@@ -80,3 +80,15 @@ def test_block_sizes_equal_the_oracle_for_every_id_and_length(O, tfq):
                 assert rc != 0, (name, n)
             else:
                 assert rc == 0 and out.value == want, (name, n, out.value, want)
+
+
+def test_feed_forward_workspaces_hold_no_more_than_their_areas(tfq):
+    """Above sixteen rows the gate, up and SwiGLU products and at most 64 MiB of scratch, whatever the format; a mixture's
+    five areas, its lists and the same scratch."""
+    L = tfq.lib()
+    up = lambda n: (n + 255) // 256 * 256
+    for B, F in ((17, 256), (333, 14336), (4096, 28672)):
+        assert L.tfq_mlp_workspace_bytes(B, F) == 3 * up(B * F * 4) + up(min(8 * B * F * 4, 64 << 20))
+    for T, k, D, F in ((64, 2, 4096, 14336), (4096, 2, 4096, 14336)):
+        areas = 2 * T * k * D * 4 + 3 * T * k * F * 4 + min(8 * T * k * F * 4, 64 << 20)
+        assert areas <= L.tfq_moe_workspace_bytes(T, k, D, F) <= areas + T * k * (3 * 512 + 2 * F // 4 + D // 4) + 65536

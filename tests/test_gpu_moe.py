@@ -658,6 +658,35 @@ def test_mlp_step_pair_on_integer_operands(O, tfq, gpu, fmt, B, D, F, xdt, mid):
         W.close()
 
 
+@pytest.mark.parametrize("fmt,B,D,F,xdt", [("Q_4", 17, 512, 4352, "f32"), ("Q_4", 129, 4352, 512, "f32"), ("Q_G_6", 200, 768, 768, "bf16"),
+                                           ("B32S4", 300, 256, 1280, "bf16"), ("Q_G_3", 333, 1280, 256, "f32")])
+def test_mlp_step_scratch_in_the_areas_not_in_use(tfq, gpu, fmt, B, D, F, xdt):
+    """More than sixteen rows, gate, up and down one after the other (the wire formats) or as the models choose: each product's
+    scratch lies in areas that the later ones fill.  Against the float64 products of the decoded matrices (fp32 throughout 3e-5,
+    bf16 rows and mid activations 5e-3); a buffer behind the workspace stays as it was."""
+    import ctypes
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(83)
+    Ws = [tfq.Weight(fmt, n, k, tfq.encode(fmt, torch.randn(n * k, device=gpu, generator=g) * 0.02)) for n, k in ((F, D), (F, D), (D, F))]
+    x = torch.randn(B, D, device=gpu, generator=g)
+    x = x.bfloat16() if xdt == "bf16" else x
+    a, b, d = (W.decode().reshape(n, k).double() for W, (n, k) in zip(Ws, ((F, D), (F, D), (D, F))))
+    u = x.double() @ a.T
+    h = u * torch.sigmoid(u) * (x.double() @ b.T)
+    want = (h.bfloat16().double() if xdt == "bf16" else h) @ d.T
+    L, code = tfq.lib(), 1 if xdt == "bf16" else 0
+    size = L.tfq_mlp_workspace_bytes(B, F)
+    buf = torch.full((size + 4096,), 77, device=gpu, dtype=torch.uint8)
+    y = torch.empty(B, D, device=gpu)
+    rc = L.tfq_mlp_step(Ws[0].handle, Ws[1].handle, Ws[2].handle, ctypes.c_void_p(x.data_ptr()), code, B, ctypes.c_void_p(y.data_ptr()), 0, code,
+                        ctypes.c_void_p(buf.data_ptr()), size, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0
+    assert float((y.double() - want).norm() / want.norm()) <= (5e-3 if xdt == "bf16" else 3e-5)
+    assert bool((buf[size:] == 77).all())
+    for W in Ws:
+        W.close()
+
+
 @pytest.mark.parametrize("fmt,B,D,F,xdt,mid", [
     ("B32S4", 3, 512, 8448, "f32", "f32"),    # down's K in three parts
     ("Q_G_8", 4, 8192, 768, "f32", "f32"),    # the longest D of the paired launch with two slot sets

@@ -487,9 +487,8 @@ int launch_moe_ffn_capacity(const tfq_weight* const* gate, const tfq_weight* con
                             size_t workspace_bytes, int64_t* dropped, hipStream_t s);
 // `scratch` (optional, device memory) lets the tile kernel split K over several workgroups per output tile when
 // the tiles alone do not fill the GPU; gemm_scratch_bytes says how much a call would use, gemm_scratch_bound is
-// what the feed-forward calls need for any matrix with at most `rows` x `cols` outputs: all the bf16 tile kernel
-// would use (at most eight parts, 256 tiles), gemm_parts_bound what they ask for on top of it for the integer one, which
-// may plan more parts and makes do with what there is.
+// what the feed-forward calls set aside for any matrix with at most `rows` x `cols` outputs: all the bf16 tile kernel
+// would use (at most eight parts, 256 tiles); the integer one may plan more parts and makes do with what there is.
 int launch_gemm(const tfq_weight* w, const void* x, int x_dtype, int M, void* y, int y_dtype,
                 hipStream_t s, void* scratch = nullptr, size_t scratch_bytes = 0);
 size_t gemm_scratch_bytes(const tfq_weight* w, int x_dtype, int M);
@@ -542,11 +541,6 @@ size_t gemm_static_scratch_bytes();
 inline size_t gemm_scratch_bound(size_t rows, size_t cols) {
     const size_t by_split = 8 * rows * cols * 4, by_tiles = (size_t)256 * 256 * 256 * 4;
     return by_split < by_tiles ? by_split : by_tiles;
-}
-// and room for its activations split beforehand (three bf16 parts and their sums), K at most `cols`
-inline size_t gemm_parts_bound(size_t rows, size_t cols) {
-    const size_t all = rows * cols * 7 + 16 * cols, cap = (size_t)300 << 20;
-    return all < cap ? all : cap;
 }
 int launch_lut4_gemm(const uint8_t* packed, const uint16_t* cb16, const float* act, float* out, int M, int N, int K,
                      hipStream_t s);

@@ -273,9 +273,7 @@ int acquire_list_slot(size_t bytes, ListSlot** out) {
 
 }  // namespace
 
-size_t moe_workspace_bytes(int T, int Ktop, int64_t D, int64_t F) {
-    return carve(nullptr, T, Ktop, D, F).total + align256(gemm_parts_bound((size_t)T * (size_t)Ktop, (size_t)(F > D ? F : D)));
-}
+size_t moe_workspace_bytes(int T, int Ktop, int64_t D, int64_t F) { return carve(nullptr, T, Ktop, D, F).total; }
 
 namespace {
 // router logits[t][e] = x[t] . Wr[e] (+ bias[e]): one wavefront per (token, expert)
@@ -1108,9 +1106,10 @@ static size_t mlp_workspace_least(int B, int64_t F) {
 }
 
 // What it is asked to bring: from three to sixteen rows also room for the partial sums of the down product's K parts (of
-// at most F outputs; a down product of more, or a shorter workspace, runs unsplit).
+// at most F outputs; a down product of more, or a shorter workspace, runs unsplit).  More rows find room for activations
+// split beforehand in the areas that are not in use.
 size_t mlp_workspace_bytes(int B, int64_t F) {
-    if (B > 16) return mlp_workspace_least(B, F) + align256(gemm_parts_bound((size_t)B, (size_t)F));
+    if (B > 16) return mlp_workspace_least(B, F);
     const size_t pair_parts = B > 4 ? std::min((size_t)8 * (size_t)B * (size_t)F * 4, (size_t)32 << 20) : 0;  // of gate and up in four K parts each
     return mlp_workspace_least(B, F) + (B > 2 ? align256(std::max(gemv_rows16_split_bytes(TFQ_B32S4, F, (F + 255) / 256 * 256), pair_parts)) : 0);
 }
@@ -1125,12 +1124,10 @@ int launch_mlp_step(const tfq_weight* gate, const tfq_weight* up, const tfq_weig
     float* g = reinterpret_cast<float*>(workspace);
     float* u = reinterpret_cast<float*>((uint8_t*)workspace + part);
     void* h = (uint8_t*)workspace + 2 * part;
-    void* scratch = B > 16 ? (uint8_t*)workspace + 3 * part : nullptr;  // K-split partials of the prefill kernel
-    const size_t scratch_bytes = B > 16 ? workspace_bytes - 3 * part : 0;
     const bool paired = canonical(gate->fmt) == canonical(up->fmt) && gemv_pair_supported(gate) && gemv_pair_supported(up);
     const bool one_set = B <= (x_dtype == TFQ_F32 ? 2 : 4);
-    // The partial sums of the down product's K parts (three to sixteen rows): behind the three areas, or in the gate and up
-    // areas, whichever is larger; what does not fit runs unsplit.
+    // The scratch of the down product (three rows and more): behind the three areas, or in the gate and up areas, whichever
+    // is larger; K parts that do not fit are not made.
     auto down_rows = [&]() {
         const size_t have_tail = workspace_bytes - 3 * part;
         const bool areas = 2 * part >= have_tail;
@@ -1162,8 +1159,9 @@ int launch_mlp_step(const tfq_weight* gate, const tfq_weight* up, const tfq_weig
         void* gy[2] = {g, u};
         if (int rc = launch_gemv_multi(gu, 2, x, x_dtype, B, gy, TFQ_F32, s)) return rc;
     } else {
-        if (int rc = launch_gemm(gate, x, x_dtype, B, g, TFQ_F32, s, scratch, scratch_bytes)) return rc;
-        if (int rc = launch_gemm(up, x, x_dtype, B, u, TFQ_F32, s, scratch, scratch_bytes)) return rc;
+        // scratch: all that lies behind the output (above sixteen rows; below, formats of their own have none)
+        if (int rc = launch_gemm(gate, x, x_dtype, B, g, TFQ_F32, s, B > 16 ? u : nullptr, B > 16 ? workspace_bytes - part : 0)) return rc;
+        if (int rc = launch_gemm(up, x, x_dtype, B, u, TFQ_F32, s, B > 16 ? h : nullptr, B > 16 ? workspace_bytes - 2 * part : 0)) return rc;
     }
     if (B <= 16 && gemv_prologue_supported(down) && (B <= 2 || (mid_dtype == TFQ_F32 && F > 28672))) {
         // silu(gate) * up happens while the down kernel stages its activations: one launch less for one or two rows.
@@ -1183,8 +1181,7 @@ int launch_mlp_step(const tfq_weight* gate, const tfq_weight* up, const tfq_weig
     else
         hipLaunchKernelGGL(silu_mul_kernel<false>, dim3((unsigned)((nh + 255) / 256)), dim3(256), 0, s, g, u, h, nh);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return hip_fail(e, "mlp_step launch");
-    if (B <= 16) return down_rows();
-    return launch_gemm(down, h, mid_dtype, B, y, y_dtype, s, scratch, scratch_bytes);
+    return down_rows();
 }
 
 }  // namespace tfq
