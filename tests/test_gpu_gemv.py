@@ -499,7 +499,7 @@ def test_gemv_rows_on_integer_operands(O, tfq, gpu, fmt, dtype, B, N, K):
     W.close()
 
 
-@pytest.mark.parametrize("fmt,dtype,B,N,K,parts", [("Q_4", "bf16", 16, 14336, 4096, 4), ("Q_4", "f32", 12, 1100, 4096, 16), ("Q_G_6", "bf16", 9, 2000, 2048, 16),
+@pytest.mark.parametrize("fmt,dtype,B,N,K,parts", [("Q_4", "bf16", 16, 14336, 4096, 4), ("Q_4", "f32", 16, 2100, 4096, 16), ("Q_G_6", "bf16", 9, 2000, 2048, 16),
                                                    ("SB256A3", "f32", 16, 4096, 4096, 8)])
 def test_gemv_workspace_is_what_the_call_uses(tfq, gpu, fmt, dtype, B, N, K, parts):
     """Five to sixteen rows on the integer tile kernel: the workspace asked for is at most `parts` partial results and a

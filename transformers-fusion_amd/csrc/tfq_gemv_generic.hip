@@ -545,6 +545,26 @@ int launch_decode_mixed(const tfq_weight* w, float* out, hipStream_t s) {
     return hip_fail(hipGetLastError(), "decode launch");
 }
 
+// About how long (us) B rows of Q_4 or Q_G_6 take here, five and more: launches of four, two and one rows, each a start and its
+// rate per million weights, of whole passes of sixteen blocks; fitted to 540 products (256 x 1024 to 28672 x 4096, 4096 x 14336,
+// 1024 x 16384; five to sixteen rows) within 5 to 8 %, at most 21 %.
+double gemv_wire_rows_us(const tfq_weight* w, bool f32, int B) {
+    const bool six = canonical(w->fmt) == TFQ_Q_G_6;
+    const int N = (int)w->N, K = (int)w->K, passes = (K + 4095) / 4096, rest = B % 4;
+    static constexpr double rate[2][2][3] = {{{0.205, 0.125, 0.087}, {0.253, 0.139, 0.086}}, {{0.249, 0.167, 0.129}, {0.301, 0.185, 0.129}}};
+    static constexpr double start[2][2] = {{2.8, 3.05}, {2.8, 2.95}}, pass[2][2] = {{0.35, 0.50}, {0.40, 0.74}};
+    const double whole = (double)N * (double)passes * 4096e-6, mw = (double)N * (double)K * 1e-6;
+    auto launches = [&](int n, int bt, bool runs) {
+        if (runs) return n * (start[six][f32] + rate[six][f32][bt == 4 ? 0 : bt == 2 ? 1 : 2] * whole + pass[six][f32] * (passes - 1));
+        return n * (start[six][f32] + ((six ? 0.14 : 0.056) + (six ? 0.105 : 0.225) * bt) * mw);
+    };
+    auto runs = [&](int bt) {
+        if (six) return bt == 4 ? run16_pays<TFQ_Q_G_6, 4>(N, K) : run16_pays<TFQ_Q_G_6, 1>(N, K);
+        return bt == 4 ? run16_pays<TFQ_Q_4, 4>(N, K) : run16_pays<TFQ_Q_4, 1>(N, K);
+    };
+    return launches(B / 4, 4, runs(4)) + launches(rest / 2, 2, runs(2)) + launches(rest % 2, 1, runs(1));
+}
+
 int launch_gemv_generic(const tfq_weight* w, const void* x, int x_dtype, int B, void* y, int y_dtype, hipStream_t s) {
     if (w->layout != TFQ_LAYOUT_WIRE) return fail(TFQ_ERR_FORMAT, "gemv: generic kernel expects the wire layout");
     if (w->N > 0x7FFFFFFF || w->K > 0x7FFFFFFF) return fail(TFQ_ERR_SHAPE, "gemv: shape too large");

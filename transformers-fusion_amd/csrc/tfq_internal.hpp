@@ -386,6 +386,7 @@ bool gemv_wide_pair_fits(const tfq_weight* gate, int x_dtype, int B);
 bool gemv_pair_supported(const tfq_weight* w);  // the paired gate / up launch with the SwiGLU epilogue
 int launch_gemv_generic(const tfq_weight* w, const void* x, int x_dtype, int B, void* y, int y_dtype,
                         hipStream_t s);
+double gemv_wire_rows_us(const tfq_weight* w, bool f32, int B);
 // a matrix whose blocks mix wire ids (TFQ_LAYOUT_MIXED)
 constexpr int kMixedIds = 112;
 int launch_gemv_mixed(const tfq_weight* w, const void* x, int x_dtype, int B, void* y, int y_dtype, hipStream_t s);
