@@ -138,8 +138,10 @@ __device__ __forceinline__ float lane_move(float v) {
 // 6.6 and 5.6, 14336 x 4096 12.8 and 12.1; held to 128 registers two rows of Q_G_6 128256 x 4096 spill: 126 for 119).
 constexpr int run_share(int fmt, int bt, bool one_pass) { return one_pass && (bt == 2 || (bt == 4 && fmt == TFQ_Q_G_6)) ? 3 : 4; }
 
-template <int FMT, int BT, bool XF32, bool ONE_PASS>
-__global__ __launch_bounds__(256, BT != 4 ? run_share(FMT, BT, ONE_PASS) : FMT == TFQ_Q_G_6 ? 3 : 2) void gemv_run16_kernel(const uint8_t* __restrict__ W, const void* __restrict__ xin,
+// FEW: two workgroups a unit at most, whose four rows of the 6-bit format then take 170 registers and no spills (1024 x 4096, eight rows
+// 8.1 us with, 7.75 without; 128256 x 4096, four rows 148 us with two on a unit, 135 with three).
+template <int FMT, int BT, bool XF32, bool ONE_PASS, bool FEW = false>
+__global__ __launch_bounds__(256, BT != 4 ? run_share(FMT, BT, ONE_PASS) : FMT == TFQ_Q_G_6 && !FEW ? 3 : 2) void gemv_run16_kernel(const uint8_t* __restrict__ W, const void* __restrict__ xin,
                                                          void* __restrict__ yout, int N, int K, int y_bf16) {
     constexpr int BB = spec_of(FMT).block_bytes, R = kRunRows;
     static_assert(R == 4);
@@ -339,8 +341,12 @@ int run(const tfq_weight* w, const void* x, int xd, void* y, int yd, hipStream_t
         const int room = 256 * run_share(FMT, BT, one_pass);
         const int groups = (N + kRunRows - 1) / kRunRows, per = (groups + room - 1) / room, grid = (groups + per - 1) / per;
         using Kernel = void (*)(const uint8_t*, const void*, void*, int, int, int);
-        const Kernel kern = xd == TFQ_F32 ? (one_pass ? gemv_run16_kernel<FMT, BT, true, true> : gemv_run16_kernel<FMT, BT, true, false>)
-                                          : (one_pass ? gemv_run16_kernel<FMT, BT, false, true> : gemv_run16_kernel<FMT, BT, false, false>);
+        Kernel kern = xd == TFQ_F32 ? (one_pass ? gemv_run16_kernel<FMT, BT, true, true> : gemv_run16_kernel<FMT, BT, true, false>)
+                                    : (one_pass ? gemv_run16_kernel<FMT, BT, false, true> : gemv_run16_kernel<FMT, BT, false, false>);
+        if constexpr (FMT == TFQ_Q_G_6 && BT == 4) {
+            if (groups <= 512) kern = xd == TFQ_F32 ? (one_pass ? gemv_run16_kernel<FMT, BT, true, true, true> : gemv_run16_kernel<FMT, BT, true, false, true>)
+                                                    : (one_pass ? gemv_run16_kernel<FMT, BT, false, true, true> : gemv_run16_kernel<FMT, BT, false, false, true>);
+        }
         hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, s, w->dev, x, y, N, K, yd == TFQ_BF16);
         return hip_fail(hipGetLastError(), "gemv launch");
         }
