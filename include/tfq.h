@@ -264,12 +264,13 @@ int tfq_gemm_ws(const tfq_weight_t* w, const void* x, int x_dtype, int M, void* 
  * serving loops, harnesses that forbid hipMalloc.  The K-split scratch is a fixed array of
  * tfq_gemm_static_scratch_bytes() = 32 MiB in the library's device image (every GPU the library runs on holds
  * its copy until the process ends); the call itself allocates nothing.  Same results, bit for bit, as tfq_gemm_ws
- * with a workspace of tfq_gemm_workspace_bytes.  Where that is more than the array holds, a product of the bf16 tile
- * kernel (bf16 x on B32S4, B32S8, Q_G_4, Q_G_8, Q_8, Q_G_3) is refused with TFQ_ERR_SHAPE; one of the integer tile
- * kernel is served, its rows in several runs.  All calls on one GPU share the array: calls that overlap in time
- * on one GPU race (issue them on one stream).  The first call on a device resolves the array's address and
- * raises the kernel's LDS limit.  ROCm 7.2 accepts both while a stream is being captured; where a runtime does
- * not, make one call of the same shape before a capture starts (the same holds for the first use of the other
+ * with a workspace of tfq_gemm_workspace_bytes.  What the bf16 tile kernel serves or could serve (bf16 x on
+ * B32S4, B32S8, Q_G_4, Q_G_8, Q_8, Q_G_3) is refused with TFQ_ERR_SHAPE where that kernel's K split takes more
+ * than the array holds; any other product of the integer tile kernel is served, its rows in several runs where
+ * needed.  All calls on one GPU share the array: calls that overlap in time on one GPU race (issue them on one
+ * stream).  The first call on a device resolves the array's address and raises the kernel's LDS limit.  ROCm
+ * 7.2 accepts both while a stream is being captured; where a runtime does not, make one call of the same shape
+ * before a capture starts (the same holds for the first use of the other
  * kernels of a tiled format; those of the wire formats raise no limit).  No counterpart in the reference: it is for callers that cannot allocate. */
 int tfq_gemm_static(const tfq_weight_t* w, const void* x, int x_dtype, int M, void* y, int y_dtype,
                     tfq_stream_t stream);
