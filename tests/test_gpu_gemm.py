@@ -205,6 +205,30 @@ def test_gemm_integer_operands_any_scratch(tfq, gpu, fmt, dtype, M, N, K):
     W.close()
 
 
+@pytest.mark.parametrize("fmt,dtype", EXACT_FMTS + [(f, "bf16") for f in ("Q_G_4", "Q_G_3", "B32S4", "B32S8", "Q_G_8", "Q_8")])
+@pytest.mark.parametrize("N,K", [(1, 256), (31, 896 + 128), (33, 1280), (200, 2816), (65, 4096), (96, 4352)])
+def test_gemm_small_products_in_one_launch(tfq, gpu, fmt, dtype, N, K):
+    """K over the wavefronts of a workgroup: fewer half blocks than wavefronts, shares of different sizes, the longest K that
+    is served and the next one; ragged tiles on either side.  Against the float64 product, the bounds of
+    test_gemm_integer_operands_any_scratch (the bf16 rows' weights are not rounded either); a row's sums do not depend on
+    the tile that it is in, nor on the rows beside it."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(31)
+    W = tfq.Weight(fmt, N, K, tfq.encode(fmt, torch.randn(N * K, device=gpu, generator=g) * 0.02))
+    dense = W.decode().reshape(N, K).double()
+    bound = 1.5e-4 if fmt in ("Q_G_8", "Q_8") else 1e-6 if dtype == "bf16" or fmt in ("Q_4", "Q_G_6") else 1e-5
+    x = torch.randn(95, K, device=gpu, generator=g)
+    x = x.bfloat16() if dtype == "bf16" else x
+    want = x.double() @ dense.T
+    all_rows = W.gemm(x, out_dtype=torch.float32)
+    for M in (17, 32, 33, 95):
+        y = W.gemm(x[:M].contiguous(), out_dtype=torch.float32)
+        assert float((y.double() - want[:M]).norm() / want[:M].norm()) <= bound, (fmt, dtype, N, K, M)
+        if 1024 <= K <= 2816:  # (every count of rows takes this kernel)
+            assert torch.equal(y, all_rows[:M])
+    W.close()
+
+
 @pytest.mark.parametrize("fmt", ["Q_4", "Q_G_6"])
 def test_gemm_integer_operands_non_finite(O, tfq, gpu, fmt):
     """Infinite, not-a-number and huge activations give what the fp32 products of the 16-row path give."""

@@ -503,7 +503,7 @@ size_t gemv_split_bytes(const tfq_weight* w);
 // their weights.  Any scratch size is served (less scratch, fewer K parts); gemm_exact_us says how long it would take.
 bool gemm_exact_serves(const tfq_weight* w, int M);
 size_t gemm_exact_scratch_bytes(const tfq_weight* w, int x_dtype, int M);
-double gemm_exact_us(const tfq_weight* w, int x_dtype, int M, size_t scratch_bytes, int matrices = 1);
+double gemm_exact_us(const tfq_weight* w, int x_dtype, int M, size_t scratch_bytes, int matrices = 1, bool solo = true);
 int launch_gemm_exact(const tfq_weight* w, const void* x, int x_dtype, int M, void* y, int y_dtype, hipStream_t s, void* scratch,
                       size_t scratch_bytes, bool keep_split = false);
 // Its pair form, y = silu(w x) * (w2 x), and its grouped form: rows first[e] to first[e + 1] (device array) of x and y go with
