@@ -1292,22 +1292,22 @@ __global__ __launch_bounds__(1024) void gemvb_kernel(GemvKernArgs args, const un
 // them).  fp32 rows are two adjacent slots each, added first like the unsplit kernel adds them.  (The parts used
 // to meet inside the kernel: device-scope stores, an arrival counter per row group, the last arriver reading all
 // parts back.  That chain of dependent memory round trips cost 6 us of a 17 us launch, 4096 x 14336 at sixteen
-// rows; this kernel and its launch boundary cost 3.5 us.)
+// rows; this kernel and its launch boundary cost 3.5 us, and some 0.7 less since the parts' loads are under way together: that
+// product 15.1 -> 14.3 us.)
 __global__ __launch_bounds__(256) void split_reduce_kernel(const float* __restrict__ partial, void* __restrict__ y, int kparts, int B,
                                                           int nrm, int y_bf16, int x_f32) {
     const int row = blockIdx.x * 256 + threadIdx.x, b = blockIdx.y;  // one output per lane
     if (row >= nrm) return;
     {
         float v = 0.0f;
+        const size_t n = (size_t)nrm;
+        const float* const p = partial + (size_t)row;
         if (x_f32) {
             float lo = 0.0f;
-            for (int c = 0; c < kparts; ++c) {
-                v += partial[((size_t)c * 16 + 2 * b) * (size_t)nrm + row];
-                lo += partial[((size_t)c * 16 + 2 * b + 1) * (size_t)nrm + row];
-            }
+            for_parts(2 * kparts, [&](int i) { return p + ((size_t)(i >> 1) * 16 + 2 * b + (i & 1)) * n; }, [&](int i, float t) { (i & 1 ? lo : v) += t; });
             v += lo;
         } else {
-            for (int c = 0; c < kparts; ++c) v += partial[((size_t)c * 16 + b) * (size_t)nrm + row];
+            for_parts(kparts, [&](int i) { return p + ((size_t)i * 16 + b) * n; }, [&](int, float t) { v += t; });
         }
         const size_t off = (size_t)b * (size_t)nrm + (size_t)row;
         if (y_bf16) reinterpret_cast<unsigned short*>(y)[off] = (unsigned short)bf16_rne(v);

@@ -609,4 +609,26 @@ __device__ __forceinline__ uint32_t stream_bits(const uint8_t* p, uint32_t size,
     return (w >> (pos & 7)) & ((1u << count) - 1u);
 }
 
+// use(i, *at(i)) for i = 0 ... n - 1, in order (n: the same in every lane).  Up to eight loads are under way together: behind
+// each other they were a memory round trip per part, which is what a kernel that adds K parts takes (it moves little else).
+template <int B, class At, class Use>
+__device__ __forceinline__ void for_parts_by(int n, At&& at, Use&& use) {
+    for (int i0 = 0; i0 < n; i0 += B) {
+        float v[B];
+#pragma unroll
+        for (int k = 0; k < B; ++k) v[k] = *at(min(i0 + k, n - 1));  // past the end: the last one again
+#pragma unroll
+        for (int k = 0; k < B; ++k) asm volatile("" : "+v"(v[k]));   // (or the last loads move behind the comparisons)
+#pragma unroll
+        for (int k = 0; k < B; ++k)
+            if (i0 + k < n) use(i0 + k, v[k]);
+    }
+}
+template <class At, class Use>
+__device__ __forceinline__ void for_parts(int n, At&& at, Use&& use) {
+    if (n <= 2) for_parts_by<2>(n, at, use);
+    else if (n <= 4) for_parts_by<4>(n, at, use);
+    else for_parts_by<8>(n, at, use);
+}
+
 }  // namespace tfq

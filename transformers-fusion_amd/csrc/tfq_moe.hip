@@ -88,10 +88,19 @@ __global__ __launch_bounds__(256) void combine_kernel(void* __restrict__ out, co
     if (i >= (int64_t)T * D) return;
     const int t = (int)(i / D), d = (int)(i - (int64_t)t * D);
     float acc = 0.0f;
-    for (int j = tok_first[t]; j < tok_first[t + 1]; ++j) {
-        const int p = tok_pairs[j];
-        const float wt = w[p];
-        if (wt > 0.0f || keep_all) acc += wt * o[(int64_t)p * D + d];
+    // four pairs at a time, so that their loads do not wait for each other (a mixture of 106 tokens, four pairs each, D 1280:
+    // 46.6 -> 44.4 us a call)
+    const int end = tok_first[t + 1];
+    for (int j = tok_first[t]; j < end; j += 4) {
+        int p[4];
+        float wt[4], v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) p[k] = tok_pairs[min(j + k, end - 1)];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) { wt[k] = w[p[k]]; v[k] = o[(int64_t)p[k] * D + d]; }
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (j + k < end && (wt[k] > 0.0f || keep_all)) acc += wt[k] * v[k];
     }
     if (OUT_BF16) reinterpret_cast<unsigned short*>(out)[i] = (unsigned short)bf16_rne(acc);
     else reinterpret_cast<float*>(out)[i] = acc;
