@@ -220,12 +220,32 @@ def test_gemm_small_products_in_one_launch(tfq, gpu, fmt, dtype, N, K):
     x = torch.randn(95, K, device=gpu, generator=g)
     x = x.bfloat16() if dtype == "bf16" else x
     want = x.double() @ dense.T
-    all_rows = W.gemm(x, out_dtype=torch.float32)
     for M in (17, 32, 33, 95):
         y = W.gemm(x[:M].contiguous(), out_dtype=torch.float32)
         assert float((y.double() - want[:M]).norm() / want[:M].norm()) <= bound, (fmt, dtype, N, K, M)
-        if 1024 <= K <= 2816:  # (every count of rows takes this kernel)
-            assert torch.equal(y, all_rows[:M])
+        if 1024 <= K <= 2816:  # (every count of rows takes this kernel, in one part of K or in several)
+            assert torch.equal(W.gemm(x[:M].flip(0).contiguous(), out_dtype=torch.float32), y.flip(0))
+    W.close()
+
+
+@pytest.mark.parametrize("fmt,dtype", [("B32S4", "bf16"), ("Q_G_4", "f32"), ("Q_G_8", "bf16"), ("SB256A3", "f32"), ("Q_4", "f32"), ("Q_G_6", "bf16")])
+@pytest.mark.parametrize("N,K", [(96, 4608), (320, 6400), (65, 14336), (1, 15872)])
+def test_gemm_small_products_in_k_parts(tfq, gpu, fmt, dtype, N, K):
+    """Few tiles of a long K: parts of K over workgroups (of unequal length where the blocks do not divide), up to more of them than
+    one batch of the launch that adds them loads.  Rows of a tile and of the next one, one to sixteen rows (gemv) and more.  The
+    bounds of test_gemm_integer_operands_any_scratch; a feed-forward's pair of matrices in parts against two products."""
+    import torch
+    print(f"gemm k parts {fmt} {dtype} N={N} K={K}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(33)
+    W = tfq.Weight(fmt, N, K, tfq.encode(fmt, torch.randn(N * K, device=gpu, generator=g) * 0.02))
+    dense = W.decode().reshape(N, K).double()
+    bound = 1.5e-4 if fmt == "Q_G_8" else 1e-6 if dtype == "bf16" or fmt in ("Q_4", "Q_G_6") else 1e-5
+    for M in (5, 16, 17, 32, 33, 70):
+        x = torch.randn(M, K, device=gpu, generator=g)
+        x = x.bfloat16() if dtype == "bf16" else x
+        want = x.double() @ dense.T
+        y = W.gemv(x) if M <= 16 else W.gemm(x, out_dtype=torch.float32)
+        assert float((y.double() - want).norm() / want.norm()) <= bound, (M, float((y.double() - want).norm() / want.norm()))
     W.close()
 
 
