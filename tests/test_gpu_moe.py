@@ -354,6 +354,37 @@ def test_moe_ffn_routed_single_token(O, tfq, gpu, fmt, D, F):
         wl.close()
 
 
+@pytest.mark.parametrize("Ktop", [1, 2, 3, 4, 5, 8, 9])
+@pytest.mark.parametrize("D", [256, 768])
+def test_moe_ffn_combine(tfq, gpu, Ktop, D):
+    """The step that adds a token's pairs, in batches of four and two with a rest, tokens without a pair or with one among them.
+    Against the sum of one-pair mixtures of the same rows in float64: fp32 sums of
+    up to nine rows (their products may come from other kernels: 1e-5, as in test_moe_ffn_routed_shapes), bf16 by one rounding more."""
+    import torch
+    E, F, T = 12, 256, 9
+    g = torch.Generator(device="cuda").manual_seed(41)
+    mat = lambda n, k: tfq.Weight("B32S4", n, k, tfq.encode("B32S4", torch.randn(n * k, device=gpu, generator=g) * 0.05))
+    ws = [[mat(F, D) for _ in range(E)], [mat(F, D) for _ in range(E)], [mat(D, F) for _ in range(E)]]
+    x = torch.randn(T, D, device=gpu, generator=g)
+    rng = np.random.default_rng(42)
+    idx = np.stack([rng.permutation(E)[:Ktop] for _ in range(T)]).astype(np.int64)
+    w = rng.uniform(0.1, 1.0, (T, Ktop)).astype(np.float32)
+    w[1, :] = 0.0
+    w[2, 1:] = 0.0
+    w[3, :-1] = 0.0
+    want = torch.zeros(T, D, dtype=torch.float64, device=gpu)
+    for j in range(Ktop):
+        want += tfq.moe_ffn(*ws, idx[:, j:j + 1].copy(), w[:, j:j + 1].copy(), x, mid_dtype=torch.float32).double()
+    top = float(want.abs().max())
+    y = tfq.moe_ffn(*ws, idx, w, x, mid_dtype=torch.float32)
+    yb = tfq.moe_ffn(*ws, idx, w, x, mid_dtype=torch.float32, out_dtype=torch.bfloat16)
+    assert float((y.double() - want).abs().max()) <= 1e-5 * top
+    assert torch.equal(yb, y.bfloat16())
+    assert not y[1].any() and not yb[1].any()
+    for wl in sum(ws, []):
+        wl.close()
+
+
 @pytest.mark.parametrize("T,Ktop,E", [(1, 1, 3), (7, 3, 5), (64, 2, 4), (128, 8, 16), (5, 2, 40)])
 def test_moe_ffn_routed_shapes(O, tfq, gpu, T, Ktop, E):
     """Call shapes of the routed form: one pair, odd counts, experts with several passes of eight and sixteen
