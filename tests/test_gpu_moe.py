@@ -409,6 +409,34 @@ def test_moe_ffn_routed_shapes(O, tfq, gpu, T, Ktop, E):
         wl.close()
 
 
+@pytest.mark.parametrize("T,Ktop,E", [(1, 3, 2), (21, 3, 64), (13, 5, 65), (128, 8, 200), (256, 4, 256)])
+def test_moe_ffn_routed_lists(tfq, gpu, T, Ktop, E):
+    """The lists of a routed call: slots of one wavefront and of all sixteen, as many experts as lanes, one more, and the most that
+    are taken; ids out of range, an expert with most of the tokens.  Against tfq_moe_ffn with the same routing (its rows are cut
+    into passes by other rules: 1e-5 as in test_moe_ffn_routed_shapes, 1e-2 where it takes the prefill GEMM)."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(43)
+    D = F = 256
+    print(f"routed lists T={T} k={Ktop} E={E}", flush=True)
+    mat = lambda: tfq.Weight("B32S4", D, F, tfq.encode("B32S4", torch.randn(D * F, device=gpu, generator=g) * 0.05))
+    gate, up, down = ([mat() for _ in range(E)] for _ in range(3))
+    rng = np.random.default_rng(44)
+    idx = np.stack([rng.permutation(E + 2)[:Ktop] - 1 for _ in range(T)]).astype(np.int64)  # (-1 and E: no expert)
+    for t in range(0, T, 3):
+        if not (idx[t] == E - 1).any():
+            idx[t, 0] = E - 1
+    w = rng.uniform(0.1, 1.0, (T, Ktop)).astype(np.float32)
+    x = torch.randn(T, D, device=gpu, generator=g).bfloat16()
+    host = tfq.moe_ffn(gate, up, down, idx, w, x, mid_dtype=torch.bfloat16)
+    y = torch.empty(T, D, device=gpu)
+    call = tfq.RoutedMoe(gate, up, down, T, Ktop)
+    call(torch.from_numpy(idx.astype(np.int32)).to(gpu), torch.from_numpy(w).to(gpu), x, y)
+    tol = 1e-2 if max(int((idx == e).sum()) for e in range(E)) > 32 else 1e-5
+    assert float((y - host).abs().max()) <= tol * float(host.abs().max())
+    for wl in gate + up + down:
+        wl.close()
+
+
 @pytest.mark.parametrize("E,T,busy,exact", [(16, 512, 0, True), (16, 512, 512, True), (16, 1280, 0, False), (16, 1280, 900, False), (4, 256, 0, True)])
 def test_moe_ffn_rows_of_each_expert_choose_the_kernel(tfq, gpu, E, T, busy, exact):
     """Prefill-sized calls with the lists on the host, `busy` tokens on expert 0 and the rest spread: up to 1024 pairs go through

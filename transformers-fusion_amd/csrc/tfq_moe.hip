@@ -794,8 +794,8 @@ __global__ __launch_bounds__(1024) void routed_lists_kernel(const int32_t* __res
                                                             const uint4* __restrict__ x, int row_u4) {
     __shared__ int s_idx[kRoutedMaxPairs];
     __shared__ int s_tok[kRoutedMaxPairs];
-    __shared__ int s_first[257];
-    __shared__ int s_cnt[256];
+    __shared__ int s_first[257], s_offA[257], s_offB[257];
+    __shared__ int s_cnt[(kRoutedMaxPairs / 64) * 256];  // slots of an expert in every wavefront's 64
     __shared__ int s_pair[kRoutedMaxPairs];
     __shared__ float s_w[kRoutedMaxPairs];
     const int P = T * Ktop, tid = threadIdx.x;
@@ -805,28 +805,70 @@ __global__ __launch_bounds__(1024) void routed_lists_kernel(const int32_t* __res
     // which the copy of the rows below dominated.)
     const uint8_t *p_gate = nullptr, *p_up = nullptr, *p_down = nullptr;
     if (tid < E) { p_gate = ptrs[tid]; p_up = ptrs[E + tid]; p_down = ptrs[2 * E + tid]; }
-    for (int e = tid; e < E; e += blockDim.x) s_cnt[e] = 0;
-    for (int sl = tid; sl < P; sl += blockDim.x) {
-        const int e = idx[sl];
-        s_w[sl] = w[sl];
-        s_idx[sl] = e >= 0 && e < E ? e : -1;
+    const int waves = (P + 63) >> 6, wave = tid >> 6, lane = tid & 63;
+    for (int i = tid; i < waves * E; i += blockDim.x) s_cnt[i] = 0;
+    int own = -1;  // the thread's slot's expert
+    if (tid < P) {
+        const int e = idx[tid];
+        s_w[tid] = w[tid];
+        own = e >= 0 && e < E ? e : -1;
+        s_idx[tid] = own;
     }
     __syncthreads();
-    // rank of a slot among the slots of its expert, in slot order
-    for (int sl = tid; sl < P; sl += blockDim.x) {
-        const int e = s_idx[sl];
-        int rank = 0;
-        if (e >= 0) {
-            for (int q = 0; q < sl; ++q) rank += s_idx[q] == e;
-            atomicAdd(&s_cnt[e], 1);
+    // Rank of a slot among the slots of its expert, in slot order: the lower lanes of its wavefront with the same expert, from
+    // ballots of the id's bits, and the counts of the wavefronts before it.  What bounds the kernel is its chain of dependent
+    // steps: a loop over all lower slots was as long as the call has pairs, and one lane added up the experts twice, with barriers
+    // around it.  us a call with that and now: 16 tokens of two slots, D 2048, 29.0 and 28.6, 32 of two among 16 experts, D 1280,
+    // 39.2 and 38.2, 106 of four 64.1 and 58.7, 128 of eight, D 4096, 130.3 and 115.1.
+    int rank = 0;
+    if (wave < waves) {
+        uint64_t same = __ballot(own >= 0);
+#pragma unroll
+        for (int b = 0; b < 8; ++b) {
+            const uint64_t set = __ballot((own >> b) & 1);
+            same &= (own >> b) & 1 ? set : ~set;
         }
-        s_pair[sl] = rank;
+        rank = __popcll(same & ((1ull << lane) - 1));
+        if (own >= 0 && rank == 0) s_cnt[wave * E + own] = __popcll(same);
     }
     __syncthreads();
-    if (tid == 0) {
-        int acc = 0;
-        for (int e = 0; e < E; ++e) { s_first[e] = acc; acc += s_cnt[e]; }
-        s_first[E] = acc;
+    if (own >= 0)
+        for (int g = 0; g < wave; ++g) rank += s_cnt[g * E + own];
+    // First pair and first problems (an expert's rows in chunks of capA / capB) of every expert: sums over up to four experts a lane,
+    // then over the lanes.  (Problems are at most as many as pairs: two counts of 16 bits.)
+    if (wave == 0) {
+        const int per = (E + 63) >> 6;
+        int pairs[4], probs[4], n = 0, m = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int e = lane * per + k;
+            int c = 0;
+            if (k < per && e < E)
+                for (int g = 0; g < waves; ++g) c += s_cnt[g * E + e];
+            pairs[k] = n;
+            probs[k] = m;
+            n += c;
+            m += (c + sh.capA - 1) / sh.capA + ((c + sh.capB - 1) / sh.capB << 16);
+        }
+        int sn = n, sm = m;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int un = __shfl_up(sn, d), um = __shfl_up(sm, d);
+            if (lane >= d) { sn += un; sm += um; }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int e = lane * per + k, first_prob = sm - m + probs[k];
+            if (k >= per || e >= E) continue;
+            s_first[e] = sn - n + pairs[k];
+            s_offA[e] = first_prob & 0xFFFF;
+            s_offB[e] = first_prob >> 16;
+        }
+        if (lane == 63) {
+            s_first[E] = sn;
+            s_offA[E] = sm & 0xFFFF;
+            s_offB[E] = sm >> 16;
+        }
     }
     __syncthreads();
     // With the gather on board the launch has several workgroups: each builds the lists in its own LDS (a few
@@ -838,19 +880,19 @@ __global__ __launch_bounds__(1024) void routed_lists_kernel(const int32_t* __res
         for (int p = total + tid; p < P; p += blockDim.x) rows[p] = 0;
         if (tid == 0) wts[P] = 0.0f;
     }
-    for (int sl = tid; sl < P; sl += blockDim.x) {
-        const int e = s_idx[sl];
-        if (e < 0) { s_pair[sl] = P; continue; }
-        const int p = s_first[e] + s_pair[sl];
-        const int t = sl / Ktop;
+    if (own < 0) {
+        if (tid < P) s_pair[tid] = P;
+    } else {
+        const int p = s_first[own] + rank;
+        const int t = tid / Ktop;
         float wt = 0.0f;
         for (int j = 0; j < Ktop; ++j)
-            if (s_idx[t * Ktop + j] == e) { wt = s_w[t * Ktop + j]; break; }
+            if (s_idx[t * Ktop + j] == own) { wt = s_w[t * Ktop + j]; break; }
         if (lead) {
             rows[p] = t;
             wts[p] = wt;
         }
-        s_pair[sl] = p;
+        s_pair[tid] = p;
         s_tok[p] = t;
     }
     __syncthreads();
@@ -885,54 +927,29 @@ __global__ __launch_bounds__(1024) void routed_lists_kernel(const int32_t* __res
     }
     // Problem tables and workgroup maps of the two grouped launches: an expert's rows in chunks of capA / capB.
     // ptrs = device addresses of the experts' packed matrices, [gate | up | down][E].
-    __shared__ int s_nA, s_nB, s_wgA, s_tilesA;
-    __shared__ int s_offA[257], s_offB[257];
-    for (int e = tid; e < E; e += blockDim.x) {  // problems of an expert in either launch: its rows in chunks of capA / capB
-        const int nt = s_first[e + 1] - s_first[e];
-        s_offA[e] = (nt + sh.capA - 1) / sh.capA;
-        s_offB[e] = (nt + sh.capB - 1) / sh.capB;
+    const int nA = s_offA[E], nB = s_offB[E];
+    // The tile-owning kernel runs a workgroup per compute unit: when a call has more problems than the plan
+    // assumed (an expert's rows in several chunks), its wavefronts take more tile pairs each, so that the
+    // workgroups still fit one round.
+    int wgA = sh.wgA, tilesA = 0;
+    if (sh.nwA) {
+        const int tiles = (sh.nrowsA + 15) >> 4;
+        int r = sh.rA;
+        while (r < 64 && nA * ((tiles + sh.nwA * r - 1) / (sh.nwA * r)) > 256) ++r;
+        tilesA = sh.nwA * r;
+        wgA = (tiles + tilesA - 1) / tilesA;
     }
-    __syncthreads();
-    if (tid == 0) {
-        int nA = 0, nB = 0;  // counts -> first problem of every expert
-        for (int e = 0; e < E; ++e) {
-            const int cA = s_offA[e], cB = s_offB[e];
-            s_offA[e] = nA;
-            s_offB[e] = nB;
-            nA += cA;
-            nB += cB;
-        }
-        s_nA = nA;
-        s_nB = nB;
-        // The tile-owning kernel runs a workgroup per compute unit: when a call has more problems than the plan
-        // assumed (an expert's rows in several chunks), its wavefronts take more tile pairs each, so that the
-        // workgroups still fit one round.
-        int wgA = sh.wgA, tilesA = 0;
-        if (sh.nwA) {
-            const int tiles = (sh.nrowsA + 15) >> 4;
-            int r = sh.rA;
-            while (r < 64 && nA * ((tiles + sh.nwA * r - 1) / (sh.nwA * r)) > 256) ++r;
-            tilesA = sh.nwA * r;
-            wgA = (tiles + tilesA - 1) / tilesA;
-        }
-        s_wgA = wgA;
-        s_tilesA = tilesA;
-    }
-    __syncthreads();
     for (int e = tid; e < E; e += blockDim.x) {  // an expert's table entries, by one thread
         const int p0 = s_first[e], nt = s_first[e + 1] - p0;
         int iA = s_offA[e], iB = s_offB[e];
         for (int b0 = 0; b0 < nt; b0 += sh.capA, ++iA)
             tabA[iA] = GemvProb{p_gate, h + (size_t)(p0 + b0) * sh.strideYA, xe + (size_t)(p0 + b0) * sh.strideXA, p_up,
-                                sh.nrowsA, min(sh.capA, nt - b0), iA * s_wgA, s_tilesA};
+                                sh.nrowsA, min(sh.capA, nt - b0), iA * wgA, tilesA};
         for (int b0 = 0; b0 < nt; b0 += sh.capB, ++iB)
             tabB[iB] = GemvProb{p_down, o + (size_t)(p0 + b0) * sh.strideYB, h + (size_t)(p0 + b0) * sh.strideXB, nullptr,
                                 sh.nrowsB, min(sh.capB, nt - b0), iB * sh.wgB, p0 + b0};  // (tiles: the problem's first pair)
     }
-    __syncthreads();
-    const int nA = s_nA, nB = s_nB;
-    const int wgA = s_wgA;  // at most sh.wgA: the grid holds the problems' workgroups
-    for (int i = tid; i < sh.maxA * sh.wgA; i += blockDim.x) mapA[i] = i / wgA < nA ? i / wgA : -1;
+    for (int i = tid; i < sh.maxA * sh.wgA; i += blockDim.x) mapA[i] = i / wgA < nA ? i / wgA : -1;  // (wgA: at most sh.wgA, the grid holds the problems' workgroups)
     for (int i = tid; i < sh.maxB * sh.wgB; i += blockDim.x) mapB[i] = i / sh.wgB < nB ? i / sh.wgB : -1;
 }
 
