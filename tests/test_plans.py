@@ -1,0 +1,51 @@
+"""The rules by which the library chooses kernels, on the CPU: what they need is a matrix's format and sizes."""
+import ctypes as C
+import os
+import random
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+FORMATS = ("B32S4", "B32S8", "Q_G_4", "Q_G_8", "Q_8", "Q_G_3", "Q_G_2", "SB256A3", "SB256A2", "Q_4", "Q_G_6")
+ANY = (1 << 63) - 1  # scratch of any size
+SOLO = 4             # shape: tiles of 32 x 32
+
+
+class Plan(C.Structure):
+    _fields_ = [("shape", C.c_int), ("ksplit", C.c_int), ("rows", C.c_int), ("launches", C.c_int), ("us", C.c_double)]
+
+
+@pytest.fixture(scope="module")
+def drv(tfq):
+    tfq.lib()
+    path = os.path.join(ROOT, "tests", "libplan_driver.so")
+    if not os.path.exists(path):
+        pytest.fail("tests/libplan_driver.so is missing: run __graft_entry__.build()")
+    d = C.CDLL(path)
+    d.drv_gemm_exact_plans.argtypes = [C.c_int, C.c_int64, C.c_int64, C.c_int, C.c_int, C.c_size_t, C.c_int, C.c_int, C.POINTER(Plan), C.POINTER(Plan)]
+    d.drv_gemm_scratch_bytes.argtypes = [C.c_int, C.c_int64, C.c_int64, C.c_int, C.c_int]
+    d.drv_gemm_scratch_bytes.restype = C.c_size_t
+    return d
+
+
+def plans(tfq, drv, fmt, N, K, f32, M, scratch=ANY, matrices=1):
+    """(all plans of the integer tile kernel, the one that is taken)"""
+    buf, taken = (Plan * 128)(), Plan()
+    n = drv.drv_gemm_exact_plans(tfq.lib().tfq_format_id(fmt.encode()), N, K, tfq.F32 if f32 else tfq.BF16, M, scratch, matrices, 128, buf, taken)
+    assert 0 < n <= 128
+    return buf[:n], taken
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+def test_the_faster_plan_among_those_of_as_many_launches(tfq, drv, fmt):
+    """What the host takes for a call is its launches' alone, so no plan of as many is faster on the GPU than the one that is taken,
+    nor one of fewer: products of 5 to 300 rows of one matrix and of a pair, with any scratch, some and none."""
+    rng = random.Random(FORMATS.index(fmt))
+    for _ in range(400):
+        N, K, M = rng.randint(64, 6144), 256 * rng.randint(1, 60), rng.randint(5, 300)
+        for f32 in (False, True):
+            for scratch in (ANY, rng.randint(0, 1 << 22), 0):
+                for matrices in (1, 2) if fmt not in ("Q_4", "Q_G_6") else (1,):
+                    every, taken = plans(tfq, drv, fmt, N, K, f32, M, scratch, matrices)
+                    fewer = [p for p in every if p.launches <= taken.launches]
+                    assert min(p.us for p in fewer) == taken.us, (N, K, M, f32, scratch, matrices, taken.shape, taken.ksplit)

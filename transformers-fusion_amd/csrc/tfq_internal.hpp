@@ -504,6 +504,14 @@ size_t gemv_split_bytes(const tfq_weight* w);
 bool gemm_exact_serves(const tfq_weight* w, int M);
 size_t gemm_exact_scratch_bytes(const tfq_weight* w, int x_dtype, int M);
 double gemm_exact_us(const tfq_weight* w, int x_dtype, int M, size_t scratch_bytes, int matrices = 1, bool solo = true);
+// The plan of a product and all that it is chosen from: shape (4: tiles of 32 x 32, K over the wavefronts of a workgroup), parts
+// of K, rows of a run, launches of the call, a model of its time on the GPU (us)
+struct GemmExactPlan {
+    int shape, ksplit, rows, launches;
+    double us;
+};
+GemmExactPlan gemm_exact_plan(const tfq_weight* w, int x_dtype, int M, size_t scratch_bytes, int matrices = 1);
+std::vector<GemmExactPlan> gemm_exact_plans(const tfq_weight* w, int x_dtype, int M, size_t scratch_bytes, int matrices = 1);
 int launch_gemm_exact(const tfq_weight* w, const void* x, int x_dtype, int M, void* y, int y_dtype, hipStream_t s, void* scratch,
                       size_t scratch_bytes, bool keep_split = false);
 // Its pair form, y = silu(w x) * (w2 x), and its grouped form: rows first[e] to first[e + 1] (device array) of x and y go with
