@@ -49,3 +49,18 @@ def test_the_faster_plan_among_those_of_as_many_launches(tfq, drv, fmt):
                     every, taken = plans(tfq, drv, fmt, N, K, f32, M, scratch, matrices)
                     fewer = [p for p in every if p.launches <= taken.launches]
                     assert min(p.us for p in fewer) == taken.us, (N, K, M, f32, scratch, matrices, taken.shape, taken.ksplit)
+
+
+@pytest.mark.parametrize("fmt,N,K,f32,M,launches", [
+    ("B32S8", 289, 3840, False, 29, 2),    # us a call, and in a graph: one launch 8.8 and 8.7, two 7.9 and 7.0
+    ("Q_G_3", 444, 1792, True, 82, 2),     # 8.9 and 8.9, 8.4 and 8.0
+    ("Q_G_2", 1472, 2560, False, 20, 2),   # 9.2 and 9.2, 7.9 and 7.4
+    ("Q_4", 306, 2048, False, 71, 2),      # 9.0 and 9.0, 7.9 and 7.3
+    ("Q_8", 256, 4096, False, 21, 2),      # 9.3 and 9.2, 8.0 and 6.8
+    ("B32S4", 1075, 1792, True, 20, 1),    # 7.7 and 7.7, 8.1 and 6.8
+    ("B32S4", 320, 1024, False, 20, 1),    # 5.2 and 5.1, 7.8 and 6.2
+    ("SB256A2", 1536, 1792, False, 18, 1),  # 7.7 and 7.7, 7.7 and 7.3
+])
+def test_a_second_launch_where_it_saves_the_call_time(tfq, drv, fmt, N, K, f32, M, launches):
+    """A second launch is taken where it makes the call shorter: two take the host 7.6 to 8.0 us."""
+    assert plans(tfq, drv, fmt, N, K, f32, M)[1].launches == launches
