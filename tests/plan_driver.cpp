@@ -36,4 +36,11 @@ size_t drv_gemm_scratch_bytes(int fmt, int64_t N, int64_t K, int x_dtype, int M)
     return tfq::gemm_scratch_bytes(&w, x_dtype, M);
 }
 
+// one to sixteen rows: what serves best, and what the decode kernels alone use
+size_t drv_gemv_rows_scratch_bytes(int fmt, int64_t N, int64_t K, int x_dtype, int B, size_t* decode) {
+    const tfq_weight w = matrix(fmt, N, K);
+    *decode = tfq::gemv_split_bytes(&w);
+    return tfq::gemv_rows_scratch_bytes(&w, x_dtype, B);
+}
+
 }  // extern "C"

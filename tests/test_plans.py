@@ -25,6 +25,8 @@ def drv(tfq):
     d.drv_gemm_exact_plans.argtypes = [C.c_int, C.c_int64, C.c_int64, C.c_int, C.c_int, C.c_size_t, C.c_int, C.c_int, C.POINTER(Plan), C.POINTER(Plan)]
     d.drv_gemm_scratch_bytes.argtypes = [C.c_int, C.c_int64, C.c_int64, C.c_int, C.c_int]
     d.drv_gemm_scratch_bytes.restype = C.c_size_t
+    d.drv_gemv_rows_scratch_bytes.argtypes = [C.c_int, C.c_int64, C.c_int64, C.c_int, C.c_int, C.POINTER(C.c_size_t)]
+    d.drv_gemv_rows_scratch_bytes.restype = C.c_size_t
     return d
 
 
@@ -64,3 +66,30 @@ def test_the_faster_plan_among_those_of_as_many_launches(tfq, drv, fmt):
 def test_a_second_launch_where_it_saves_the_call_time(tfq, drv, fmt, N, K, f32, M, launches):
     """A second launch is taken where it makes the call shorter: two take the host 7.6 to 8.0 us."""
     assert plans(tfq, drv, fmt, N, K, f32, M)[1].launches == launches
+
+
+@pytest.mark.parametrize("fmt,N,K,f32,B,tiles", [
+    ("SB256A2", 1318, 2304, True, 5, True),    # us in a graph: decode kernels 10.1, integer tile kernel 7.3
+    ("SB256A3", 1152, 1280, True, 8, True),    # 9.4, 7.1
+    ("Q_G_3", 1088, 3840, False, 11, True),    # 9.4, 7.5
+    ("Q_4", 1536, 1024, True, 8, True),        # 9.0, 6.6
+    ("Q_G_3", 1466, 1536, True, 6, True),      # 8.2, 7.7
+    ("Q_G_3", 1152, 1536, True, 7, True),      # 8.7, 7.3
+    ("Q_G_2", 1216, 2304, False, 10, True),    # 8.2, 7.3
+    ("B32S8", 512, 6400, True, 8, True),       # 9.4, 8.0
+    ("B32S4", 1024, 8192, True, 7, True),      # 9.0, 7.8
+    ("B32S4", 432, 8448, True, 7, False),      # 8.0, 8.9
+    ("Q_8", 384, 8448, True, 7, False),        # 8.8, 9.4
+    ("B32S4", 576, 8960, True, 5, False),      # 8.1, 9.0
+    ("SB256A3", 14336, 4096, False, 8, False),  # 13, 18
+    ("Q_G_4", 14336, 4096, True, 16, True),    # 25, 22
+])
+def test_five_to_sixteen_rows_by_the_gpu_time_of_both_kernels(tfq, drv, fmt, N, K, f32, B, tiles):
+    """The decode kernels and the integer tile kernel are compared by their times on the GPU, whatever the launches: seen by the
+    scratch that is asked for, which is what the kernel that serves uses."""
+    dt, fid, decode = tfq.F32 if f32 else tfq.BF16, tfq.lib().tfq_format_id(fmt.encode()), C.c_size_t()
+    need = drv.drv_gemv_rows_scratch_bytes(fid, N, K, dt, B, C.byref(decode))
+    plan = plans(tfq, drv, fmt, N, K, f32, B)[1]
+    parts = 4 * plan.ksplit * B * N if plan.ksplit > 1 else 0
+    assert parts != decode.value  # (else the scratch would not tell)
+    assert need == (max(decode.value, parts) if tiles else decode.value)

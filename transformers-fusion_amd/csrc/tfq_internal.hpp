@@ -500,7 +500,8 @@ int launch_gemv_rows(const tfq_weight* w, const void* x, int x_dtype, int B, voi
 size_t gemv_rows_scratch_bytes(const tfq_weight* w, int x_dtype, int B);
 size_t gemv_split_bytes(const tfq_weight* w);
 // The tile kernel with integer operands (tfq_gemm_exact.hip), reached through launch_gemm: products that may not round
-// their weights.  Any scratch size is served (less scratch, fewer K parts); gemm_exact_us says how long it would take.
+// their weights.  Any scratch size is served (less scratch, fewer K parts); gemm_exact_us says how long it would take
+// on the GPU, like the models of the other kernels that it is compared with.
 bool gemm_exact_serves(const tfq_weight* w, int M);
 size_t gemm_exact_scratch_bytes(const tfq_weight* w, int x_dtype, int M);
 double gemm_exact_us(const tfq_weight* w, int x_dtype, int M, size_t scratch_bytes, int matrices = 1, bool solo = true);
