@@ -31,9 +31,20 @@ int drv_gemm_exact_plans(int fmt, int64_t N, int64_t K, int x_dtype, int M, size
     return (int)v.size();
 }
 
+int drv_gemm_takes_exact(int fmt, int64_t N, int64_t K, int x_dtype, int M, size_t scratch) {
+    const tfq_weight w = matrix(fmt, N, K);
+    return tfq::gemm_takes_exact(&w, x_dtype, M, scratch);
+}
+
 size_t drv_gemm_scratch_bytes(int fmt, int64_t N, int64_t K, int x_dtype, int M) {
     const tfq_weight w = matrix(fmt, N, K);
     return tfq::gemm_scratch_bytes(&w, x_dtype, M);
+}
+
+// whether tfq_mlp_step of these sizes has gate and up in one launch of the integer tile kernel
+int drv_mlp_pairs(int fmt, int64_t N, int64_t K, int x_dtype, int M) {
+    const tfq_weight w = matrix(fmt, N, K);
+    return M > 4 && tfq::gemm_exact_pair_serves(&w, &w, x_dtype, M) && tfq::gemm_pair_pays(&w, x_dtype, M);
 }
 
 // one to sixteen rows: what serves best, and what the decode kernels alone use

@@ -228,6 +228,30 @@ def test_gemm_small_products_in_one_launch(tfq, gpu, fmt, dtype, N, K):
     W.close()
 
 
+@pytest.mark.parametrize("fmt", ["B32S4", "B32S8", "Q_G_4", "Q_G_8", "Q_8", "Q_G_3", "Q_G_2", "SB256A3", "SB256A2", "Q_4", "Q_G_6"])
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+def test_gemm_small_products_longest_walk(tfq, gpu, rules, fmt, dtype):
+    """Four steps of every wavefront over its LDS, each written by some lanes and read by others: the longest K in one part, which
+    a call without scratch has, of ragged tiles.  Bounds as above; a row does not depend on those beside it, the whole tile's."""
+    import torch
+    N, K = 2017, 3072 if fmt in ("Q_4", "Q_G_6") and dtype == "f32" else 4096
+    print(f"gemm longest walk {fmt} {dtype} N={N} K={K}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(32)
+    W = tfq.Weight(fmt, N, K, tfq.encode(fmt, torch.randn(N * K, device=gpu, generator=g) * 0.02))
+    dense = W.decode().reshape(N, K).double()
+    bound = 1.5e-4 if fmt in ("Q_G_8", "Q_8") else 1e-6 if dtype == "bf16" or fmt in ("Q_4", "Q_G_6") else 1e-5
+    for M in (50, 95):
+        plan = rules.product(fmt, N, K, dtype == "f32", M, scratch=0)
+        assert (plan.shape, plan.ksplit) == (rules.SOLO, 1)
+        x = torch.randn(M, K, device=gpu, generator=g)
+        x = x.bfloat16() if dtype == "bf16" else x
+        want = x.double() @ dense.T
+        y = W.gemm(x, out_dtype=torch.float32, workspace=False)
+        assert float((y.double() - want).norm() / want.norm()) <= bound, M
+        assert torch.equal(W.gemm(x.flip(0).contiguous(), out_dtype=torch.float32, workspace=False), y.flip(0)), M
+    W.close()
+
+
 @pytest.mark.parametrize("fmt,dtype", [("B32S4", "bf16"), ("Q_G_4", "f32"), ("Q_G_8", "bf16"), ("SB256A3", "f32"), ("Q_4", "f32"), ("Q_G_6", "bf16")])
 @pytest.mark.parametrize("N,K", [(96, 4608), (320, 6400), (65, 14336), (1, 15872)])
 def test_gemm_small_products_in_k_parts(tfq, gpu, fmt, dtype, N, K):

@@ -1,54 +1,22 @@
 """The rules by which the library chooses kernels, on the CPU: what they need is a matrix's format and sizes."""
-import ctypes as C
-import os
 import random
 
 import pytest
 
-ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 FORMATS = ("B32S4", "B32S8", "Q_G_4", "Q_G_8", "Q_8", "Q_G_3", "Q_G_2", "SB256A3", "SB256A2", "Q_4", "Q_G_6")
-ANY = (1 << 63) - 1  # scratch of any size
-SOLO = 4             # shape: tiles of 32 x 32
-
-
-class Plan(C.Structure):
-    _fields_ = [("shape", C.c_int), ("ksplit", C.c_int), ("rows", C.c_int), ("launches", C.c_int), ("us", C.c_double)]
-
-
-@pytest.fixture(scope="module")
-def drv(tfq):
-    tfq.lib()
-    path = os.path.join(ROOT, "tests", "libplan_driver.so")
-    if not os.path.exists(path):
-        pytest.fail("tests/libplan_driver.so is missing: run __graft_entry__.build()")
-    d = C.CDLL(path)
-    d.drv_gemm_exact_plans.argtypes = [C.c_int, C.c_int64, C.c_int64, C.c_int, C.c_int, C.c_size_t, C.c_int, C.c_int, C.POINTER(Plan), C.POINTER(Plan)]
-    d.drv_gemm_scratch_bytes.argtypes = [C.c_int, C.c_int64, C.c_int64, C.c_int, C.c_int]
-    d.drv_gemm_scratch_bytes.restype = C.c_size_t
-    d.drv_gemv_rows_scratch_bytes.argtypes = [C.c_int, C.c_int64, C.c_int64, C.c_int, C.c_int, C.POINTER(C.c_size_t)]
-    d.drv_gemv_rows_scratch_bytes.restype = C.c_size_t
-    return d
-
-
-def plans(tfq, drv, fmt, N, K, f32, M, scratch=ANY, matrices=1):
-    """(all plans of the integer tile kernel, the one that is taken)"""
-    buf, taken = (Plan * 128)(), Plan()
-    n = drv.drv_gemm_exact_plans(tfq.lib().tfq_format_id(fmt.encode()), N, K, tfq.F32 if f32 else tfq.BF16, M, scratch, matrices, 128, buf, taken)
-    assert 0 < n <= 128
-    return buf[:n], taken
 
 
 @pytest.mark.parametrize("fmt", FORMATS)
-def test_the_faster_plan_among_those_of_as_many_launches(tfq, drv, fmt):
+def test_the_faster_plan_among_those_of_as_many_launches(rules, fmt):
     """What the host takes for a call is its launches' alone, so no plan of as many is faster on the GPU than the one that is taken,
     nor one of fewer: products of 5 to 300 rows of one matrix and of a pair, with any scratch, some and none."""
     rng = random.Random(FORMATS.index(fmt))
     for _ in range(400):
         N, K, M = rng.randint(64, 6144), 256 * rng.randint(1, 60), rng.randint(5, 300)
         for f32 in (False, True):
-            for scratch in (ANY, rng.randint(0, 1 << 22), 0):
+            for scratch in (rules.ANY, rng.randint(0, 1 << 22), 0):
                 for matrices in (1, 2) if fmt not in ("Q_4", "Q_G_6") else (1,):
-                    every, taken = plans(tfq, drv, fmt, N, K, f32, M, scratch, matrices)
+                    every, taken = rules.plans(fmt, N, K, f32, M, scratch, matrices)
                     fewer = [p for p in every if p.launches <= taken.launches]
                     assert min(p.us for p in fewer) == taken.us, (N, K, M, f32, scratch, matrices, taken.shape, taken.ksplit)
 
@@ -63,9 +31,9 @@ def test_the_faster_plan_among_those_of_as_many_launches(tfq, drv, fmt):
     ("B32S4", 320, 1024, False, 20, 1),    # 5.2 and 5.1, 7.8 and 6.2
     ("SB256A2", 1536, 1792, False, 18, 1),  # 7.7 and 7.7, 7.7 and 7.3
 ])
-def test_a_second_launch_where_it_saves_the_call_time(tfq, drv, fmt, N, K, f32, M, launches):
+def test_a_second_launch_where_it_saves_the_call_time(rules, fmt, N, K, f32, M, launches):
     """A second launch is taken where it makes the call shorter: two take the host 7.6 to 8.0 us."""
-    assert plans(tfq, drv, fmt, N, K, f32, M)[1].launches == launches
+    assert rules.plans(fmt, N, K, f32, M)[1].launches == launches
 
 
 @pytest.mark.parametrize("fmt,N,K,f32,B,tiles", [
@@ -84,12 +52,11 @@ def test_a_second_launch_where_it_saves_the_call_time(tfq, drv, fmt, N, K, f32, 
     ("SB256A3", 14336, 4096, False, 8, False),  # 13, 18
     ("Q_G_4", 14336, 4096, True, 16, True),    # 25, 22
 ])
-def test_five_to_sixteen_rows_by_the_gpu_time_of_both_kernels(tfq, drv, fmt, N, K, f32, B, tiles):
+def test_five_to_sixteen_rows_by_the_gpu_time_of_both_kernels(rules, fmt, N, K, f32, B, tiles):
     """The decode kernels and the integer tile kernel are compared by their times on the GPU, whatever the launches: seen by the
     scratch that is asked for, which is what the kernel that serves uses."""
-    dt, fid, decode = tfq.F32 if f32 else tfq.BF16, tfq.lib().tfq_format_id(fmt.encode()), C.c_size_t()
-    need = drv.drv_gemv_rows_scratch_bytes(fid, N, K, dt, B, C.byref(decode))
-    plan = plans(tfq, drv, fmt, N, K, f32, B)[1]
+    need, decode = rules.rows_scratch(fmt, N, K, f32, B)
+    plan = rules.plans(fmt, N, K, f32, B)[1]
     parts = 4 * plan.ksplit * B * N if plan.ksplit > 1 else 0
-    assert parts != decode.value  # (else the scratch would not tell)
-    assert need == (max(decode.value, parts) if tiles else decode.value)
+    assert parts != decode  # (else the scratch would not tell)
+    assert need == (max(decode, parts) if tiles else decode)

@@ -512,6 +512,7 @@ struct GemmExactPlan {
     double us;
 };
 GemmExactPlan gemm_exact_plan(const tfq_weight* w, int x_dtype, int M, size_t scratch_bytes, int matrices = 1);
+bool gemm_takes_exact(const tfq_weight* w, int x_dtype, int M, size_t scratch_bytes);  // whether a call of tfq_gemm_ws, or tfq_gemv_ws, goes there
 std::vector<GemmExactPlan> gemm_exact_plans(const tfq_weight* w, int x_dtype, int M, size_t scratch_bytes, int matrices = 1);
 int launch_gemm_exact(const tfq_weight* w, const void* x, int x_dtype, int M, void* y, int y_dtype, hipStream_t s, void* scratch,
                       size_t scratch_bytes, bool keep_split = false);
