@@ -207,24 +207,29 @@ def test_gemm_integer_operands_any_scratch(tfq, gpu, fmt, dtype, M, N, K):
 
 @pytest.mark.parametrize("fmt,dtype", EXACT_FMTS + [(f, "bf16") for f in ("Q_G_4", "Q_G_3", "B32S4", "B32S8", "Q_G_8", "Q_8")])
 @pytest.mark.parametrize("N,K", [(1, 256), (31, 896 + 128), (33, 1280), (200, 2816), (65, 4096), (96, 4352)])
-def test_gemm_small_products_in_one_launch(tfq, gpu, fmt, dtype, N, K):
-    """K over the wavefronts of a workgroup: fewer half blocks than wavefronts, shares of different sizes, the longest K that
-    is served and the next one; ragged tiles on either side.  Against the float64 product, the bounds of
+def test_gemm_small_products_in_one_launch(tfq, gpu, rules, fmt, dtype, N, K):
+    """Tiles of 32 x 32, K over the wavefronts of a workgroup: fewer half blocks than wavefronts, shares of different sizes, ragged
+    tiles on either side.  With the workspace that is asked for the first three sizes are mostly one launch, the others K parts of
+    such tiles; without it all that are served there are one launch.  Against the float64 product, the bounds of
     test_gemm_integer_operands_any_scratch (the bf16 rows' weights are not rounded either); a row's sums do not depend on
     the tile that it is in, nor on the rows beside it."""
     import torch
     g = torch.Generator(device="cuda").manual_seed(31)
     W = tfq.Weight(fmt, N, K, tfq.encode(fmt, torch.randn(N * K, device=gpu, generator=g) * 0.02))
     dense = W.decode().reshape(N, K).double()
-    bound = 1.5e-4 if fmt in ("Q_G_8", "Q_8") else 1e-6 if dtype == "bf16" or fmt in ("Q_4", "Q_G_6") else 1e-5
+    bound = 1.5e-4 if fmt in ("Q_G_8", "Q_8") else 1e-6 if dtype == "bf16" or fmt in ("Q_4", "Q_4_K_H", "Q_G_6") else 1e-5
     x = torch.randn(95, K, device=gpu, generator=g)
     x = x.bfloat16() if dtype == "bf16" else x
     want = x.double() @ dense.T
     for M in (17, 32, 33, 95):
-        y = W.gemm(x[:M].contiguous(), out_dtype=torch.float32)
-        assert float((y.double() - want[:M]).norm() / want[:M].norm()) <= bound, (fmt, dtype, N, K, M)
-        if 1024 <= K <= 2816:  # (every count of rows takes this kernel, in one part of K or in several)
-            assert torch.equal(W.gemm(x[:M].flip(0).contiguous(), out_dtype=torch.float32), y.flip(0))
+        for workspace in (True, False):
+            plan = rules.product(fmt, N, K, dtype == "f32", M, None if workspace else 0)
+            if not workspace and (plan is None or plan.shape != rules.SOLO):
+                continue  # (other kernels' rows)
+            assert plan.shape == rules.SOLO and (workspace or plan.ksplit == 1)
+            y = W.gemm(x[:M].contiguous(), out_dtype=torch.float32, workspace=workspace)
+            assert float((y.double() - want[:M]).norm() / want[:M].norm()) <= bound, (fmt, dtype, N, K, M)
+            assert torch.equal(W.gemm(x[:M].flip(0).contiguous(), out_dtype=torch.float32, workspace=workspace), y.flip(0))
     W.close()
 
 
@@ -255,9 +260,8 @@ def test_gemm_small_products_longest_walk(tfq, gpu, rules, fmt, dtype):
 @pytest.mark.parametrize("fmt,dtype", [("B32S4", "bf16"), ("Q_G_4", "f32"), ("Q_G_8", "bf16"), ("SB256A3", "f32"), ("Q_4", "f32"), ("Q_G_6", "bf16")])
 @pytest.mark.parametrize("N,K", [(96, 4608), (320, 6400), (65, 14336), (1, 15872)])
 def test_gemm_small_products_in_k_parts(tfq, gpu, fmt, dtype, N, K):
-    """Few tiles of a long K: parts of K over workgroups (of unequal length where the blocks do not divide), up to more of them than
-    one batch of the launch that adds them loads.  Rows of a tile and of the next one, one to sixteen rows (gemv) and more.  The
-    bounds of test_gemm_integer_operands_any_scratch; a feed-forward's pair of matrices in parts against two products."""
+    """Few tiles of a long K: eight parts of K over workgroups, of unequal length where the blocks do not divide.  Rows of a tile and of
+    the next one, one to sixteen rows (gemv) and more.  The bounds of test_gemm_integer_operands_any_scratch."""
     import torch
     print(f"gemm k parts {fmt} {dtype} N={N} K={K}", flush=True)
     g = torch.Generator(device="cuda").manual_seed(33)
@@ -270,6 +274,27 @@ def test_gemm_small_products_in_k_parts(tfq, gpu, fmt, dtype, N, K):
         want = x.double() @ dense.T
         y = W.gemv(x) if M <= 16 else W.gemm(x, out_dtype=torch.float32)
         assert float((y.double() - want).norm() / want.norm()) <= bound, (M, float((y.double() - want).norm() / want.norm()))
+    W.close()
+
+
+@pytest.mark.parametrize("fmt,dtype,M,N,K,shape,parts", [
+    ("Q_G_3", "f32", 241, 399, 2304, 4, 2), ("B32S8", "f32", 233, 294, 1792, 4, 3), ("SB256A3", "f32", 161, 53, 1536, 4, 6), ("Q_G_6", "f32", 18, 34, 1792, 4, 7),
+    ("SB256A2", "f32", 208, 329, 2816, 3, 11), ("Q_G_4", "f32", 206, 228, 6912, 3, 14), ("B32S4", "f32", 228, 222, 8192, 3, 16), ("Q_4", "bf16", 241, 212, 7936, 3, 16),
+    ("Q_G_8", "bf16", 232, 528, 7936, 2, 11), ("Q_G_6", "bf16", 231, 404, 7936, 2, 16)])
+def test_gemm_k_parts_of_every_count(tfq, gpu, rules, fmt, dtype, M, N, K, shape, parts):
+    """K parts in counts of two to sixteen: one batch of the loads of the launch that adds them, a whole and a ragged second one.
+    (Bounds as above.)"""
+    import torch
+    plan = rules.product(fmt, N, K, dtype == "f32", M)
+    assert (plan.shape, plan.ksplit) == (shape, parts)
+    g = torch.Generator(device="cuda").manual_seed(34)
+    W = tfq.Weight(fmt, N, K, tfq.encode(fmt, torch.randn(N * K, device=gpu, generator=g) * 0.02))
+    bound = 1.5e-4 if fmt == "Q_G_8" else 1e-6 if dtype == "bf16" or fmt in ("Q_4", "Q_G_6") else 1e-5
+    x = torch.randn(M, K, device=gpu, generator=g)
+    x = x.bfloat16() if dtype == "bf16" else x
+    want = x.double() @ W.decode().reshape(N, K).double().T
+    y = W.gemm(x, out_dtype=torch.float32)
+    assert float((y.double() - want).norm() / want.norm()) <= bound
     W.close()
 
 

@@ -112,6 +112,27 @@ def test_router_one_launch_or_two(tfq, gpu, E, T):
         assert all(torch.equal(a[t:t + 1], b) for a, b in zip(got, alone))
 
 
+@pytest.mark.parametrize("E", [1, 2, 4, 5, 7, 8, 9])
+def test_router_of_few_experts_ties(tfq, gpu, E):
+    """Up to eight experts meet over eight lanes, one more over all: every k up to E, rows of the router repeated so that logits and
+    probabilities tie exactly, all of them in one token.  Probabilities, picks and weights are, bit for bit, tfq_moe_route's
+    of the logits (which has the general form), and the picks are in order, the lower index first among equals."""
+    import torch
+    T, D = 37, 1088
+    gen = torch.Generator().manual_seed(E)
+    x = torch.randn(T, D, generator=gen).to(gpu)
+    x[3] = 0.0
+    Wr = (torch.randn(E, D, generator=gen) * 0.05).to(gpu)
+    Wr[1::2] = Wr[0::2][:E // 2]
+    for k in range(1, E + 1):
+        logits, probs, idx, w = tfq.moe_router(x, Wr, k)
+        assert torch.equal(logits[:, 1::2], logits[:, 0::2][:, :E // 2])
+        for a, b in zip((probs, idx, w), tfq.moe_route(logits, k)):
+            assert torch.equal(a, b), k
+        order = [sorted(range(E), key=lambda e: (-p[e], e))[:k] for p in probs.cpu().tolist()]
+        assert idx.cpu().tolist() == order
+
+
 def _experts(O, tfq, fmt, E, D, F, seed):
     gate, up, down, hg, hu, hd = [], [], [], [], [], []
     for e in range(E):
@@ -678,14 +699,22 @@ def test_moe_ffn_grouped_tiles(O, tfq, gpu, fmt, counts, D, F):
         W.close()
 
 
-@pytest.mark.parametrize("fmt,B,D,F,xdt,mid", [
-    ("B32S4", 9, 512, 8448, "f32", "f32"),     # below seventeen rows: K parts of the pair in the workspace
-    ("Q_G_8", 16, 768, 4352, "f32", "f32"),
-    ("Q_G_4", 33, 512, 768, "bf16", "bf16"),
-    ("SB256A3", 65, 256, 1280, "f32", "bf16"),
-    ("B32S8", 129, 768, 512, "f32", "f32"),    # activations split beforehand
+@pytest.mark.parametrize("fmt,B,D,F,xdt,mid,plan", [  # plan: shape (4: 32 x 32 tiles, 1: activations split beforehand) and K parts of the pair
+    ("B32S4", 9, 512, 8448, "f32", "f32", (3, 1)),
+    ("Q_G_8", 16, 768, 4352, "f32", "f32", (4, 1)),
+    ("Q_G_4", 33, 512, 768, "bf16", "bf16", (4, 1)),
+    ("SB256A3", 65, 256, 1280, "f32", "bf16", (4, 1)),
+    ("B32S8", 129, 768, 512, "f32", "f32", (4, 1)),
+    ("B32S4", 9, 4096, 768, "f32", "f32", (4, 5)),      # (with the least workspace in one part of another shape)
+    ("Q_G_3", 16, 2304, 512, "f32", "f32", (4, 5)),     # parts of one and two blocks
+    ("Q_G_8", 32, 6400, 256, "bf16", "bf16", (4, 5)),
+    ("Q_G_4", 33, 3072, 512, "bf16", "f32", (4, 5)),
+    ("SB256A3", 20, 4352, 256, "f32", "f32", (4, 5)),
+    ("Q_G_2", 40, 2560, 1024, "bf16", "bf16", (3, 5)),
+    ("B32S8", 130, 2560, 1792, "bf16", "bf16", (1, 5)),
+    ("Q_G_4", 259, 1536, 2048, "f32", "f32", (1, 3)),
 ])
-def test_mlp_step_pair_on_integer_operands(O, tfq, gpu, fmt, B, D, F, xdt, mid):
+def test_mlp_step_pair_on_integer_operands(O, tfq, gpu, rules, fmt, B, D, F, xdt, mid, plan):
     """gate and up in one launch of the integer tile kernel, whole and in K parts: against the float64 products of the
     decoded matrices (the companded line 3e-4, bf16 mid activations 5e-3, otherwise 3e-5 as above); a buffer behind the
     workspace stays as it was."""
@@ -704,6 +733,8 @@ def test_mlp_step_pair_on_integer_operands(O, tfq, gpu, fmt, B, D, F, xdt, mid):
     L = tfq.lib()
     part = (B * F * 4 + 255) // 256 * 256
     least = 3 * part + (min(8 * B * F * 4, 256 * 256 * 256 * 4) + 255) // 256 * 256 * (B > 16)
+    taken = rules.pair(fmt, F, D, xdt == "f32", B, L.tfq_mlp_workspace_bytes(B, F) - part)
+    assert (taken.shape, taken.ksplit) == plan
     for size in (L.tfq_mlp_workspace_bytes(B, F), least):
         buf = torch.full((size + 4096,), 77, device=gpu, dtype=torch.uint8)
         y = torch.empty(B, D, device=gpu)
