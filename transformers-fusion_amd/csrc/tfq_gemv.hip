@@ -1292,8 +1292,8 @@ __global__ __launch_bounds__(1024) void gemvb_kernel(GemvKernArgs args, const un
 // them).  fp32 rows are two adjacent slots each, added first like the unsplit kernel adds them.  (The parts used
 // to meet inside the kernel: device-scope stores, an arrival counter per row group, the last arriver reading all
 // parts back.  That chain of dependent memory round trips cost 6 us of a 17 us launch, 4096 x 14336 at sixteen
-// rows; this kernel and its launch boundary cost 3.5 us, and some 0.7 less since the parts' loads are under way together: that
-// product 15.1 -> 14.3 us.)
+// rows; this kernel and its launch boundary cost 3.5 us, and some 0.8 less since the parts' loads are under way together: that
+// product, in a graph over matrices that no cache holds, Q_G_4 15.1 -> 14.3 us, B32S4 13.9 -> 13.1.)
 __global__ __launch_bounds__(256) void split_reduce_kernel(const float* __restrict__ partial, void* __restrict__ y, int kparts, int B,
                                                           int nrm, int y_bf16, int x_f32) {
     const int row = blockIdx.x * 256 + threadIdx.x, b = blockIdx.y;  // one output per lane
