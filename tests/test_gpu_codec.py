@@ -209,6 +209,9 @@ def test_iterative_encoders_many_blocks(O, tfq, gpu, fmt):
     bb = O.block_bytes(fmt)
     bad = np.nonzero((got.reshape(-1, bb) != want.reshape(-1, bb)).any(1))[0]
     assert bad.size == 0, f"{bad.size} of {w.size // 256} blocks differ, first {bad[:5]}"
+    if fmt in ("Q_G_4", "Q_G_3", "Q_G_2", "SB256A3", "SB256A2"):  # (another kernel above 24576 blocks)
+        lot = tfq.encode(fmt, torch.from_numpy(w).to(gpu).repeat(4)).reshape(4, -1)
+        assert bool((lot == torch.from_numpy(want.reshape(-1)).to(gpu)).all())
 
 
 @pytest.mark.parametrize("fmt", ["Q_G_4", "Q_G_3", "Q_G_2", "SB256A3", "Q_1_5", "Q_G_8", "Q_8", "Q_4", "Q_3", "Q_6"])
@@ -235,12 +238,13 @@ def test_iterative_encoders_where_fast_arithmetic_ends(O, tfq, gpu, fmt):
     got = tfq.encode(fmt, torch.from_numpy(w.reshape(-1)).to(gpu)).cpu().numpy().reshape(-1, bb)
     bad = np.nonzero((got != want).any(1))[0]
     assert bad.size == 0, f"{bad.size} of {len(w)} blocks differ, first {bad[:8]}"
-    many = torch.from_numpy(w).to(gpu).repeat(9000 // len(w) + 1, 1)
-    big = tfq.encode(fmt, many.reshape(-1)).reshape(-1, len(w), bb)
-    assert bool((big == torch.from_numpy(want).to(gpu)).all())
     few = tfq.encode(fmt, torch.from_numpy(odd.reshape(-1)).to(gpu))
-    lot = tfq.encode(fmt, torch.from_numpy(odd).to(gpu).repeat(1500, 1).reshape(-1)).reshape(-1, few.numel())
-    assert bool((lot == few).all())
+    for blocks in (9000, 25000):  # (the affine formats have another kernel above 24576)
+        many = torch.from_numpy(w).to(gpu).repeat(blocks // len(w) + 1, 1)
+        big = tfq.encode(fmt, many.reshape(-1)).reshape(-1, len(w), bb)
+        assert bool((big == torch.from_numpy(want).to(gpu)).all()), blocks
+        lot = tfq.encode(fmt, torch.from_numpy(odd).to(gpu).repeat(blocks // len(odd), 1).reshape(-1)).reshape(-1, few.numel())
+        assert bool((lot == few).all()), blocks
 
 
 @pytest.mark.parametrize("fmt", ["Q_G_4", "Q_G_2", "Q_G_3", "SB256A2", "SB256A3"])
@@ -269,6 +273,41 @@ def test_affine_encoders_two_kernels_agree(O, tfq, gpu, fmt):
     general = torch.cat(parts)
     for size in (24576, 24577, 24578, 24584, n):
         assert torch.equal(tfq.encode(fmt, w[:size].reshape(-1)).reshape(-1, bb), general[:size]), size
+
+
+@pytest.mark.parametrize("fmt", ["Q_G_4", "Q_G_3", "Q_G_2", "SB256A2", "SB256A3"])
+def test_affine_encoder_groups_with_offsets_of_their_own(O, tfq, gpu, fmt):
+    """Groups whose spread is small against how far their offsets lie apart: in the first refinement many have one level for all of
+    their weights, so that s and m stay the ones of the group fit, whose sums hold the exact squares of the levels and not, as
+    a refinement's, their float products.  The blocks of offset_groups.npz (per format those of some 400000 such blocks,
+    normal offsets and spreads, whose payload changed where a refinement's sums stood in for the fit's) against the oracle; 150000 random
+    ones, and ones with an outlier a group, against calls of up to 24576 blocks, which take double sums in every pass.
+    Every wavefront holds copies of one block: one that holds several takes the double sums for all of them wherever one does."""
+    import torch
+    print(f"encode offsets {fmt}", flush=True)
+    bb, ng = O.block_bytes(fmt), 8 if fmt in ("Q_G_4", "Q_G_3") else 16
+    gsz, copies = 256 // ng, 64 // ng
+    found = np.load(os.path.join(G, "offset_groups.npz"))
+    for w in found[fmt] if fmt in found.files else ():
+        want = torch.from_numpy(O.encode_tensor(fmt, w)).to(gpu)
+        got = tfq.encode(fmt, torch.from_numpy(w).to(gpu).repeat(24584)).reshape(-1, bb)
+        assert bool((got == want).all()), (got[0] != want).nonzero().flatten().tolist()
+    g = torch.Generator(device="cuda")
+    g.manual_seed(31)
+    n = 24576
+    u = lambda lo, hi: torch.pow(2.0, torch.rand(n, 1, 1, device=gpu, generator=g) * (hi - lo) + lo)
+    for kind in ("spread", "spread", "spread", "narrow", "outlier", "outlier"):
+        a = u(-4, -1) if kind == "spread" else 0.03
+        b = a * u(-8, -3) if kind == "spread" else 0.03 * u(-9, -6) if kind == "narrow" else 2e-4
+        w = torch.randn(n, ng, 1, device=gpu, generator=g) * a + torch.randn(n, ng, gsz, device=gpu, generator=g) * b
+        if kind == "outlier":
+            at = torch.randint(0, gsz, (n, ng, 1), device=gpu, generator=g)
+            w.scatter_add_(2, at, torch.randn(n, ng, 1, device=gpu, generator=g) * 0.03)
+        w = w.reshape(n, 256)
+        general = tfq.encode(fmt, w.reshape(-1)).reshape(n, 1, bb)
+        many = tfq.encode(fmt, w.repeat_interleave(copies, 0).reshape(-1)).reshape(n, copies, bb)
+        bad = (many != general).any(2).any(1).nonzero().flatten().tolist()
+        assert not bad, (kind, len(bad), bad[:8])
 
 
 MIX_FORMATS = ["Q_MX_3_5", "Q_MX_4_5", "Q_MX_6_5", "Q_MX_8_5", "Q_MX_12_5", "Q_MX_16_5", "Q_MX_24_5",

@@ -416,11 +416,14 @@ __global__ __launch_bounds__(64, 4) void encode_affine_kernel(const float* __res
     struct Blocks {
         uint4 planes[gsz == 32 ? 4 : 0][quads / 4][64];  // the weights as integers X
         union {
-            float2 sums[2][64];  // (value, its integer code) of every group: scales, and offsets with their sign turned
-            float errors[6][64];
+            float errors[6][64];  // of the fit
+            struct {              // of what follows
+                float2 sums[2][64];  // (value, its integer code) of every group: scales, and offsets with their sign turned
+                double2 joint_level[1 << bits];  // a level, and its square as the refinements have it, a float product
+            };
         };
         uint8_t hcode[128];
-        double2 level[1 << bits];  // a level n * unit, and its square as a float product
+        double2 level[1 << bits];  // a level n * unit, and its exact square
     };
     // (one or the other: together they would leave room for fewer wavefronts per SIMD)
     __shared__ union { Team team; Blocks blocks; } lds;
@@ -431,8 +434,10 @@ __global__ __launch_bounds__(64, 4) void encode_affine_kernel(const float* __res
     auto& errors = lds.blocks.errors;
     auto& hcode = lds.blocks.hcode;
     auto& level = lds.blocks.level;
+    auto& joint_level = lds.blocks.joint_level;
     const int t = threadIdx.x, g = t & (ng - 1), first = t & ~(ng - 1);
-    if (t < 1 << bits) level[t] = double2{(double)((float)t * unit), (double)((float)t * unit * ((float)t * unit))};
+    const float own_level = (float)t * unit;
+    if (t < 1 << bits) level[t] = double2{(double)own_level, (double)own_level * (double)own_level};
     __syncthreads();
     const int64_t mine = (int64_t)(blockIdx.x - with_short) * (64 / ng) + t / ng;
     const int64_t blk = mine < nblocks ? mine : nblocks - 1;  // past the end: the last block again, stored by nobody
@@ -494,12 +499,13 @@ __global__ __launch_bounds__(64, 4) void encode_affine_kernel(const float* __res
     float s = range, m = minw;
     float off_s = 0.0f, off_m = 0.0f;  // how far s and m may be from the reference's: 0, or they are a quick_solve of `was`
     uint32_t p[quads], was[quads];
-    // The reference's double sums over the levels `was`, and its solution.  JOINT: the square of a level is a float product, not fused.
-    auto solve = [&](auto joint) __attribute__((always_inline)) {
+    // The reference's double sums over the levels `was`, and its solution.  The fit's squares of levels are fused, and so exact, a
+    // refinement's are float products.  JOINT: of is `level` or `joint_level`, a lane's own choice.
+    auto solve = [&](const double2* of, auto joint) __attribute__((always_inline)) {
         double sl = 0, sl2 = 0, sxl = 0;
 #pragma unroll
         for (int i = 0; i < gsz; ++i) {
-            const double2* const at = level + (was[i / 4] >> (8 * (i % 4)) & 0xFFu);
+            const double2* const at = of + (was[i / 4] >> (8 * (i % 4)) & 0xFFu);
             const double l = at->x;
             sl += l;
             if constexpr (decltype(joint)::value) sl2 += at->y;
@@ -581,7 +587,7 @@ __global__ __launch_bounds__(64, 4) void encode_affine_kernel(const float* __res
         bool exact = false, polished = false, settled = false, divide = false;
 #pragma unroll 1
         for (int iter = 0;;) {
-            if (exact) solve(Group{});
+            if (exact) solve(level, Group{});
             exact = false;
             if (iter == 5) break;
             if (iter == 4 && !polished) {
@@ -705,6 +711,9 @@ __global__ __launch_bounds__(64, 4) void encode_affine_kernel(const float* __res
         sure = sure && lo == hi && fabsf(v) >= 1.25e-7f && fabsf(v) < 65000.0f;  // (smaller ones the reference does not round)
         return (float)lo;
     };
+    __syncthreads();  // (the errors' room)
+    if (t < 1 << bits) joint_level[t] = double2{(double)own_level, (double)(own_level * own_level)};
+    __syncthreads();
     float d, dm;
     int sc, mc;
     bool dead = false;  // all scales vanish: d = 0, codes 0, dm stays 1
@@ -718,7 +727,7 @@ __global__ __launch_bounds__(64, 4) void encode_affine_kernel(const float* __res
         mc = quick_code(-m, off_m, dm, -bias, mq - bias);
         if (__all(sure && (sc != 0 || off_s == 0.0f))) break;  // (without a scale the first refinement would not replace s and m)
         if (__any(off_s > 0.0f)) {
-            if (off_s > 0.0f) solve(Group{});
+            if (off_s > 0.0f) solve(level, Group{});
             continue;
         }
         dead = max_s <= eps;
@@ -778,11 +787,14 @@ __global__ __launch_bounds__(64, 4) void encode_affine_kernel(const float* __res
         for (;;) {
             quick_codes(nsc, nmc, nd, ndm);
             if (__all(dead || (sure && !failed))) break;
-            if (__any(failed || off_s > 0.0f)) {  // once more with the reference's own s and m
+            if (__any(failed || off_s > 0.0f)) {
+                // Once more with the reference's own s and m.  Those of a lane that fails in the first refinement are the fit's:
+                // wherever a lane has a scale and no failure the refinement has replaced them, and a lane without a scale
+                // came with its own.
 #pragma unroll 1
                 for (int again = 0; again < 2; ++again) {
                     if (again && failed) keep_levels();
-                    if (again ? failed : off_s > 0.0f) solve(Joint{});
+                    if (again ? failed : off_s > 0.0f) solve(again == 0 && iter == 0 && failed ? level : joint_level, Joint{});
                 }
                 failed = false;
                 continue;
