@@ -836,8 +836,8 @@ def test_sixteen_weight_runs_over_the_grid(O, tfq, gpu, fmt, N, K):
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("N,K", [(130, 4096), (67, 1792)])
 def test_six_bit_rows_of_any_magnitude(O, tfq, gpu, N, K, dtype):
-    """Q_G_6 of one pass multiplies codes as subnormal numbers with activations brought near the top of fp32's range, row by row:
-    rows of 1e-30 and 1e30 side by side, rows of 1e35 (whose sums of codes times activations are in range, 7e37 a run at most), runs of
+    """Q_G_6 of one pass multiplies codes as subnormal numbers with activations brought near the top of fp32's range, sixteen by sixteen:
+    rows down to 1e-37, of 1e-30 and 1e30 side by side, rows of 1e35 (whose sums of codes times activations are in range, 7e37 a run at most), runs of
     sixteen of one row that differ by 1e20, a zero row.  Bound: fp32 sums of exact products, as
     above, of each output against its terms; a zero row gives zeros."""
     import torch
@@ -846,7 +846,8 @@ def test_six_bit_rows_of_any_magnitude(O, tfq, gpu, N, K, dtype):
     dense = torch.from_numpy(O.decode_tensor("Q_G_6", pay, N * K).reshape(N, K)).to(gpu).double()
     base = torch.from_numpy(O.rng_normal(12, K, 1.0)).to(gpu)
     runs = torch.where(torch.arange(K, device=gpu) // 16 % 2 == 0, 1.0e-10, 1.0e10)
-    for rows in ([1e-30], [1e30], [1e35], [1e-30, 1e30], [1e30, 1e-30], [1e35, 1.0], [runs], [runs, 0.0], [0.0]):
+    for rows in ([1e-30], [1e-33], [1e-35], [1e-37], [1e30], [1e35], [1e-30, 1e30], [1e30, 1e-30], [1e-33, 1e-36], [1e35, 1.0], [1.0, 1e-35],
+                 [runs], [runs * 1e-25], [runs, 0.0], [0.0]):
         x = torch.stack([base * r for r in rows])
         x = x.bfloat16() if dtype == "bf16" else x
         y, want, terms = W.gemv(x).double(), x.double() @ dense.T, x.double().abs() @ dense.abs().T
