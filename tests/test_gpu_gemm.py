@@ -458,3 +458,19 @@ def test_k_parts_of_the_bf16_tiles_are_added_whole(O, tfq, gpu, M, N):
         y = W.gemm(x, out_dtype=dt).double()
         assert bool(((y - want).abs() <= terms * 2.0 ** -8 * 0.5 + (want.abs() * 2.0 ** -8 if dt == torch.bfloat16 else 0.0)).all()), dt
     W.close()
+
+
+def test_k_parts_of_the_bf16_tiles_one_and_four_outputs_a_lane(O, tfq, gpu):
+    """Four outputs a lane add the K parts in the order of one: a matrix and the same without its last row, whose products have a multiple
+    of four outputs and one more than that, agree bit for bit where they share rows."""
+    import torch
+    K, N, M = 2048, 4736, 455
+    w = torch.randn(N * K, generator=torch.Generator().manual_seed(3)).to(gpu) * 0.02
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(4)).to(gpu).bfloat16()
+    whole, less = (tfq.Weight("Q_8", n, K, tfq.encode("Q_8", w[:n * K])) for n in (N, N - 1))
+    parts = [int(tfq.lib().tfq_gemm_workspace_bytes(W.handle, 1, M)) / (4 * M * n) for W, n in ((whole, N), (less, N - 1))]
+    assert parts[0] == parts[1] in (2.0, 4.0, 8.0), parts
+    for dt in (torch.float32, torch.bfloat16):
+        assert torch.equal(whole.gemm(x, out_dtype=dt)[:, :N - 1], less.gemm(x, out_dtype=dt)), dt
+    whole.close()
+    less.close()
