@@ -716,7 +716,8 @@ __global__ __launch_bounds__(64, 4) void encode_affine_kernel(const float* __res
     __syncthreads();
     float d, dm;
     int sc, mc;
-    bool dead = false;  // all scales vanish: d = 0, codes 0, dm stays 1
+    bool dead = false;     // all scales vanish: d = 0, codes 0, dm stays 1
+    bool refined = false;  // `was` are a refinement's levels, not the fit's
 #pragma unroll 1
     for (;;) {
         const float max_s = block_max(fabsf(s)), max_m = block_max(fabsf(m));
@@ -725,7 +726,7 @@ __global__ __launch_bounds__(64, 4) void encode_affine_kernel(const float* __res
         dm = quick_half(max_m * (1.0f / (float)bias), __builtin_fmaf(block_max(off_m), 1.01f / (float)bias, 5.0f * kUlp / (float)bias * max_m));
         sc = quick_code(s, off_s, d, 0, scq);
         mc = quick_code(-m, off_m, dm, -bias, mq - bias);
-        if (__all(sure && (sc != 0 || off_s == 0.0f))) break;  // (without a scale the first refinement would not replace s and m)
+        if (__all(sure)) break;
         if (__any(off_s > 0.0f)) {
             if (off_s > 0.0f) solve(level, Group{});
             continue;
@@ -778,8 +779,15 @@ __global__ __launch_bounds__(64, 4) void encode_affine_kernel(const float* __res
         }
         if (iter == 5) break;  // (the payload's levels)
         if (eff_s != 0.0f) {
-            failed = !quick_solve(p, Joint{});
-            if (!failed) keep_levels();
+            if (quick_solve(p, Joint{})) {
+                keep_levels();
+                refined = true;
+            } else if (plain) {
+                // One level for all weights, as where a group's offset is far from dm times its code: the reference's D is the
+                // rounding of that level's square, and s and m stay unless it is positive.  (With its sums taken there instead
+                // 58.7 M weights of Q_G_2, groups of a spread of 0.004 about offsets of 0.05, 384 us, 305 so.)
+                failed = joint_level[p[0] & 0xFFu].y > level[p[0] & 0xFFu].y;
+            } else failed = true;
         }
         int nsc, nmc;
         float nd, ndm;
@@ -788,13 +796,14 @@ __global__ __launch_bounds__(64, 4) void encode_affine_kernel(const float* __res
             quick_codes(nsc, nmc, nd, ndm);
             if (__all(dead || (sure && !failed))) break;
             if (__any(failed || off_s > 0.0f)) {
-                // Once more with the reference's own s and m.  Those of a lane that fails in the first refinement are the fit's:
-                // wherever a lane has a scale and no failure the refinement has replaced them, and a lane without a scale
-                // came with its own.
+                // Once more with the reference's own s and m, which are the fit's where no refinement has replaced them.
 #pragma unroll 1
                 for (int again = 0; again < 2; ++again) {
-                    if (again && failed) keep_levels();
-                    if (again ? failed : off_s > 0.0f) solve(again == 0 && iter == 0 && failed ? level : joint_level, Joint{});
+                    if (again && failed) {
+                        keep_levels();
+                        refined = true;
+                    }
+                    if (again ? failed : off_s > 0.0f) solve(refined ? joint_level : level, Joint{});
                 }
                 failed = false;
                 continue;
