@@ -292,7 +292,7 @@ __global__ __launch_bounds__(256) void encode_q1_kernel(const float* __restrict_
 // wavefronts meet the latter in the fit, three quarters once in their five refinements; a build that never does takes 25 us
 // less.  The polish compares six errors that are formed in fp32 first.
 // 58.7 M weights of Q_G_4: 7.46 ms with one block per wavefront and the division, 268 to 290 us with all sums in double,
-// 236 now; Q_G_3 269 -> 234, Q_G_2 344 -> 306, SB256A3 351 -> 308, SB256A2 351 -> 307; smaller calls by
+// 236 now; Q_G_3 269 -> 233, Q_G_2 344 -> 305, SB256A3 351 -> 301, SB256A2 351 -> 307; smaller calls by
 // encode_affine_summed_kernel.  Four wavefronts a SIMD: three have 17 % less of its issue.
 __device__ __forceinline__ uint32_t unit_nearest_dev(float value, int bits) {
     const float v = fmaxf(0.0f, fminf(1.0f, value));
@@ -1128,7 +1128,8 @@ static void launch_encode_affine(const float* w, int64_t nblocks, uint8_t* dst, 
     // every pass and integer sums: Q_G_4 786432 weights 23.5 and 25.0, 5 M 38.7 and 40.9, 8 M 54.5 and 49.6; Q_G_3 1 M 23.7 and 28.8, 5 M 37.7
     // and 38.2, 8 M 53.8 and 49.3; Q_G_2 786432 17.5 and 20.2, 5 M 39.6 and 39.9, 8 M 58.5 and 54.7; SB256A2 524288 18.0 and 20.0, 8 M
     // 59.7 and 55.5; SB256A3 2 M 23.2 and 24.7, 8 M 59.5 and 55.7.  (Between, a few per cent either way with the weights.)  Q_1_5
-    // at every size timed: 262144 19.7 and 26.5, 8 M 48.0 and 52.7, 16 M 83.5 and 87.3.
+    // at every size timed: 262144 19.7 and 26.5, 8 M 48.0 and 52.7, 16 M 83.5 and 87.3.  All of normal weights; ones that reach a bound in
+    // nearly every refinement are slower at any size (16 M of Q_G_4: of 1e-6 93 and 115, u^8 90 and 104, two values 89 and 94).
     if constexpr (FMT != TFQ_Q_1_5) {
         if (nblocks > 24576) {
             hipLaunchKernelGGL(encode_affine_kernel<FMT>, grid, dim3(64), 0, s, w, dst, nblocks, job);
